@@ -64,7 +64,18 @@ struct lee_ctx {
     unsigned fb_mask = 0;   // the forms lee_options.path allows, bit f for form f
     int rk_variant = -1;    // RK4 air-stage launch shape (kRkTiles index), -1 until tuned
     bool rk_xfaces = false; // that shape's air stage takes the x-face nodes of the interior rows
-    bool fb_xfaces = false; // the split FB passes take them
+    // row form of the stencils (lee_row.h): whether the domain can run it, its launch plan, the
+    // ring of tiles around the interior box, the x layers' merged profiles and the step
+    // arguments for either parity of the buffer roles (refreshed when the roles, the y1 gate or
+    // the frame change, never inside a capture)
+    bool row_ok = false;
+    RowPlan plan{};
+    int *ring = nullptr;
+    void *xprof[3] = {};
+    void *row_args = nullptr, *row_lines = nullptr;       // lines: ny rows, then nz planes
+    std::vector<double> line_prof[6][3], line_m[2], line_t;  // of the frame, as uploaded (y, z)
+    std::vector<uintptr_t> row_key;
+    uintptr_t frame_gen = 0;
     // RK4 air-stage arguments of the four stages in device memory and the host copy they were
     // uploaded from (refreshed when buffer roles or the y1 gate change, never inside a capture)
     void *rk_args_dev = nullptr;
@@ -410,6 +421,24 @@ int upload_frame(lee_ctx *c, int N)
         if ((rc = upload(c, c->prof[s][1], P[s]->c.data(), P[s]->c.size()))) return rc;
         if ((rc = upload(c, c->prof[s][2], P[s]->d.data(), P[s]->d.size()))) return rc;
     }
+    if (c->row_ok) {
+        // the x layers do not overlap: one table holds both (zero outside)
+        const std::vector<double> *A[3] = {&t.x1.s, &t.x1.c, &t.x1.d}, *B[3] = {&t.x2.s, &t.x2.c, &t.x2.d};
+        for (int q = 0; q < 3; ++q) {
+            std::vector<double> v(*A[q]);
+            for (size_t i = 0; i < v.size(); ++i)
+                if ((int)i >= m.nx - m.I2) v[i] = (*B[q])[i];
+            if ((rc = upload(c, c->xprof[q], v.data(), v.size()))) return rc;
+        }
+        for (int s = 2; s < 6; ++s) {
+            c->line_prof[s][0] = P[s]->s; c->line_prof[s][1] = P[s]->c; c->line_prof[s][2] = P[s]->d;
+        }
+        c->line_m[0] = t.Yy; c->line_m[1] = t.Zz;
+        if (c->prec == 32 && !m.terrain)
+            for (auto &v : c->line_m)
+                for (size_t i = 0; i < v.size(); ++i) v[i] = i >= 1 && i + 1 < v.size() ? 1.0 / v[i] : 0.0;
+        c->line_t = m.terrain ? t.ter.tk : std::vector<double>(m.nz, 0.0);
+    }
     if (m.has_wind && m.wind_v_only) {
         // velocity_method 7 on the device: over terrain the ground under a node changes with
         // the frame; on a flat grid the field is the same in every frame
@@ -717,14 +746,99 @@ template <typename T> void enqueue_rk4_step(lee_ctx *c, double *rec_slot)
     c->steps += 1;
 }
 
-// Face-walk arguments of the split FB passes: they take the x-face nodes of the interior rows
-// (the face passes then walk only the x planes' edge rings); returns whether they do.
-template <typename T> bool fb_face_args(const lee_ctx *c, const AirArgs<T> &a, BCArgs<T> &b)
+// Whether the FB step runs in row form.
+bool fb_rows(const lee_ctx *c) { return c->row_ok && !c->fused; }
+
+// Brings the row kernels' device arguments up to date for the gate state (J1, y1on): one block
+// per parity of the buffer roles (slot c->cur), which alternate every step, so that a step
+// uploads nothing.
+template <typename T> int row_args_sync(lee_ctx *c, int J1, int y1on)
 {
-    if (c->fused || !fb_passes_take_xfaces<T>(a)) return false;
-    b.xring = 1;
-    b.nb_air = boundary_count<T>(c->m.nx, c->m.ny, c->m.nz, true);
-    return true;
+    const Model &m = c->m;
+    const int cur = c->cur, qcur = c->qcur, rel = cur ^ qcur;
+    double *psi[2] = {c->psi, c->psi2}, *gpsi[2] = {c->gpsi, c->gpsi2};
+    // the histories read at parity 0 (those in use alternate with the fields)
+    const bool fp = m.east_tdbc, fg = m.ground;
+    double *p0 = psi[fp ? cur : 0], *g0 = gpsi[fg ? cur : 0];
+    const std::vector<uintptr_t> key = {(uintptr_t)J1, (uintptr_t)y1on, (uintptr_t)rel, (uintptr_t)p0, (uintptr_t)g0, c->frame_gen};
+    if (key == c->row_key) return LEE_OK;
+    if (c->capturing) return set_err(c, LEE_ERR_STATE, "step arguments changed inside a captured chunk");
+    std::vector<RowLine<T>> lines((size_t)m.ny + m.nz);
+    for (int ax = 1; ax < 3; ++ax)
+        for (int n = 0; n < (ax == 1 ? m.ny : m.nz); ++n) {
+            RowLine<T> &l = lines[(ax == 1 ? 0 : m.ny) + n];
+            std::memset(&l, 0, sizeof l);
+            const SlabGeom &lo = m.slab[2 * ax], &hi = m.slab[2 * ax + 1];
+            const int w1 = ax == 1 ? J1 : m.K1, w2 = ax == 1 ? m.J2 : m.K2, len = ax == 1 ? m.ny : m.nz;
+            const bool in1 = lo.n && n < lo.lo + lo.n && (ax == 2 || y1on), in2 = hi.n && n >= hi.lo;
+            l.m = (T)c->line_m[ax - 1][n];
+            l.t = ax == 2 ? (T)c->line_t[n] : T(0);
+            if (!in1 && !in2) continue;
+            const SlabGeom &g = in1 ? lo : hi;
+            const long long step = ax == 1 ? m.nx : (long long)m.nx * m.ny;
+            l.has = 1;
+            l.act = in1 ? n < w1 : n >= len - w2;
+            l.off = (int)((in1 || !lo.n ? 0 : (long long)lo.count(m.nx, m.ny, m.nz)) + step * (n - g.lo));
+            l.ks = ax == 1 ? m.nx * g.n : 0;
+            const std::vector<double> *pr = c->line_prof[2 * ax + (in1 ? 0 : 1)];
+            l.s = (T)pr[0][n]; l.c = (T)pr[1][n]; l.d = (T)pr[2][n];
+        }
+    std::vector<unsigned char> host(2 * sizeof(RowArgs<T>));
+    for (int par = 0; par < 2; ++par) {
+        c->cur = par; c->qcur = par ^ rel;
+        const int sp = fp ? par ^ cur : 0, sg = fg ? par ^ cur : 0;
+        c->psi = psi[sp]; c->psi2 = psi[sp ^ 1];
+        c->gpsi = gpsi[sg]; c->gpsi2 = gpsi[sg ^ 1];
+        RowArgs<T> r;
+        std::memset(&r, 0, sizeof r);
+        r.a = air_args<T>(c, J1, y1on);
+        r.b = bc_args<T>(c, r.a, nullptr);
+        const SlabGeom &x1 = m.slab[0], &x2 = m.slab[1];
+        r.geo = RowGeo{m.nx, m.ny, m.nz, m.south_porous ? m.pnz : 0, c->plan.j0, c->plan.p.nty, x1.lo + x1.n,
+                       x2.n ? x2.lo : INT_MAX, m.I1, x2.n ? m.nx - m.I2 : INT_MAX, x1.n, x2.n,
+                       (x1.n ? (int)x1.count(m.nx, m.ny, m.nz) : 0) - x2.lo, m.south_porous, m.iface_copy, m.ground,
+                       m.east_tdbc, (int)m.ri.size()};
+        r.yl = (const RowLine<T> *)c->row_lines;
+        r.zl = (const RowLine<T> *)c->row_lines + m.ny;
+        r.xs = (const T *)c->xprof[0]; r.xc = (const T *)c->xprof[1]; r.xd = (const T *)c->xprof[2];
+        for (int ax = 0; ax < 3; ++ax) {
+            const int s0 = m.slab[2 * ax].n ? 2 * ax : 2 * ax + 1;
+            for (int f = 0; f < 4; ++f) { r.q[ax].o[f] = r.a.Qo[s0][f]; r.q[ax].n[f] = r.a.Qn[s0][f]; }
+        }
+        r.pgama = (T)m.p_gama; r.pinvb = (T)m.p_invbeta; r.peff = (T)m.p_eff;
+        std::memcpy(host.data() + par * sizeof r, &r, sizeof r);
+    }
+    c->cur = cur; c->qcur = qcur;
+    c->psi = psi[0]; c->psi2 = psi[1]; c->gpsi = gpsi[0]; c->gpsi2 = gpsi[1];
+    HIPCHK(c, hipMemcpyAsync(c->row_args, host.data(), host.size(), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->row_lines, lines.data(), lines.size() * sizeof(RowLine<T>), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->row_key = key;
+    return LEE_OK;
+}
+template <typename T> const RowArgs<T> *row_args_now(const lee_ctx *c) { return (const RowArgs<T> *)c->row_args + c->cur; }
+// Row arguments of the coming step, without advancing the gate counter.
+template <typename T> int row_args_peek(lee_ctx *c)
+{
+    const long long save = c->counter;
+    int J1, y1on;
+    gate_tick(c, J1, y1on);
+    c->counter = save;
+    return row_args_sync<T>(c, J1, y1on);
+}
+
+// The two phases of an FB_p_v step in row form.
+template <typename T> void row_p(lee_ctx *c, int form, double *rec)
+{
+    const Model &m = c->m;
+    launch_row_p<T>(row_args_now<T>(c), c->plan, m.has_wind, m.terrain, c->plan.has_in && form != 1, form == 0 && m.nx % 4 == 0, rec,
+                    c->stream);
+}
+template <typename T> void row_v(lee_ctx *c, int form)
+{
+    const Model &m = c->m;
+    launch_row_v<T>(row_args_now<T>(c), c->plan, m.has_wind, m.terrain, c->plan.has_in && form != 1, form == 0 && m.nx % 4 == 0,
+                    c->stream);
 }
 
 // One FB_p_v step (airpore.cpp:589-614): launches only, receivers into rec_slot.
@@ -734,54 +848,60 @@ template <typename T> void enqueue_fb_step(lee_ctx *c, double *rec_slot)
     hipStream_t s = c->stream;
     int J1, y1on;
     gate_tick(c, J1, y1on);
-    AirArgs<T> a = air_args<T>(c, J1, y1on);
-    PoreArgs<T> pa{};
-    if (m.south_porous) pa = PoreArgs<T>{pore_grid<T>(c), (T)m.p_gama, (T)m.p_invbeta, (T)m.p_eff};
-    BCArgs<T> b = bc_args<T>(c, a, rec_slot);
     if (c->fb_form < 0) c->fb_form = (c->fb_mask & 1u) ? 0 : 3;  // not tuned: the path's default
     c->fused = fb_form_fused(c->fb_form);
-    const bool pad = c->fb_form == 1, vec_ok = c->fb_form != 6;
-    const int per_cu = c->fused ? kFbPerCu[c->fb_form - 2] : 0;
-    c->fb_xfaces = fb_face_args<T>(c, a, b);
-    if (c->fused) {
-        // porous pressure first: the air South face reads its plane Kp-2 through the interface
-        if (m.south_porous) {
-            prof_mark(c, KS_PORE_P, true);
-            launch_pore_p<T>(pa, s);
-            prof_mark(c, KS_PORE_P, false);
-        }
-        prof_mark(c, KS_AIR_FB, true);
-        launch_air_fb<T>(a, m.has_wind, s, per_cu);
-        prof_mark(c, KS_AIR_FB, false);
-        prof_mark(c, KS_BC_P, true);
-        launch_bc_p_all<T>(b, s);
-        prof_mark(c, KS_BC_P, false);
-    } else {
-        // ---- pressure phase (airpore.cpp:366-398); receivers sample level n first
+    if (fb_rows(c)) {
+        if (row_args_sync<T>(c, J1, y1on)) c->args_fault = true;
+        // pressure phase (airpore.cpp:366-398) with the receivers of level n, then the velocities
+        // (airpore.cpp:324-364)
         prof_mark(c, KS_AIR_P, true);
-        launch_air_p<T>(a, m.has_wind, s, pad, vec_ok);
+        row_p<T>(c, c->fb_form, rec_slot);
         prof_mark(c, KS_AIR_P, false);
-        if (m.south_porous) {
+        prof_mark(c, KS_AIR_V, true);
+        row_v<T>(c, c->fb_form);
+        prof_mark(c, KS_AIR_V, false);
+    } else {
+        AirArgs<T> a = air_args<T>(c, J1, y1on);
+        PoreArgs<T> pa{};
+        if (m.south_porous) pa = PoreArgs<T>{pore_grid<T>(c), (T)m.p_gama, (T)m.p_invbeta, (T)m.p_eff};
+        BCArgs<T> b = bc_args<T>(c, a, rec_slot);
+        auto pore_p = [&]() {
+            if (!m.south_porous) return;
             prof_mark(c, KS_PORE_P, true);
             launch_pore_p<T>(pa, s);
             prof_mark(c, KS_PORE_P, false);
+        };
+        auto bc_p = [&]() {
+            prof_mark(c, KS_BC_P, true);
+            launch_bc_p_all<T>(b, s);
+            prof_mark(c, KS_BC_P, false);
+        };
+        if (c->fused) {
+            // porous pressure first: the air South face reads its plane Kp-2 through the interface
+            pore_p();
+            prof_mark(c, KS_AIR_FB, true);
+            launch_air_fb<T>(a, m.has_wind, s, kFbPerCu[c->fb_form - 2]);
+            prof_mark(c, KS_AIR_FB, false);
+            bc_p();
+        } else {
+            prof_mark(c, KS_AIR_P, true);
+            launch_air_p<T>(a, m.has_wind, s);
+            prof_mark(c, KS_AIR_P, false);
+            pore_p();
+            bc_p();
+            prof_mark(c, KS_AIR_V, true);
+            launch_air_v<T>(a, m.has_wind, s);
+            prof_mark(c, KS_AIR_V, false);
         }
-        prof_mark(c, KS_BC_P, true);
-        launch_bc_p_all<T>(b, s);
-        prof_mark(c, KS_BC_P, false);
-        // ---- velocity phase (airpore.cpp:324-364)
-        prof_mark(c, KS_AIR_V, true);
-        launch_air_v<T>(a, m.has_wind, s, pad, vec_ok);
-        prof_mark(c, KS_AIR_V, false);
+        if (m.south_porous) {
+            prof_mark(c, KS_PORE_V, true);
+            launch_pore_v<T>(pa, s);
+            prof_mark(c, KS_PORE_V, false);
+        }
+        prof_mark(c, KS_BC_V, true);
+        launch_bc_v_all<T>(b, s);
+        prof_mark(c, KS_BC_V, false);
     }
-    if (m.south_porous) {
-        prof_mark(c, KS_PORE_V, true);
-        launch_pore_v<T>(pa, s);
-        prof_mark(c, KS_PORE_V, false);
-    }
-    prof_mark(c, KS_BC_V, true);
-    launch_bc_v_all<T>(b, s);
-    prof_mark(c, KS_BC_V, false);
     if (m.east_tdbc) std::swap(c->psi, c->psi2);
     if (m.ground) std::swap(c->gpsi, c->gpsi2);
     inject_source<T>(c, (T *)c->air[(c->cur ^ 1) * 4 + 3]);
@@ -821,6 +941,9 @@ template <typename T> int graph_steps(lee_ctx *c, int n)
     if (m.rk4) {  // the chunk's stage arguments (constant over it) into device memory first
         int rc = rk_args_peek<T>(c);
         if (rc) return rc;
+    } else if (fb_rows(c)) {
+        int rc = row_args_peek<T>(c);
+        if (rc) return rc;
     }
     for (auto &g : c->graphs)
         if (g.n == n && g.cur == c->cur && g.qcur == c->qcur && g.gate_on == gate_on && g.psi == (void *)c->psi &&
@@ -848,7 +971,7 @@ template <typename T> int graph_steps(lee_ctx *c, int n)
     if (c->args_fault) {
         (void)hipGraphDestroy(graph);
         c->args_fault = false;
-        return set_err(c, LEE_ERR_STATE, "RK4 stage arguments changed inside a captured chunk");
+        return set_err(c, LEE_ERR_STATE, "step arguments changed inside a captured chunk");
     }
     hipError_t ie = hipGraphInstantiate(&e.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
@@ -924,36 +1047,47 @@ template <typename T> int tune_rk(lee_ctx *c)
     return LEE_OK;
 }
 
-// Autotuner of the FB_p_v air passes: times each launch form the path allows on the air and
-// face passes of the coming step (they write only level n+1, its auxiliaries and the
-// receiver buffer, all of which the step itself rewrites) and keeps the fastest.  The porous
-// passes are the same in every form and are left out.
+// Autotuner of the FB_p_v passes: times each candidate form on the coming step's passes (they
+// write only level n+1, its auxiliaries and the receiver buffer, all of which the step itself
+// rewrites) and keeps the fastest.  The fused pass took three times as long as the others on
+// every grid measured (1.10 against 0.36 ms on 512 x 256 x 128 in FP32) and is a candidate only
+// where the path asks for it; without an interior box the row form has one form.
 template <typename T> int tune_fb(lee_ctx *c)
 {
     const Model &m = c->m;
+    unsigned cand = c->fb_mask & kFbSplitForms ? c->fb_mask & kFbSplitForms : c->fb_mask;
+    if (cand & kFbSplitForms) {
+        c->fused = false;
+        if (!c->row_ok || !c->plan.has_in) {
+            c->fb_form = 1;  // the whole domain at once
+            return LEE_OK;
+        }
+    }
     const long long save = c->counter;
     int J1, y1on;
     gate_tick(c, J1, y1on);
     c->counter = save;
     const AirArgs<T> a = air_args<T>(c, J1, y1on);
+    BCArgs<T> b = bc_args<T>(c, a, c->rec_buf);
     float t[kFbForms];
     for (int f = 0; f < kFbForms; ++f) t[f] = 1e30f;
     for (int pass = 0; pass < 2; ++pass)
         for (int f = 0; f < kFbForms; ++f) {
-            if (!(c->fb_mask >> f & 1u)) continue;
+            if (!(cand >> f & 1u)) continue;
             c->fused = fb_form_fused(f);
-            BCArgs<T> b = bc_args<T>(c, a, c->rec_buf);
-            (void)fb_face_args<T>(c, a, b);
+            if (!c->fused) {
+                int rc = row_args_sync<T>(c, J1, y1on);
+                if (rc) return rc;
+            }
             auto passes = [&]() {
                 if (c->fused) {
                     launch_air_fb<T>(a, m.has_wind, c->stream, kFbPerCu[f - 2]);
                     launch_bc_p_all<T>(b, c->stream);
+                    launch_bc_v_all<T>(b, c->stream);
                 } else {
-                    launch_air_p<T>(a, m.has_wind, c->stream, f == 1, f != 6);
-                    launch_bc_p_all<T>(b, c->stream);
-                    launch_air_v<T>(a, m.has_wind, c->stream, f == 1, f != 6);
+                    row_p<T>(c, f, c->rec_buf);
+                    row_v<T>(c, f);
                 }
-                launch_bc_v_all<T>(b, c->stream);
             };
             passes();  // warm-up
             HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -967,7 +1101,7 @@ template <typename T> int tune_fb(lee_ctx *c)
     HIPCHK(c, hipGetLastError());
     int pick = -1;
     for (int f = 0; f < kFbForms; ++f)
-        if ((c->fb_mask >> f & 1u) && (pick < 0 || t[f] < t[pick])) pick = f;
+        if ((cand >> f & 1u) && (pick < 0 || t[f] < t[pick])) pick = f;
     c->fb_form = pick;
     c->fused = fb_form_fused(pick);
     return LEE_OK;
@@ -1004,7 +1138,7 @@ template <typename T> int run_steps(lee_ctx *c, int nsteps, double *rec_out)
         }
         if (c->args_fault) {
             c->args_fault = false;
-            return set_err(c, LEE_ERR_DEVICE, "RK4 stage arguments could not be uploaded: " + c->err);
+            return set_err(c, LEE_ERR_DEVICE, "the step arguments could not be uploaded: " + c->err);
         }
         HIPCHK(c, hipGetLastError());
         if (rec_out && nr) {
@@ -1066,6 +1200,20 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
             C->fb_form = o.fb_form - 1;
         }
         C->fused = fb_form_fused(C->fb_form) || o.path == LEE_PATH_FUSED;
+        // row form: no embedded obstacle, the two slabs of an axis apart, tile and auxiliary
+        // indices within their fields
+        bool apart = true;
+        for (int ax = 0; ax < 3; ++ax) {
+            const SlabGeom &lo = mm.slab[2 * ax], &hi = mm.slab[2 * ax + 1];
+            if (lo.n && hi.n && hi.lo < lo.n) apart = false;
+        }
+        bool fits = true;
+        for (int ax = 0; ax < 3; ++ax) {
+            const long long e = (long long)mm.slab[2 * ax].count(mm.nx, mm.ny, mm.nz) + (long long)mm.slab[2 * ax + 1].count(mm.nx, mm.ny, mm.nz);
+            fits = fits && e * (long long)(ax == 0 ? C->esz : 1) < (1LL << 31);
+        }
+        C->row_ok = !mm.obstacle && apart && fits && (mm.nx + 63) / 64 < (1 << 16) && mm.ny / 4 < (1 << 14) &&
+                    (long long)mm.nz + mm.pnz + 64 < 65536;
         // the boundary kernels decode node indices in 32 bits
         const long long nb = boundary_count<double>(mm.nx, mm.ny, mm.nz) +
                              (mm.south_porous ? boundary_count<double>(mm.pnx, mm.pny, mm.pnz) : 0) + (long long)mm.ri.size();
@@ -1091,6 +1239,26 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
     if (m.south_porous)
         if ((rc = dalloc(C, &C->pmx, m.pnx * es)) || (rc = dalloc(C, &C->pmy, m.pny * es)) || (rc = dalloc(C, &C->pmz, m.pnz * es)))
             return rc;
+    if (C->row_ok) {
+        RowGeom rg{m.nx, m.ny, m.nz, m.south_porous ? m.pnz : 0, m.iface_copy, m.ground, (int)m.ri.size(), {}, {},
+                   {m.I1, m.I2, m.J3, m.J2, m.K1, m.K2}};
+        for (int s = 0; s < 6; ++s) { rg.qn[s] = m.slab[s].n; rg.qlo[s] = m.slab[s].lo; }
+        std::vector<int> ring;
+        row_plan(C->plan, ring, rg);
+        if (!ring.empty()) {
+            if ((rc = dalloc(C, (void **)&C->ring, ring.size() * sizeof(int)))) return rc;
+            HIPCHK(C, hipMemcpyAsync(C->ring, ring.data(), ring.size() * sizeof(int), hipMemcpyHostToDevice, C->stream));
+            HIPCHK(C, hipStreamSynchronize(C->stream));
+        }
+        C->plan.p.ring = C->plan.v.ring = C->ring;
+        for (int q = 0; q < 3; ++q)
+            if ((rc = dalloc(C, &C->xprof[q], (size_t)m.nx * es))) return rc;
+        if (!m.rk4) {
+            const size_t sz = C->prec == 64 ? sizeof(RowArgs<double>) : sizeof(RowArgs<float>);
+            const size_t sl = C->prec == 64 ? sizeof(RowLine<double>) : sizeof(RowLine<float>);
+            if ((rc = dalloc(C, &C->row_args, 2 * sz)) || (rc = dalloc(C, &C->row_lines, (size_t)(m.ny + m.nz) * sl))) return rc;
+        }
+    }
     int len[6] = {m.nx, m.nx, m.ny, m.ny, m.nz, m.nz};
     size_t qmax = 0;
     for (int s = 0; s < 6; ++s) {
@@ -1099,8 +1267,15 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
         size_t cnt = m.slab[s].count(m.nx, m.ny, m.nz);
         qmax = std::max(qmax, cnt);
         for (int h = 0; h < 2; ++h)
-            for (int f = 0; f < 4; ++f)
-                if ((rc = dalloc(C, &C->Q[h][s][f], cnt * es))) return rc;
+            for (int f = 0; f < 4; ++f) {
+                // the two slabs of an axis share a block per field (RowQ), the low one first
+                const size_t c1 = s % 2 == 0 ? m.slab[s + 1].count(m.nx, m.ny, m.nz) : 0;
+                if (s % 2 && m.slab[s - 1].n) {
+                    if (cnt) C->Q[h][s][f] = (char *)C->Q[h][s - 1][f] + m.slab[s - 1].count(m.nx, m.ny, m.nz) * es;
+                } else if ((rc = dalloc(C, &C->Q[h][s][f], cnt ? (cnt + c1) * es : 0))) {
+                    return rc;
+                }
+            }
     }
     if ((rc = dalloc(C, (void **)&C->psi, (size_t)m.nx * m.nz * 6 * 8))) return rc;
     if ((rc = dalloc(C, (void **)&C->psi2, (size_t)m.nx * m.nz * 6 * 8))) return rc;
@@ -1251,6 +1426,7 @@ int lee_frame_setup(lee_ctx *c, int N)
     rc = upload_frame(c, N);
     if (rc) return rc;
     c->mf_count = N;
+    c->frame_gen += 1;
     return LEE_OK;
 }
 
@@ -1801,12 +1977,14 @@ int lee_kernel_stats(const lee_ctx *c, lee_kstat *out, int cap)
     const double wrk = m.has_wind ? (m.wind_v_only ? 1.0 : 3.0) * m.nx * m.ny * m.nz : 0.0;
     // x-face nodes of the interior rows, when the RK4 air stage's launch shape takes them
     const double nxf = c->rk_xfaces ? 2.0 * (m.ny - 2) * (m.nz - 2) : 0.0;
-    const double fxf = c->fb_xfaces ? 2.0 * (m.ny - 2) * (m.nz - 2) : 0.0;  // the same for the FB passes
+    // the row form's FB phases hold the porous layer and the faces as well
+    const double fr = !m.rk4 && fb_rows(c) ? 1.0 : 0.0;
     const char *names[KS_N] = {"air_p", "air_v", "pore_p", "pore_v", "air_fb", "bc_p", "bc_v", "rk_air", "rk_pore", "rk_bnd"};
-    double bytes[KS_N] = {(5 * inner + qp + wind + 2 * fxf) * es, (7 * inner + qv + wind + 6 * fxf) * es, 5 * pinner * es,
-                          7 * pinner * es, (8 * inner + qf + wind) * es, 2 * (nb - fxf) * es, 6 * (nb - fxf) * es + psi,
+    double bytes[KS_N] = {(5 * (inner + fr * pinner) + qp + wind + 2 * fr * nb) * es,
+                          (7 * (inner + fr * pinner) + qv + wind + 6 * fr * nb) * es + fr * psi, 5 * pinner * es,
+                          7 * pinner * es, (8 * inner + qf + wind) * es, 2 * nb * es, 6 * nb * es + psi,
                           (rkw * inner + qrk + wrk + 8 * nxf) * es, prkw * pinner * es, 8 * (nb - nxf) * es};
-    double pts[KS_N] = {inner, inner, pinner, pinner, inner, nb - fxf, nb - fxf, inner, pinner, nb - nxf};
+    double pts[KS_N] = {inner + fr * pinner, inner + fr * pinner, pinner, pinner, inner, nb, nb, inner, pinner, nb - nxf};
     int n = 0;
     for (int k = 0; k < KS_N && n < cap; ++k) {
         lee_kstat s = c->kstat[k];

@@ -10,6 +10,7 @@
 
 #include <cstddef>
 #include <type_traits>
+#include <vector>
 
 namespace lee {
 
@@ -130,6 +131,66 @@ template <typename T> struct BCArgs {
     int nrec;
     gptr<double> rec_out;
 };
+// ---- row form (lee_row.h) ---------------------------------------------------------------
+// What a wavefront needs to know of its row (per j) or plane (per k), one record so that it comes
+// in one scalar load: the layer auxiliaries' element offset (the two slabs of an axis share a
+// block), the profile, the metric and (planes) the terrain's t_k.  Row j of plane k of a y slab
+// starts at off + ks k, of a z slab at off + nx j.
+template <typename T> struct RowLine {
+    int has, act;  // the line lies in a slab; its layer terms apply
+    int off, ks;
+    T s, c, d, m, t;
+};
+struct RowGeo {
+    int nx, ny, nz, pnz, j0, nty;  // j0: row of the first tile's first wavefront
+    int xa, xb, xi1, xi2;          // x1 holds i < xa, x2 i >= xb; terms apply for i < xi1, i >= xi2
+    int n0, n1, d2;                // planes of the x slabs, element of (x2, i) minus i
+    int porous, coupled, ground, tdbc, nrec;
+};
+// Arguments of one step's row kernels (device memory).  q: per axis the base of the axis's two
+// slabs per field, before and after.  a and b hold the coefficients, fields, porous grid (b.pore) and face
+// data; the x layers' profiles are merged (zero outside).
+template <typename T> struct RowQ { gptr<const T> o[4]; gptr<T> n[4]; };
+template <typename T> struct RowArgs {
+    RowGeo geo;
+    gptr<const RowLine<T>> yl, zl;
+    gptr<const T> xs, xc, xd;
+    RowQ<T> q[3];
+    T pgama, pinvb, peff;
+    AirArgs<T> a;
+    BCArgs<T> b;
+};
+// A box of whole tiles (64 x 4 points) outside every layer: tile columns tx .. tx+nbx-1, tile
+// rows ty .. ty+nby-1 (points j0 + 4 ty ...), planes k .. k+nk-1.
+struct RowBox { int tx, nbx, ty, nby, k, nk, j0; };
+// Block ranges of one launch.  Whole domain: a grid of ntx x nty tiles over z = air planes, then
+// porous planes, the ground plane and the receivers.  Around an interior box: blocks first[q] ..
+// first[q+1]-1 of section q (planes 1 .. ka-1, planes kb .., the ring of planes ka .. kb-1 listed
+// in `ring` as tx | ty << 16, porous, ground, receivers).
+struct RowLaunch {
+    int ntx, nty, z, zair, zpore, zground;
+    int ka, kb, nring;
+    int first[7];
+    const int *ring;
+};
+struct RowPlan {
+    bool has_in;
+    int j0;  // row of the first tile's first wavefront
+    RowBox in;
+    RowLaunch p, v;
+};
+struct RowGeom {
+    int nx, ny, nz, pnz, coupled, ground, nrec;
+    int qn[6], qlo[6], w[6];  // slabs and layer widths, x1 x2 y1 y2 z1 z2
+};
+void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m);
+// One phase of the FB_p_v step: split = the interior box in a launch of its own (vec: several
+// points per lane) and the rest in another, else everything in one.  rec: the step's receiver row.
+template <typename T> void launch_row_p(const RowArgs<T> *ad, const RowPlan &pl, bool wind, bool terrain, bool split,
+                                        bool vec, double *rec, hipStream_t s);
+template <typename T> void launch_row_v(const RowArgs<T> *ad, const RowPlan &pl, bool wind, bool terrain, bool split,
+                                        bool vec, hipStream_t s);
+
 // ---- RK4 (extension) ------------------------------------------------------------------
 // Registers: level n (xn), the accumulator acc = xn + sum_s b_s k_s, and the destination
 // (the next stage state xn + a_s k_s, or level n+1 = acc + b_4 k_4 after the last stage).
@@ -178,9 +239,6 @@ void launch_rk_air_v(const RKArgs<T> &r, const RKArgs<T> *rd, int wind, bool ter
 // Whether shape v's air stage also takes the x-face nodes of the interior rows (the boundary
 // stage then walks only the x planes' edge rings: BCArgs::xring).
 template <typename T> bool rk_stage_takes_xfaces(const RKArgs<T> &r, int v);
-// Whether the split FB passes (launch_air_p / launch_air_v) take the x-face nodes of the
-// interior rows (the face passes then walk only the x planes' edge rings).
-template <typename T> bool fb_passes_take_xfaces(const AirArgs<T> &a);
 template <typename T> void launch_rk_pore(const RKPoreArgs<T> &r, bool terrain, hipStream_t s);
 // r: the stage arguments on the host (node count), rd: the same in device memory (read by the
 // kernel; by value the block was copied to scratch for the slab indexing)
@@ -230,21 +288,18 @@ template <typename T> long long boundary_count(int nx, int ny, int nz, bool xrin
 template <typename T> void launch_bc_p_all(const BCArgs<T> &a, hipStream_t s);
 template <typename T> void launch_bc_v_all(const BCArgs<T> &a, hipStream_t s);
 
-// pad: the box lists of the split launches with each plane's tiles padded to a multiple of 8
-// (a tile column on one XCD under round-robin dispatch; padding tiles do nothing).
-// vec_ok: the interior box may run the vector form (several points per lane, FP32 only)
-template <typename T> void launch_air_p(const AirArgs<T> &a, bool wind, hipStream_t s, bool pad = false,
-                                          bool vec_ok = true);
-template <typename T> void launch_air_v(const AirArgs<T> &a, bool wind, hipStream_t s, bool pad = false,
-                                          bool vec_ok = true);
+// General form of the FB_p_v air passes (embedded obstacles, grids narrower than their layers).
+template <typename T> void launch_air_p(const AirArgs<T> &a, bool wind, hipStream_t s);
+template <typename T> void launch_air_v(const AirArgs<T> &a, bool wind, hipStream_t s);
 // Both air phases in one pass (pressure then velocity, plane by plane); see lee_kernels.hip.
 // Returns false when the grid does not fit the fused kernel (nx - 2 > 1024).
 template <typename T> bool fused_fits(int nx);
 // per_cu: the pencil depth is the planes / chunks that give about per_cu blocks per CU
 template <typename T> void launch_air_fb(const AirArgs<T> &a, bool wind, hipStream_t s, int per_cu = 4);
-// Launch forms of the FB_p_v air passes (the FB autotuner picks one; identical bits): 0 the
-// split passes, 1 the split passes with padded box lists, 2 .. 5 the fused pass with pencils
-// for kFbPerCu[form - 2] blocks per CU, 6 the split passes with the one-point interior.
+// Launch forms of the FB_p_v air passes (identical bits): 0 the interior box and the rest in a
+// launch each per phase, the interior several points per lane where it pays; 1 the whole domain
+// in one launch per phase; 2 .. 5 the fused pass with pencils for kFbPerCu[form - 2] blocks per
+// CU; 6 as 0 with one point per lane.
 constexpr int kFbPerCu[4] = {2, 4, 8, 16};
 constexpr int kFbForms = 7;
 constexpr bool fb_form_fused(int f) { return f >= 2 && f < 6; }

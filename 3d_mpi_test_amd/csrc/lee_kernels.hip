@@ -11,6 +11,7 @@
 // z_over_Z are non-zero, and every product with a zero term is dropped here.  Dropping
 // an exact zero from a sum leaves the value unchanged (only the sign of an exact-zero
 // result can differ).
+#include "lee_core.h"
 #include "lee_kernels.h"
 
 #include <algorithm>
@@ -85,39 +86,6 @@ template <int NB> __device__ __forceinline__ void list_point(const BoxList<NB> &
     list_point_(l, t, i, j, k, std::make_integer_sequence<int, NB>{});
 }
 
-template <typename T> __device__ __forceinline__ void metric(const Grid<T> &g, int i, int j, int k, T &mX, T &mY, T &mZ)
-{
-    if constexpr (std::is_same<T, double>::value) {
-        // Jacobian of calculation_2D.cpp:424-430 and Geo_over_var (df_over_var.cpp:5-9)
-        double xx = g.mx[i], yy = g.my[j], zz = g.mz[k];
-        double J = 1.0 / (xx * yy * zz);
-        mX = (yy * zz) * J;
-        mY = (xx * zz) * J;
-        mZ = (xx * yy) * J;
-    } else {
-        mX = g.mx[i]; mY = g.my[j]; mZ = g.mz[k];
-    }
-}
-
-// Terrain-following grid: X_over_x, Y_over_y as in the reference, Z_over_z = Zz[k]*sh(i,j),
-// Z_over_x = hx(i,j)*tk[k], Z_over_y = hy(i,j)*tk[k].  Of the nine inverse-metric terms of
-// Geo_over_var (df_over_var.cpp:5-9) five are non-zero: xX, yY, zZ and the cross terms
-// zX = -(Yy*Zx)*J, zY = -(Xx*Zy)*J.  The tables hold X_over_x ... (not reciprocals) in both
-// precisions.
-template <typename T> __device__ __forceinline__ void metric_terrain(const Grid<T> &g, int i, int j, int k, T &mX, T &mY,
-                                                                     T &mZ, T &zX, T &zY)
-{
-    const size_t c = (size_t)i + (size_t)g.nx * j;
-    const T xx = g.mx[i], yy = g.my[j], zz = g.mz[k] * g.tsh[c];
-    const T Zx = g.thx[c] * g.ttk[k], Zy = g.thy[c] * g.ttk[k];
-    const T J = T(1) / (xx * yy * zz);
-    mX = (yy * zz) * J;
-    mY = (xx * zz) * J;
-    mZ = (xx * yy) * J;
-    zX = (-(yy * Zx)) * J;
-    zY = (-(xx * Zy)) * J;
-}
-
 __device__ __forceinline__ size_t qxi(int ii, int j, int k, int n, int ny) { return (size_t)ii + (size_t)n * ((size_t)j + (size_t)ny * k); }
 __device__ __forceinline__ size_t qyi(int i, int jj, int k, int nx, int n) { return (size_t)i + (size_t)nx * ((size_t)jj + (size_t)n * k); }
 __device__ __forceinline__ size_t qzi(int i, int j, int kk, int nx, int ny) { return (size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * kk); }
@@ -145,121 +113,6 @@ template <typename T, int L = 7> __device__ __forceinline__ OwnQ<T> own_slabs(co
     o.idx[4] = o.in[4] ? qzi(i, j, k - a.qlo[4], nx, ny) : 0;
     o.idx[5] = o.in[5] ? qzi(i, j, k - a.qlo[5], nx, ny) : 0;
     return o;
-}
-
-// ------------------------------------------------------------------------------------
-// The interior arithmetic of the pressure and velocity increments for the mean flows of
-// velocity_method 0 and 7 (none, or V along y only), from the point's neighbour values.  The
-// one-point stencils below and the four-point form of the RK4 stage both call these, so every
-// launch shape computes the same bits.
-// ------------------------------------------------------------------------------------
-template <typename T> struct Nb {
-    T mX, mY, mZ, zX, zY;                        // inverse metric (zX = zY = 0 on a flat grid)
-    T pc, p_im, p_jp, p_jm, p_kp, p_km;          // p and its neighbours (i-1, j+-1, k+-1)
-    T uc, u_ip, u_jp, u_jm, u_kp, u_km;          // u
-    T vc, v_jp, v_jm, v_kp, v_km;                // v
-    T wc, w_jp, w_jm, w_kp, w_km;                // w
-    T Vc, V_ip, V_im, V_jp, V_jm, V_kp, V_km;    // mean flow along y
-};
-
-// dt*R_p without the layer terms (air.cpp:1953-2043); also the damped terms ddx, ddy and
-// the difference dwz the layer terms use.
-template <typename T, int WM, bool TERRAIN, bool CEN>
-__device__ __forceinline__ T dp_core(const AirArgs<T> &a, const Nb<T> &n, T &ddx, T &ddy, T &dwz)
-{
-    const Grid<T> &g = a.g;
-    const T dxi = g.dxi, dyi = g.dyi, dzi = g.dzi, dt = g.dt;
-    const T mX = n.mX, mY = n.mY, mZ = n.mZ, zX = n.zX, zY = n.zY, pc = n.pc;
-    const T dux = n.u_ip - n.uc;
-    const T dvy = n.v_jp - n.vc;
-    dwz = n.w_kp - n.wc;
-    T duz = T(0), dvz = T(0);
-    T div;
-    if constexpr (TERRAIN) {
-        duz = n.u_kp - n.uc;
-        dvz = n.v_kp - n.vc;
-        div = (((((mX * dux) * dxi) + ((zX * duz) * dzi)) + ((mY * dvy) * dyi)) + ((zY * dvz) * dzi)) + ((mZ * dwz) * dzi);
-    } else {
-        div = (((mX * dux) * dxi) + ((mY * dvy) * dyi)) + ((mZ * dwz) * dzi);
-    }
-    ddx = (mX * dux) * dxi;
-    ddy = (mY * dvy) * dyi;
-    if constexpr (TERRAIN) {
-        ddx = ddx + (zX * duz) * dzi;
-        ddy = ddy + (zY * dvz) * dzi;
-    }
-    T r;
-    if constexpr (WM == 2) {
-        // mean flow along y only (U = W = 0): the terms with U or W are exact zeros
-        const T Vc = n.Vc;
-        const T c2 = ((Vc * mY) * dyi) * dt;
-        T VY = ((mY * (n.V_jp - n.V_jm)) * dyi) * T(0.5);
-        if constexpr (CEN) r = -(c2 * ((n.p_jp - n.p_jm) * T(0.5)));
-        else r = -(c2 * (pc - n.p_jm));
-        if constexpr (TERRAIN) {
-            const T c3 = ((Vc * zY) * dzi) * dt;
-            VY = VY + ((zY * (n.V_kp - n.V_km)) * dzi) * T(0.5);
-            if constexpr (CEN) r = r - c3 * ((n.p_kp - n.p_km) * T(0.5));
-            else r = r - c3 * (pc - n.p_km);
-        }
-        r += (((-a.gam) * pc) * dt) * VY;
-        r += (((-a.gam) * a.Pav) * dt) * div;
-    } else {
-        r = (((-a.gam) * a.Pav) * dt) * div;
-    }
-    return r;
-}
-
-// dt*R_u, dt*R_v, dt*R_w without the layer terms (air.cpp:1476-1578); also the pressure
-// gradients gpx, gpy, gpz the layer terms use.
-template <typename T, int WM, bool TERRAIN, bool CEN>
-__device__ __forceinline__ void duvw_core(const AirArgs<T> &a, const Nb<T> &n, T &gpx, T &gpy, T &gpz, T &du, T &dv,
-                                          T &dw)
-{
-    const Grid<T> &g = a.g;
-    const T dxi = g.dxi, dyi = g.dyi, dzi = g.dzi, dt = g.dt, Aav = a.Aav;
-    const T mX = n.mX, mY = n.mY, mZ = n.mZ, zX = n.zX, zY = n.zY, pc = n.pc;
-    const T bpz = pc - n.p_km;
-    gpx = (mX * (pc - n.p_im)) * dxi;
-    gpy = (mY * (pc - n.p_jm)) * dyi;
-    gpz = (mZ * bpz) * dzi;
-    if constexpr (TERRAIN) {
-        gpx = gpx + (zX * bpz) * dzi;
-        gpy = gpy + (zY * bpz) * dzi;
-    }
-    const T uc = n.uc, vc = n.vc, wc = n.wc;
-    if constexpr (WM == 2) {
-        // mean flow along y only (U = W = 0): the terms with U or W or their gradients vanish
-        const T Vc = n.Vc;
-        const T c2 = ((Vc * mY) * dyi) * dt;
-        T VX = ((mX * (n.V_ip - n.V_im)) * dxi) * T(0.5);
-        T VY = ((mY * (n.V_jp - n.V_jm)) * dyi) * T(0.5);
-        const T VZ = ((mZ * (n.V_kp - n.V_km)) * dzi) * T(0.5);
-        // d/dY (and d/dZ over terrain) of one component: forward (reference) or central
-        auto d1 = [&](T fp, T fm, T fc) {
-            if constexpr (CEN) return (fp - fm) * T(0.5);
-            else return fp - fc;
-        };
-        du = -(c2 * d1(n.u_jp, n.u_jm, uc));
-        dv = -(c2 * d1(n.v_jp, n.v_jm, vc));
-        dw = -(c2 * d1(n.w_jp, n.w_jm, wc));
-        if constexpr (TERRAIN) {
-            const T c3 = ((Vc * zY) * dzi) * dt;
-            VX = VX + ((zX * (n.V_kp - n.V_km)) * dzi) * T(0.5);
-            VY = VY + ((zY * (n.V_kp - n.V_km)) * dzi) * T(0.5);
-            du = du - c3 * d1(n.u_kp, n.u_km, uc);
-            dv = dv - c3 * d1(n.v_kp, n.v_km, vc);
-            dw = dw - c3 * d1(n.w_kp, n.w_km, wc);
-        }
-        du += ((-Aav) * dt) * gpx;
-        dv += (((-uc) * VX) * dt - (vc * VY) * dt) - (wc * VZ) * dt;
-        dv += ((-Aav) * dt) * gpy;
-        dw += ((-Aav) * dt) * gpz;
-    } else {
-        du = ((-Aav) * dt) * gpx;
-        dv = ((-Aav) * dt) * gpy;
-        dw = ((-Aav) * dt) * gpz;
-    }
 }
 
 // Neighbour values of one point for dp_core (DP) and/or duvw_core (DUVW), read from memory;
@@ -655,29 +508,18 @@ template <typename T> __device__ __forceinline__ int obstacle_id(const AirArgs<T
 // FB pressure update at one interior point: calculation_2D::Cal_pressure
 // (calculation_2D.cpp:598-608) and Update_PML_Qp (air.cpp:2388-2439).  Writes p^{n+1} and
 // the point's Q_p and returns p^{n+1}.
-// L as for air_dp; below 7 the point is also outside the obstacle (the split launches run
-// only without one).
-// XF: the lanes on the x faces take the face node p = p(1 or nx - 2) and its Q_p, as
-// rk_air_point (the Front / Back copy of calculation_2D.cpp:696-705 that the pressure face
-// pass gives such a node).
-template <typename T, bool WIND, bool TERRAIN = false, int L = 7, bool XF = false, bool OBST = true>
+// OBST: the point may lie in an embedded obstacle.
+template <typename T, bool WIND, bool TERRAIN = false, bool OBST = true>
 __device__ __forceinline__ T air_p_point(const AirArgs<T> &a, int i, int j, int k)
 {
     const Grid<T> &g = a.g;
     const size_t id = (size_t)i + (size_t)g.nx * ((size_t)j + (size_t)g.ny * k);
-    if constexpr (L == 0) {
-        const T pnew = g.pn[id] + air_dp<T, WIND ? 1 : 0, TERRAIN, false, 0>(a, i, j, k);
-        g.pnn[id] = pnew;
-        return pnew;
-    }
-    const bool face = XF && (i == 0 || i == g.nx - 1);
-    const OwnQ<T> own = own_slabs<T, L>(a, i, j, k);
+    const OwnQ<T> own = own_slabs<T>(a, i, j, k);
     T qp_old[6];
 #pragma unroll
     for (int s = 0; s < 6; ++s) qp_old[s] = own.in[s] ? a.Qo[s][3][own.idx[s]] : T(0);
-    T r = T(0);
-    if (!face) r = air_dp<T, WIND ? 1 : 0, TERRAIN, false, L>(a, i, j, k);
-    if (const int mo = OBST && L == 7 && !XF ? obstacle_id(a, i, j, k) : 0) {
+    T r = air_dp<T, WIND ? 1 : 0, TERRAIN>(a, i, j, k);
+    if (const int mo = OBST ? obstacle_id(a, i, j, k) : 0) {
         // inside the obstacle the porous-medium continuity equation replaces the increment
         // (air.cpp:2294-2318)
         T mX, mY, mZ;
@@ -687,12 +529,7 @@ __device__ __forceinline__ T air_p_point(const AirArgs<T> &a, int i, int j, int 
                       ((mZ * (g.wn[id + sxy] - g.wn[id])) * g.dzi);
         r = (-a.ogama[mo]) * div;
     }
-    T pnew = g.pn[id] + r;
-    if constexpr (XF) {
-        const int lane = (int)threadIdx.x;
-        const T v = __shfl(pnew, i == 0 ? lane + 1 : i == g.nx - 1 ? lane - 1 : lane, 64);
-        if (face) pnew = v;
-    }
+    const T pnew = g.pn[id] + r;
     g.pnn[id] = pnew;
     // Q_p += dt*p of this point; the value is final, face conditions only touch boundary nodes
 #pragma unroll
@@ -780,22 +617,12 @@ __device__ __forceinline__ void air_duvw(const AirArgs<T> &a, int i, int j, int 
 
 // FB velocity update at one interior point with p at n+1: calculation_2D::Cal_velocity
 // (calculation_2D.cpp:564-574) and Update_PML_Qvw (air.cpp:2323-2386).
-// XF as for air_p_point: u = 0, v and w copied (calculation_2D.cpp:784-864).
-template <typename T, bool WIND, bool TERRAIN = false, int L = 7, bool XF = false, bool OBST = true>
+template <typename T, bool WIND, bool TERRAIN = false, bool OBST = true>
 __device__ __forceinline__ void air_v_point(const AirArgs<T> &a, int i, int j, int k)
 {
     const Grid<T> &g = a.g;
     const size_t id = (size_t)i + (size_t)g.nx * ((size_t)j + (size_t)g.ny * k);
-    if constexpr (L == 0) {
-        T du, dv, dw;
-        air_duvw<T, WIND ? 1 : 0, TERRAIN, false, 0>(a, i, j, k, du, dv, dw);
-        g.unn[id] = g.un[id] + du;
-        g.vnn[id] = g.vn[id] + dv;
-        g.wnn[id] = g.wn[id] + dw;
-        return;
-    }
-    const bool face = XF && (i == 0 || i == g.nx - 1);
-    const OwnQ<T> own = own_slabs<T, L>(a, i, j, k);
+    const OwnQ<T> own = own_slabs<T>(a, i, j, k);
     T qu_old[6], qv_old[6], qw_old[6];
 #pragma unroll
     for (int s = 0; s < 6; ++s) {
@@ -803,10 +630,10 @@ __device__ __forceinline__ void air_v_point(const AirArgs<T> &a, int i, int j, i
         qv_old[s] = own.in[s] ? a.Qo[s][1][own.idx[s]] : T(0);
         qw_old[s] = own.in[s] ? a.Qo[s][2][own.idx[s]] : T(0);
     }
-    T du = T(0), dv = T(0), dw = T(0);
-    if (!face) air_duvw<T, WIND ? 1 : 0, TERRAIN, false, L>(a, i, j, k, du, dv, dw);
+    T du, dv, dw;
+    air_duvw<T, WIND ? 1 : 0, TERRAIN>(a, i, j, k, du, dv, dw);
     const T dt = g.dt;
-    if (const int mo = OBST && L == 7 && !XF ? obstacle_id(a, i, j, k) : 0) {
+    if (const int mo = OBST ? obstacle_id(a, i, j, k) : 0) {
         // inside the obstacle the porous-medium momentum equation replaces the increments
         // (air.cpp:1907-1945)
         T mX, mY, mZ;
@@ -820,12 +647,7 @@ __device__ __forceinline__ void air_v_point(const AirArgs<T> &a, int i, int j, i
         dv = (f * ((mY * (pc - p[id - g.nx])) * g.dyi) + vc * ib) - vc;
         dw = (f * ((mZ * (pc - p[id - sxy])) * g.dzi) + wc * ib) - wc;
     }
-    T un = g.un[id] + du, vn = g.vn[id] + dv, wn = g.wn[id] + dw;
-    if constexpr (XF) {
-        const int lane = (int)threadIdx.x, from = i == 0 ? lane + 1 : i == g.nx - 1 ? lane - 1 : lane;
-        const T v1 = __shfl(vn, from, 64), w1 = __shfl(wn, from, 64);
-        if (face) { un = T(0); vn = v1; wn = w1; }
-    }
+    const T un = g.un[id] + du, vn = g.vn[id] + dv, wn = g.wn[id] + dw;
     g.unn[id] = un;
     g.vnn[id] = vn;
     g.wnn[id] = wn;
@@ -846,120 +668,6 @@ __global__ __launch_bounds__(BX * BY) void k_air_p(const AirArgs<T> a)
     const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y + 1, k = blockIdx.z + 1;
     if (i < 1 || i >= a.g.nx - 1 || j >= a.g.ny - 1) return;
     (void)air_p_point<T, WIND, TERRAIN>(a, i, j, k);
-}
-
-// Split forms of the two passes: a launch per box list, with the layer terms of the slab axes
-// L its points can meet (0 for the interior box, one axis for the faces of the shell, 7 for
-// its edges); together they cover the points of k_air_p / k_air_v with the same arithmetic.
-// The split never runs with an embedded obstacle (split_regions refuses one), so the edge
-// kernels are compiled without the obstacle branch.
-// On the 512 x 256 x 128 grid with its 20-point layers (FP32) the interior launches take
-// 39 + 54 us for 53 % of the points, the layer launches the rest of the 143 + 180 us.
-template <typename T, bool WIND, bool TERRAIN, int L, int NB, bool XF = false>
-__global__ __launch_bounds__(BX * BY) void k_air_p_box(const AirArgs<T> a, const BoxList<NB> l)
-{
-    int i, j, k;
-    list_point(l, blockIdx.x, i, j, k);
-    if (i < (XF ? 0 : 1) || i >= a.g.nx - (XF ? 0 : 1) || j >= a.g.ny - 1) return;
-    (void)air_p_point<T, WIND, TERRAIN, L, XF, false>(a, i, j, k);
-}
-template <typename T, bool WIND, bool TERRAIN, int L, int NB, bool XF = false>
-__global__ __launch_bounds__(BX * BY) void k_air_v_box(const AirArgs<T> a, const BoxList<NB> l)
-{
-    int i, j, k;
-    list_point(l, blockIdx.x, i, j, k);
-    if (i < (XF ? 0 : 1) || i >= a.g.nx - (XF ? 0 : 1) || j >= a.g.ny - 1) return;
-    air_v_point<T, WIND, TERRAIN, L, XF, false>(a, i, j, k);
-}
-
-// The interior box of the split passes without a mean flow, in vector accesses: a lane takes
-// P consecutive points of a row (P * sizeof(T) a multiple of 16 bytes), LT = BX * BY / P lanes
-// one 64 x BY tile of the list, a block of 256 lanes 256 / LT tiles.  Every field the
-// increments read at the points and at their j, k neighbours (j + 1, k + 1 for the pressure,
-// j - 1, k - 1 for the velocity) is one vector load per lane; the i + 1 (i - 1) neighbour of
-// the lane's last (first) point is a load of its own.  Each point's increment is dp_core /
-// duvw_core over the same neighbour values as the one-point form (air_p_point /
-// air_v_point with L = 0), so the bits are the same.  Rows must start aligned to the vector
-// (fb_interior_vec: nx a multiple of P, the arrays' bases aligned).
-template <typename T, int P> using VecP = T __attribute__((ext_vector_type(P)));
-template <typename T, int P> __device__ __forceinline__ VecP<T, P> ldv(gptr<T> f, size_t q)
-{
-    return *(const __attribute__((address_space(1))) VecP<T, P> *)(f.p + q);
-}
-template <typename T, int P> __device__ __forceinline__ void stv(gptr<T> f, size_t q, const VecP<T, P> &v)
-{
-    *(__attribute__((address_space(1))) VecP<T, P> *)(f.p + q) = v;
-}
-// Point (i, j, k) of the lane's first point, false for a padding tile, a tile past the list's
-// end or a row past the last interior one.
-template <typename T, int P>
-__device__ __forceinline__ bool vec_point(const AirArgs<T> &a, const BoxList<1> &l, int ntiles, int &i, int &j, int &k)
-{
-    constexpr int LR = BX / P;
-    const int t = (int)(blockIdx.x * blockDim.y + threadIdx.y);
-    if (t >= ntiles) return false;
-    list_point(l, t, i, j, k);  // i = tile origin + threadIdx.x, j = first row + threadIdx.y + 1
-    if (i < 0) return false;
-    const int lane = (int)threadIdx.x, row = lane / LR;
-    i += (lane - row * LR) * P - lane;
-    j += row - (int)threadIdx.y;
-    return j < a.g.ny - 1 && i >= 1 && i + P <= a.g.nx - 1;
-}
-// The pressure form runs on a separable grid only: over terrain (u and v at k + 1 and the
-// per-column metric tables as well) the four-point pressure pass was slower than the
-// one-point one, and the velocity pass faster.
-template <typename T, int P>
-__global__ __launch_bounds__(256) void k_air_p_vec(const AirArgs<T> a, const BoxList<1> l, int ntiles)
-{
-    typedef VecP<T, P> V;
-    int i, j, k;
-    if (!vec_point<T, P>(a, l, ntiles, i, j, k)) return;
-    const Grid<T> &g = a.g;
-    const size_t nx = (size_t)g.nx, sxy = nx * g.ny, id = (size_t)i + nx * ((size_t)j + (size_t)g.ny * k);
-    const V pc = ldv<T, P>(g.pn, id), uc = ldv<T, P>(g.un, id), vc = ldv<T, P>(g.vn, id), wc = ldv<T, P>(g.wn, id);
-    const V vjp = ldv<T, P>(g.vn, id + nx), wkp = ldv<T, P>(g.wn, id + sxy);
-    const T ulast = g.un[id + P];
-    V out;
-#pragma unroll
-    for (int e = 0; e < P; ++e) {
-        Nb<T> n;
-        n.zX = T(0); n.zY = T(0);
-        metric(g, i + e, j, k, n.mX, n.mY, n.mZ);
-        n.pc = pc[e]; n.uc = uc[e]; n.vc = vc[e]; n.wc = wc[e];
-        n.u_ip = e + 1 < P ? uc[(e + 1) & (P - 1)] : ulast;
-        n.v_jp = vjp[e]; n.w_kp = wkp[e];
-        T ddx, ddy, dwz;
-        out[e] = pc[e] + dp_core<T, 0, false, false>(a, n, ddx, ddy, dwz);
-    }
-    stv<T, P>(g.pnn, id, out);
-}
-template <typename T, bool TERRAIN, int P>
-__global__ __launch_bounds__(256) void k_air_v_vec(const AirArgs<T> a, const BoxList<1> l, int ntiles)
-{
-    typedef VecP<T, P> V;
-    int i, j, k;
-    if (!vec_point<T, P>(a, l, ntiles, i, j, k)) return;
-    const Grid<T> &g = a.g;
-    const size_t nx = (size_t)g.nx, sxy = nx * g.ny, id = (size_t)i + nx * ((size_t)j + (size_t)g.ny * k);
-    const V pc = ldv<T, P>(g.pnn, id), pjm = ldv<T, P>(g.pnn, id - nx), pkm = ldv<T, P>(g.pnn, id - sxy);
-    const V uc = ldv<T, P>(g.un, id), vc = ldv<T, P>(g.vn, id), wc = ldv<T, P>(g.wn, id);
-    const T pfirst = g.pnn[id - 1];
-    V uo, vo, wo;
-#pragma unroll
-    for (int e = 0; e < P; ++e) {
-        Nb<T> n;
-        n.zX = T(0); n.zY = T(0);
-        if constexpr (TERRAIN) metric_terrain(g, i + e, j, k, n.mX, n.mY, n.mZ, n.zX, n.zY);
-        else metric(g, i + e, j, k, n.mX, n.mY, n.mZ);
-        n.uc = uc[e]; n.vc = vc[e]; n.wc = wc[e];
-        n.pc = pc[e];
-        n.p_im = e > 0 ? pc[(e + P - 1) & (P - 1)] : pfirst;
-        n.p_jm = pjm[e]; n.p_km = pkm[e];
-        T gpx, gpy, gpz, du, dv, dw;
-        duvw_core<T, 0, TERRAIN, false>(a, n, gpx, gpy, gpz, du, dv, dw);
-        uo[e] = uc[e] + du; vo[e] = vc[e] + dv; wo[e] = wc[e] + dw;
-    }
-    stv<T, P>(g.unn, id, uo); stv<T, P>(g.vnn, id, vo); stv<T, P>(g.wnn, id, wo);
 }
 
 template <typename T, bool WIND, bool TERRAIN>
@@ -1034,7 +742,7 @@ __global__ __launch_bounds__(64 * (FB_TY + 1)) void k_air_fb(const AirArgs<T> a,
         int ii = i, jj = j, ipp = ip, jpp = jp;
         asm volatile("" : "+v"(ii), "+v"(jj), "+v"(ipp), "+v"(jpp));
         if (!ptask || (face && !faces)) return;
-        const T p = air_p_point<T, WIND, false, 7, false, false>(a, ipp, jpp, k);
+        const T p = air_p_point<T, WIND, false, false>(a, ipp, jpp, k);
         const size_t c = (size_t)ii + (size_t)nx * jj;
         if (face) {
             // Front (calculation_2D.cpp:696-705) or West (676-685) face node
@@ -1058,7 +766,7 @@ __global__ __launch_bounds__(64 * (FB_TY + 1)) void k_air_fb(const AirArgs<T> a,
         if (own) {
             int ii = i, jj = j;
             asm volatile("" : "+v"(ii), "+v"(jj));
-            air_v_point<T, WIND, false, 7, false, false>(a, ii, jj, k);
+            air_v_point<T, WIND, false, false>(a, ii, jj, k);
         }
         if (k + 1 < k1) pressure(k + 1, true);
     }
@@ -1971,69 +1679,10 @@ unsigned flat_blocks(size_t total)
 
 }  // namespace
 
-// Whether the split FB passes take the x-face nodes of the interior rows (the interior is
-// not empty and the East face lane has its neighbour in its own 64-point row); the face
-// passes then walk only the x planes' edge rings.
-template <typename T> bool fb_passes_take_xfaces(const AirArgs<T> &a)
+template <typename T> void launch_air_p(const AirArgs<T> &a, bool wind, hipStream_t s)
 {
-    Regions R;
-    return a.g.nx % BX != 1 && split_regions(a, R, false);
-}
-
-// Points per lane of the interior box's vector form (k_air_p_vec / k_air_v_vec), 0 for the
-// one-point form.
-template <typename T> constexpr int kFbVecP = sizeof(T) == 4 ? 4 : 0;
-// Whether the interior box of the split passes runs the vector form: no mean flow, rows of a
-// multiple of P points and every array of the two time levels aligned to the vector.
-template <typename T> bool fb_interior_vec(const AirArgs<T> &a, bool wind)
-{
-    constexpr int P = kFbVecP<T>;
-    if (P == 0) return false;
-    const Grid<T> &g = a.g;
-    const uintptr_t al = (uintptr_t)(T *)g.un | (uintptr_t)(T *)g.vn | (uintptr_t)(T *)g.wn | (uintptr_t)(T *)g.pn |
-                         (uintptr_t)(T *)g.unn | (uintptr_t)(T *)g.vnn | (uintptr_t)(T *)g.wnn | (uintptr_t)(T *)g.pnn;
-    return !wind && g.nx % P == 0 && al % (P * sizeof(T)) == 0;
-}
-template <typename T, bool TERRAIN, bool PRESSURE>
-void launch_air_vec(const AirArgs<T> &a, const BoxList<1> &l, hipStream_t s)
-{
-    constexpr int P = kFbVecP<T> ? kFbVecP<T> : 1;
-    constexpr int LT = BX * BY / P, TPB = 256 / LT;  // lanes per tile, tiles per block
-    const int nt = (int)list_blocks(l);
-    const dim3 grid((unsigned)((nt + TPB - 1) / TPB)), block(LT, TPB);
-    if constexpr (PRESSURE) {
-        static_assert(!TERRAIN, "the pressure pass's vector form runs on a separable grid");
-        hipLaunchKernelGGL((k_air_p_vec<T, P>), grid, block, 0, s, a, l, nt);
-    } else {
-        hipLaunchKernelGGL((k_air_v_vec<T, TERRAIN, P>), grid, block, 0, s, a, l, nt);
-    }
-}
-
-template <typename T> void launch_air_p(const AirArgs<T> &a, bool wind, hipStream_t s, bool pad, bool vec_ok)
-{
-    dim3 g = interior_grid(a.g.nx, a.g.ny, a.g.nz), b(BX, BY);
-    const bool ter = a.g.tsh != nullptr;
-    Regions R;
-    if (split_regions(a, R, pad)) {
-        // the pressure pass's vector form on a separable grid only
-        const bool xf = fb_passes_take_xfaces<T>(a), vec = vec_ok && !ter && fb_interior_vec<T>(a, wind);
-#define LEE_PS(W, TER)                                                                                       \
-    do {                                                                                                     \
-        if (R.in.n && vec) launch_air_vec<T, false, true>(a, R.in, s);                                          \
-        else if (R.in.n) hipLaunchKernelGGL((k_air_p_box<T, W, TER, 0, 1>), dim3(list_blocks(R.in)), b, 0, s, a, R.in); \
-        if (R.ax[0].n && xf) hipLaunchKernelGGL((k_air_p_box<T, W, TER, 1, 2, true>), dim3(list_blocks(R.ax[0])), b, 0, s, a, R.ax[0]); \
-        else if (R.ax[0].n) hipLaunchKernelGGL((k_air_p_box<T, W, TER, 1, 2>), dim3(list_blocks(R.ax[0])), b, 0, s, a, R.ax[0]); \
-        if (R.ax[1].n) hipLaunchKernelGGL((k_air_p_box<T, W, TER, 2, 2>), dim3(list_blocks(R.ax[1])), b, 0, s, a, R.ax[1]); \
-        if (R.ax[2].n) hipLaunchKernelGGL((k_air_p_box<T, W, TER, 4, 2>), dim3(list_blocks(R.ax[2])), b, 0, s, a, R.ax[2]); \
-        if (R.edge.n && xf) hipLaunchKernelGGL((k_air_p_box<T, W, TER, 7, 12, true>), dim3(list_blocks(R.edge)), b, 0, s, a, R.edge); \
-        else if (R.edge.n) hipLaunchKernelGGL((k_air_p_box<T, W, TER, 7, 12>), dim3(list_blocks(R.edge)), b, 0, s, a, R.edge); \
-    } while (0)
-        if (ter) { if (wind) LEE_PS(true, true); else LEE_PS(false, true); }
-        else { if (wind) LEE_PS(true, false); else LEE_PS(false, false); }
-#undef LEE_PS
-        return;
-    }
-    if (ter) {
+    const dim3 g = interior_grid(a.g.nx, a.g.ny, a.g.nz), b(BX, BY);
+    if (a.g.tsh) {
         if (wind) hipLaunchKernelGGL((k_air_p<T, true, true>), g, b, 0, s, a);
         else hipLaunchKernelGGL((k_air_p<T, false, true>), g, b, 0, s, a);
     } else {
@@ -2041,30 +1690,10 @@ template <typename T> void launch_air_p(const AirArgs<T> &a, bool wind, hipStrea
         else hipLaunchKernelGGL((k_air_p<T, false, false>), g, b, 0, s, a);
     }
 }
-template <typename T> void launch_air_v(const AirArgs<T> &a, bool wind, hipStream_t s, bool pad, bool vec_ok)
+template <typename T> void launch_air_v(const AirArgs<T> &a, bool wind, hipStream_t s)
 {
-    dim3 g = interior_grid(a.g.nx, a.g.ny, a.g.nz), b(BX, BY);
-    const bool ter = a.g.tsh != nullptr;
-    Regions R;
-    if (split_regions(a, R, pad)) {
-        const bool xf = fb_passes_take_xfaces<T>(a), vec = vec_ok && fb_interior_vec<T>(a, wind);
-#define LEE_VS(W, TER)                                                                                       \
-    do {                                                                                                     \
-        if (R.in.n && vec) launch_air_vec<T, TER, false>(a, R.in, s);                                           \
-        else if (R.in.n) hipLaunchKernelGGL((k_air_v_box<T, W, TER, 0, 1>), dim3(list_blocks(R.in)), b, 0, s, a, R.in); \
-        if (R.ax[0].n && xf) hipLaunchKernelGGL((k_air_v_box<T, W, TER, 1, 2, true>), dim3(list_blocks(R.ax[0])), b, 0, s, a, R.ax[0]); \
-        else if (R.ax[0].n) hipLaunchKernelGGL((k_air_v_box<T, W, TER, 1, 2>), dim3(list_blocks(R.ax[0])), b, 0, s, a, R.ax[0]); \
-        if (R.ax[1].n) hipLaunchKernelGGL((k_air_v_box<T, W, TER, 2, 2>), dim3(list_blocks(R.ax[1])), b, 0, s, a, R.ax[1]); \
-        if (R.ax[2].n) hipLaunchKernelGGL((k_air_v_box<T, W, TER, 4, 2>), dim3(list_blocks(R.ax[2])), b, 0, s, a, R.ax[2]); \
-        if (R.edge.n && xf) hipLaunchKernelGGL((k_air_v_box<T, W, TER, 7, 12, true>), dim3(list_blocks(R.edge)), b, 0, s, a, R.edge); \
-        else if (R.edge.n) hipLaunchKernelGGL((k_air_v_box<T, W, TER, 7, 12>), dim3(list_blocks(R.edge)), b, 0, s, a, R.edge); \
-    } while (0)
-        if (ter) { if (wind) LEE_VS(true, true); else LEE_VS(false, true); }
-        else { if (wind) LEE_VS(true, false); else LEE_VS(false, false); }
-#undef LEE_VS
-        return;
-    }
-    if (ter) {
+    const dim3 g = interior_grid(a.g.nx, a.g.ny, a.g.nz), b(BX, BY);
+    if (a.g.tsh) {
         if (wind) hipLaunchKernelGGL((k_air_v<T, true, true>), g, b, 0, s, a);
         else hipLaunchKernelGGL((k_air_v<T, false, true>), g, b, 0, s, a);
     } else {
@@ -2363,15 +1992,14 @@ void launch_copy_words(float *dst, const float *src, size_t n, hipStream_t s)
 }
 
 #define LEE_INST(T)                                                                                          \
-    template void launch_air_p<T>(const AirArgs<T> &, bool, hipStream_t, bool, bool);                              \
-    template void launch_air_v<T>(const AirArgs<T> &, bool, hipStream_t, bool, bool);                              \
+    template void launch_air_p<T>(const AirArgs<T> &, bool, hipStream_t);                                    \
+    template void launch_air_v<T>(const AirArgs<T> &, bool, hipStream_t);                                    \
     template bool fused_fits<T>(int);                                                                        \
     template void launch_rk_air<T>(const RKArgs<T> &, const RKArgs<T> *, int, bool, hipStream_t);            \
     template void launch_rk_pore<T>(const RKPoreArgs<T> &, bool, hipStream_t);                               \
     template void launch_rk_air_batch<T>(const RKArgs<T> *, const int *, int, int, int, bool, int, hipStream_t); \
     template void launch_rk_air_v<T>(const RKArgs<T> &, const RKArgs<T> *, int, bool, int, hipStream_t);     \
     template bool rk_stage_takes_xfaces<T>(const RKArgs<T> &, int);                                           \
-    template bool fb_passes_take_xfaces<T>(const AirArgs<T> &);                                              \
     template void launch_rk_pore_batch<T>(const RKPoreArgs<T> *, const int *, int, int, bool, int, hipStream_t); \
     template void launch_sample_batch<T>(const T *const *, const long long *, int, double *, hipStream_t);     \
     template void launch_air_fb<T>(const AirArgs<T> &, bool, hipStream_t, int);                              \
