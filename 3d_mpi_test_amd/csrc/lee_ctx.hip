@@ -62,8 +62,7 @@ struct lee_ctx {
     bool fused = false;     // both air phases in one kernel (k_air_fb)
     int fb_form = -1;       // FB_p_v air-pass launch form (kFbForms), -1 until tuned
     unsigned fb_mask = 0;   // the forms lee_options.path allows, bit f for form f
-    int rk_variant = -1;    // RK4 air-stage launch shape (kRkTiles index), -1 until tuned
-    bool rk_xfaces = false; // that shape's air stage takes the x-face nodes of the interior rows
+    int rk_variant = -1;    // RK4 air-stage launch shape (lee_options.rk_tile - 1), -1 until tuned
     // row form of the stencils (lee_row.h): whether the domain can run it, its launch plan, the
     // ring of tiles around the interior box, the x layers' merged profiles and the step
     // arguments for either parity of the buffer roles (refreshed when the roles, the y1 gate or
@@ -86,6 +85,8 @@ struct lee_ctx {
     // error ([0] air, [1] porous; u v w p; the air accumulator is one block of the four
     // fields interleaved, at rk_acc[0][0]), and of the auxiliaries (stage state, accumulator)
     void *rk_sb[2][4] = {}, *rk_acc[2][4] = {}, *rk_lo[2][4] = {}, *rk_err[2][4] = {};
+    void *rk_sc[2][4] = {};  // row form: the third stage's state
+    // general form: the auxiliaries' stage state and accumulator
     void *rkq_sb[6][4] = {};
     void *rkq_acc[6][4] = {};  // [s][0]: the slab's four accumulators interleaved ([s][1..3] unused)
     // terrain tables (sh, hx, hy per (i,j); tk per k) of the air [0] and porous [1] grids
@@ -350,7 +351,6 @@ template <typename T> BCArgs<T> bc_args(lee_ctx *c, const AirArgs<T> &aa, double
     if (m.south_porous) b.pore = pore_grid<T>(c);
     else { std::memset(&b.pore, 0, sizeof b.pore); }
     b.porous = m.south_porous; b.iface = m.south_porous && m.iface_copy; b.tdbc = m.east_tdbc; b.y1on = aa.y1on;
-    b.xring = 0;  // the boundary passes walk whole x planes unless a launch shape takes their rows
     b.nb_air = boundary_count<T>(m.nx, m.ny, m.nz);
     b.nb_pore = m.south_porous ? boundary_count<T>(m.pnx, m.pny, m.pnz) : 0;
     for (int s = 0; s < 6; ++s) {
@@ -478,6 +478,18 @@ int upload_frame(lee_ctx *c, int N)
     return LEE_OK;
 }
 
+// Row form RK4: while its time gate is closed the y1 layer's auxiliaries are left alone, whichever
+// set a step starts from, so both sets hold the same values.
+int sync_y1_sets(lee_ctx *c)
+{
+    const Model &m = c->m;
+    if (!m.rk4 || !c->row_ok || !m.slab[2].n) return LEE_OK;
+    const size_t cnt = m.slab[2].count(m.nx, m.ny, m.nz);
+    for (int f = 0; f < 4; ++f)
+        HIPCHK(c, hipMemcpyAsync(c->Q[c->qcur ^ 1][2][f], c->Q[c->qcur][2][f], cnt * c->esz, hipMemcpyDeviceToDevice, c->stream));
+    return LEE_OK;
+}
+
 template <typename T> int frame_shift(lee_ctx *c, int N)
 {
     const Model &m = c->m;
@@ -529,6 +541,7 @@ template <typename T> int frame_shift(lee_ctx *c, int N)
                 launch_shift_yslab<T>((T *)q, (const T *)c->shift_tmp, m.nx, g.n, m.nz, lo, m.ny, tempJ, m.lead, s, c->stream);
             }
         }
+    if (int rc = sync_y1_sets(c)) return rc;
     HIPCHK(c, hipGetLastError());
     return LEE_OK;
 }
@@ -595,6 +608,123 @@ template <typename T> void inject_source(lee_ctx *c, T *p)
                          m.d.src[1], m.d.src[2], gc, c->src_ps[N / c->src_period], c->stream);
 }
 
+// ---- row form: what its kernels need of the domain ------------------------------------
+bool rk_rows(const lee_ctx *c) { return c->m.rk4 && c->row_ok; }
+
+// The records of the frame's rows (ny) and planes (nz) for the gate state (J1, y1on).
+template <typename T> std::vector<RowLine<T>> row_lines_of(const lee_ctx *c, int J1, int y1on)
+{
+    const Model &m = c->m;
+    std::vector<RowLine<T>> lines((size_t)m.ny + m.nz);
+    for (int ax = 1; ax < 3; ++ax)
+        for (int n = 0; n < (ax == 1 ? m.ny : m.nz); ++n) {
+            RowLine<T> &l = lines[(ax == 1 ? 0 : m.ny) + n];
+            std::memset(&l, 0, sizeof l);
+            const SlabGeom &lo = m.slab[2 * ax], &hi = m.slab[2 * ax + 1];
+            const int w1 = ax == 1 ? J1 : m.K1, w2 = ax == 1 ? m.J2 : m.K2, len = ax == 1 ? m.ny : m.nz;
+            const bool in1 = lo.n && n < lo.lo + lo.n && (ax == 2 || y1on), in2 = hi.n && n >= hi.lo;
+            l.m = (T)c->line_m[ax - 1][n];
+            l.t = ax == 2 ? (T)c->line_t[n] : T(0);
+            if (!in1 && !in2) continue;
+            const SlabGeom &g = in1 ? lo : hi;
+            const long long step = ax == 1 ? m.nx : (long long)m.nx * m.ny;
+            l.has = 1;
+            l.act = in1 ? n < w1 : n >= len - w2;
+            l.off = (int)((in1 || !lo.n ? 0 : (long long)lo.count(m.nx, m.ny, m.nz)) + step * (n - g.lo));
+            l.ks = ax == 1 ? m.nx * g.n : 0;
+            const std::vector<double> *pr = c->line_prof[2 * ax + (in1 ? 0 : 1)];
+            l.s = (T)pr[0][n]; l.c = (T)pr[1][n]; l.d = (T)pr[2][n];
+        }
+    return lines;
+}
+RowGeo row_geo(const lee_ctx *c)
+{
+    const Model &m = c->m;
+    const SlabGeom &x1 = m.slab[0], &x2 = m.slab[1];
+    return RowGeo{m.nx, m.ny, m.nz, m.south_porous ? m.pnz : 0, c->plan.p.nty, c->plan.i0, c->plan.j0, x1.lo + x1.n,
+                  x2.n ? x2.lo : INT_MAX, m.I1, x2.n ? m.nx - m.I2 : INT_MAX, x1.n, x2.n,
+                  (x1.n ? (int)x1.count(m.nx, m.ny, m.nz) : 0) - x2.lo, m.south_porous, m.iface_copy, m.ground,
+                  m.east_tdbc, (int)m.ri.size()};
+}
+
+// Arguments of RK4 stage st in row form, from the context's buffer roles: the stages run
+// X -> A -> B -> C -> X, the auxiliaries from set qcur to the other one.
+template <typename T> void rk_row_args(lee_ctx *c, int st, int J1, int y1on, RkRowArgs<T> &r)
+{
+    const Model &m = c->m;
+    std::memset(&r, 0, sizeof r);
+    T *buf[2][4][4];  // air, porous: X A B C
+    for (int d = 0; d < 2; ++d)
+        for (int f = 0; f < 4; ++f) {
+            void **lev = d ? c->pore : c->air;
+            buf[d][0][f] = (T *)lev[c->cur * 4 + f];
+            buf[d][1][f] = (T *)lev[(c->cur ^ 1) * 4 + f];
+            buf[d][2][f] = (T *)c->rk_sb[d][f];
+            buf[d][3][f] = (T *)c->rk_sc[d][f];
+        }
+    r.geo = row_geo(c);
+    r.ntile = c->plan.p.ntx * c->plan.p.nty;
+    r.zair = m.nz - 2;
+    r.yl = (const RowLine<T> *)c->row_lines;
+    r.zl = (const RowLine<T> *)c->row_lines + m.ny;
+    r.xs = (const T *)c->xprof[0]; r.xc = (const T *)c->xprof[1]; r.xd = (const T *)c->xprof[2];
+    r.a = air_args<T>(c, J1, y1on);
+    Grid<T> &g = r.a.g;
+    g.un = buf[0][st][0]; g.vn = buf[0][st][1]; g.wn = buf[0][st][2]; g.pn = buf[0][st][3];
+    g.unn = g.vnn = g.wnn = nullptr;
+    g.pnn = buf[0][st][3];  // the velocity increment reads the stage pressure
+    r.pore = pore_grid<T>(c);
+    r.pore.un = buf[1][st][0]; r.pore.vn = buf[1][st][1]; r.pore.wn = buf[1][st][2]; r.pore.pn = buf[1][st][3];
+    r.pore.unn = r.pore.vnn = r.pore.wnn = r.pore.pnn = nullptr;
+    for (int f = 0; f < 4; ++f) {
+        r.xn[f] = buf[0][0][f]; r.y1[f] = buf[0][1][f];
+        r.pv[f] = buf[0][st ? st - 1 : 0][f];
+        r.dst[f] = buf[0][(st + 1) % 4][f];
+        r.err[f] = (T *)c->rk_err[0][f];
+        r.pxn[f] = buf[1][0][f];
+        r.pdst[f] = buf[1][(st + 1) % 4][f];
+        r.pacc[f] = (T *)c->rk_acc[1][f]; r.plo[f] = (T *)c->rk_lo[1][f]; r.perr[f] = (T *)c->rk_err[1][f];
+    }
+    r.acc = (T *)c->rk_acc[0][0];
+    for (int ax = 0; ax < 3; ++ax) {
+        const int s0 = m.slab[2 * ax].n ? 2 * ax : 2 * ax + 1;
+        for (int f = 0; f < 4; ++f) { r.q[ax].o[f] = (const T *)c->Q[c->qcur][s0][f]; r.q[ax].n[f] = (T *)c->Q[c->qcur ^ 1][s0][f]; }
+    }
+    const T step[4] = {T(0.5), T(0.5), T(1), T(0)};
+    r.ca = step[st];
+    r.cp = st ? step[st - 1] : T(0);
+    r.pgama = (T)m.p_gama; r.peff = (T)m.p_eff;
+    const double E = std::exp(-m.p_beta), E2 = std::exp(-0.5 * m.p_beta);
+    const double cf[5] = {E, E2, E2 * 0.5, E / 6.0, E2 / 3.0};
+    for (int q = 0; q < 5; ++q) r.cf[q] = (T)cf[q];
+    r.rec_idx = c->rec_idx;
+}
+
+// The eight blocks (set qcur 0 and 1, four stages each) of the row kernels' arguments and the
+// rows' records, for the gate state (J1, y1on), uploaded when the buffer roles, the gate or the
+// frame change: a step alternates the auxiliaries' sets and uploads nothing.
+template <typename T> int rk_rows_sync(lee_ctx *c, int J1, int y1on)
+{
+    const std::vector<uintptr_t> key = {(uintptr_t)J1, (uintptr_t)y1on, (uintptr_t)c->cur, c->frame_gen};
+    if (key == c->row_key) return LEE_OK;
+    if (c->capturing) return set_err(c, LEE_ERR_STATE, "step arguments changed inside a captured chunk");
+    const std::vector<RowLine<T>> lines = row_lines_of<T>(c, J1, y1on);
+    std::vector<unsigned char> host(8 * sizeof(RkRowArgs<T>));
+    const int q = c->qcur;
+    for (int n = 0; n < 8; ++n) {
+        RkRowArgs<T> r;
+        c->qcur = n / 4;
+        rk_row_args<T>(c, n % 4, J1, y1on, r);
+        std::memcpy(host.data() + n * sizeof r, &r, sizeof r);
+    }
+    c->qcur = q;
+    HIPCHK(c, hipMemcpyAsync(c->row_args, host.data(), host.size(), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpyAsync(c->row_lines, lines.data(), lines.size() * sizeof(RowLine<T>), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->row_key = key;
+    return LEE_OK;
+}
+
 // Kernel arguments of RK4 stage `st` for the y1 gate state (J1, y1on): stage state -> next
 // stage state of the air, of the porous layer, and the face walks of the destination.
 template <typename T>
@@ -648,12 +778,6 @@ void rk4_stage_args(lee_ctx *c, int st, int J1, int y1on, RKArgs<T> &r, RKPoreAr
     b.b = bc_args<T>(c, r.a, nullptr);
     b.b.tdbc = 0;
     b.b.nrec = 0;
-    c->rk_xfaces = rk_stage_takes_xfaces<T>(r, c->rk_variant);
-    if (c->rk_xfaces) {
-        // the air stage's launch shape takes the x-face nodes of the interior rows
-        b.b.xring = 1;
-        b.b.nb_air = boundary_count<T>(m.nx, m.ny, m.nz, true);
-    }
     b.b.air.unn = dst[0]; b.b.air.vnn = dst[1]; b.b.air.wnn = dst[2]; b.b.air.pnn = dst[3];
     if (m.south_porous) {
         b.b.pore.unn = pdst[0]; b.b.pore.vnn = pdst[1]; b.b.pore.wnn = pdst[2]; b.b.pore.pnn = pdst[3];
@@ -669,15 +793,14 @@ int rk_wind_mode(const Model &m) { return m.has_wind ? (m.wind_v_only ? 2 : 1) :
 // Brings the device copy of the four stage arguments (air stage, then boundary stage: four
 // RKArgs followed by four RKBndArgs) up to date for the gate state (J1, y1on).  A change is rare (frame shifts, the y1 gate opening) and waits for the copy.
 // The arguments depend on the buffer roles (level and auxiliary sets, the FP32 error and
-// second stage buffers a frame shift swaps), the gate state and the air stage's launch shape
-// (which may take the x-face nodes from the boundary stage): that is the key.
+// second stage buffers a frame shift swaps) and the gate state: that is the key.
 template <typename T> int rk_args_sync(lee_ctx *c, int J1, int y1on)
 {
     const size_t sz = sizeof(RKArgs<T>), szb = sizeof(RKBndArgs<T>);
     static_assert(sizeof(RKArgs<T>) % alignof(RKBndArgs<T>) == 0, "boundary blocks follow the air blocks");
-    const uintptr_t key[9] = {(uintptr_t)c->cur, (uintptr_t)c->qcur, (uintptr_t)J1, (uintptr_t)y1on,
+    const uintptr_t key[8] = {(uintptr_t)c->cur, (uintptr_t)c->qcur, (uintptr_t)J1, (uintptr_t)y1on,
                               (uintptr_t)c->rk_sb[0][0], (uintptr_t)c->rk_err[0][0], (uintptr_t)c->rk_sb[1][0],
-                              (uintptr_t)c->rk_err[1][0], (uintptr_t)(intptr_t)c->rk_variant};
+                              (uintptr_t)c->rk_err[1][0]};
     std::vector<unsigned char> now((const unsigned char *)key, (const unsigned char *)key + sizeof key);
     if (c->rk_args_dev && now == c->rk_args_key) return LEE_OK;
     if (c->capturing) return set_err(c, LEE_ERR_STATE, "RK4 stage arguments changed inside a captured chunk");
@@ -708,7 +831,14 @@ template <typename T> int rk_args_peek(lee_ctx *c)
     int J1, y1on;
     gate_tick(c, J1, y1on);
     c->counter = save;
-    return rk_args_sync<T>(c, J1, y1on);
+    return rk_rows(c) ? rk_rows_sync<T>(c, J1, y1on) : rk_args_sync<T>(c, J1, y1on);
+}
+
+// Stage st in row form, launch shape v.
+template <typename T> void rk_row_stage(lee_ctx *c, int st, int v, double *rec)
+{
+    launch_rk_row<T>((const RkRowArgs<T> *)c->row_args + 4 * c->qcur + st, c->plan, st, rk_wind_mode(c->m), c->m.terrain,
+                     c->plan.has_in && v >= kRkSplit, rec, c->stream);
 }
 
 // One RK4 step: launches only (no host synchronisation), receivers into rec_slot.
@@ -716,38 +846,47 @@ template <typename T> void enqueue_rk4_step(lee_ctx *c, double *rec_slot)
 {
     Model &m = c->m;
     hipStream_t s = c->stream;
-    const int nr = (int)m.ri.size();
-    const int wind = rk_wind_mode(m);
     int J1, y1on;
     gate_tick(c, J1, y1on);
-    if (rk_args_sync<T>(c, J1, y1on)) c->args_fault = true;
-    // receivers sample level n before the step (airpore.cpp:573-580)
-    launch_sample<T>((const T *)c->air[c->cur * 4 + 3], c->rec_idx, nr, rec_slot, s);
-    const RKArgs<T> *rd = (const RKArgs<T> *)c->rk_args_dev;
-    const RKBndArgs<T> *bd = (const RKBndArgs<T> *)((const unsigned char *)c->rk_args_dev + 4 * sizeof(RKArgs<T>));
-    for (int st = 0; st < 4; ++st) {
-        RKArgs<T> r;
-        RKPoreArgs<T> pr;
-        RKBndArgs<T> b;
-        rk4_stage_args<T>(c, st, J1, y1on, r, pr, b);
-        prof_mark(c, KS_RK_AIR, true);
-        launch_rk_air_v<T>(r, rd + st, wind, m.terrain, c->rk_variant, s);
-        prof_mark(c, KS_RK_AIR, false);
-        if (m.south_porous) {
-            prof_mark(c, KS_RK_PORE, true);
-            launch_rk_pore<T>(pr, m.terrain, s);
-            prof_mark(c, KS_RK_PORE, false);
+    if (rk_rows(c)) {
+        if (rk_rows_sync<T>(c, J1, y1on)) c->args_fault = true;
+        for (int st = 0; st < 4; ++st) {
+            prof_mark(c, KS_RK_AIR, true);
+            rk_row_stage<T>(c, st, c->rk_variant, rec_slot);
+            prof_mark(c, KS_RK_AIR, false);
         }
-        prof_mark(c, KS_RK_BND, true);
-        launch_rk_bnd<T>(b, bd + st, s);
-        prof_mark(c, KS_RK_BND, false);
+        c->qcur ^= 1;
+    } else {
+        const int nr = (int)m.ri.size();
+        if (rk_args_sync<T>(c, J1, y1on)) c->args_fault = true;
+        // receivers sample level n before the step (airpore.cpp:573-580)
+        launch_sample<T>((const T *)c->air[c->cur * 4 + 3], c->rec_idx, nr, rec_slot, s);
+        const RKArgs<T> *rd = (const RKArgs<T> *)c->rk_args_dev;
+        const RKBndArgs<T> *bd = (const RKBndArgs<T> *)((const unsigned char *)c->rk_args_dev + 4 * sizeof(RKArgs<T>));
+        for (int st = 0; st < 4; ++st) {
+            RKArgs<T> r;
+            RKPoreArgs<T> pr;
+            RKBndArgs<T> b;
+            rk4_stage_args<T>(c, st, J1, y1on, r, pr, b);
+            prof_mark(c, KS_RK_AIR, true);
+            launch_rk_air<T>(r, rd + st, rk_wind_mode(m), m.terrain, s);
+            prof_mark(c, KS_RK_AIR, false);
+            if (m.south_porous) {
+                prof_mark(c, KS_RK_PORE, true);
+                launch_rk_pore<T>(pr, m.terrain, s);
+                prof_mark(c, KS_RK_PORE, false);
+            }
+            prof_mark(c, KS_RK_BND, true);
+            launch_rk_bnd<T>(b, bd + st, s);
+            prof_mark(c, KS_RK_BND, false);
+        }
     }
     inject_source<T>(c, (T *)c->air[c->cur * 4 + 3]);
     c->steps += 1;
 }
 
 // Whether the FB step runs in row form.
-bool fb_rows(const lee_ctx *c) { return c->row_ok && !c->fused; }
+bool fb_rows(const lee_ctx *c) { return !c->m.rk4 && c->row_ok && !c->fused; }
 
 // Brings the row kernels' device arguments up to date for the gate state (J1, y1on): one block
 // per parity of the buffer roles (slot c->cur), which alternate every step, so that a step
@@ -763,26 +902,7 @@ template <typename T> int row_args_sync(lee_ctx *c, int J1, int y1on)
     const std::vector<uintptr_t> key = {(uintptr_t)J1, (uintptr_t)y1on, (uintptr_t)rel, (uintptr_t)p0, (uintptr_t)g0, c->frame_gen};
     if (key == c->row_key) return LEE_OK;
     if (c->capturing) return set_err(c, LEE_ERR_STATE, "step arguments changed inside a captured chunk");
-    std::vector<RowLine<T>> lines((size_t)m.ny + m.nz);
-    for (int ax = 1; ax < 3; ++ax)
-        for (int n = 0; n < (ax == 1 ? m.ny : m.nz); ++n) {
-            RowLine<T> &l = lines[(ax == 1 ? 0 : m.ny) + n];
-            std::memset(&l, 0, sizeof l);
-            const SlabGeom &lo = m.slab[2 * ax], &hi = m.slab[2 * ax + 1];
-            const int w1 = ax == 1 ? J1 : m.K1, w2 = ax == 1 ? m.J2 : m.K2, len = ax == 1 ? m.ny : m.nz;
-            const bool in1 = lo.n && n < lo.lo + lo.n && (ax == 2 || y1on), in2 = hi.n && n >= hi.lo;
-            l.m = (T)c->line_m[ax - 1][n];
-            l.t = ax == 2 ? (T)c->line_t[n] : T(0);
-            if (!in1 && !in2) continue;
-            const SlabGeom &g = in1 ? lo : hi;
-            const long long step = ax == 1 ? m.nx : (long long)m.nx * m.ny;
-            l.has = 1;
-            l.act = in1 ? n < w1 : n >= len - w2;
-            l.off = (int)((in1 || !lo.n ? 0 : (long long)lo.count(m.nx, m.ny, m.nz)) + step * (n - g.lo));
-            l.ks = ax == 1 ? m.nx * g.n : 0;
-            const std::vector<double> *pr = c->line_prof[2 * ax + (in1 ? 0 : 1)];
-            l.s = (T)pr[0][n]; l.c = (T)pr[1][n]; l.d = (T)pr[2][n];
-        }
+    const std::vector<RowLine<T>> lines = row_lines_of<T>(c, J1, y1on);
     std::vector<unsigned char> host(2 * sizeof(RowArgs<T>));
     for (int par = 0; par < 2; ++par) {
         c->cur = par; c->qcur = par ^ rel;
@@ -793,11 +913,7 @@ template <typename T> int row_args_sync(lee_ctx *c, int J1, int y1on)
         std::memset(&r, 0, sizeof r);
         r.a = air_args<T>(c, J1, y1on);
         r.b = bc_args<T>(c, r.a, nullptr);
-        const SlabGeom &x1 = m.slab[0], &x2 = m.slab[1];
-        r.geo = RowGeo{m.nx, m.ny, m.nz, m.south_porous ? m.pnz : 0, c->plan.j0, c->plan.p.nty, x1.lo + x1.n,
-                       x2.n ? x2.lo : INT_MAX, m.I1, x2.n ? m.nx - m.I2 : INT_MAX, x1.n, x2.n,
-                       (x1.n ? (int)x1.count(m.nx, m.ny, m.nz) : 0) - x2.lo, m.south_porous, m.iface_copy, m.ground,
-                       m.east_tdbc, (int)m.ri.size()};
+        r.geo = row_geo(c);
         r.yl = (const RowLine<T> *)c->row_lines;
         r.zl = (const RowLine<T> *)c->row_lines + m.ny;
         r.xs = (const T *)c->xprof[0]; r.xc = (const T *)c->xprof[1]; r.xd = (const T *)c->xprof[2];
@@ -949,11 +1065,13 @@ template <typename T> int graph_steps(lee_ctx *c, int n)
         if (g.n == n && g.cur == c->cur && g.qcur == c->qcur && g.gate_on == gate_on && g.psi == (void *)c->psi &&
             g.gpsi == (void *)c->gpsi) {
             HIPCHK(c, hipGraphLaunch(g.exec, c->stream));
-            if (!m.rk4) {
-                if (n & 1) {
+            if (n & 1) {
+                if (!m.rk4) {
                     c->cur ^= 1; c->qcur ^= 1;
                     if (m.east_tdbc) std::swap(c->psi, c->psi2);
                     if (m.ground) std::swap(c->gpsi, c->gpsi2);
+                } else if (rk_rows(c)) {
+                    c->qcur ^= 1;
                 }
             }
             if (gate) c->counter += n;
@@ -985,50 +1103,27 @@ template <typename T> int graph_steps(lee_ctx *c, int n)
     return LEE_OK;
 }
 
-// Autotuner of the RK4 air stage: times each launch shape on the air and boundary launches of
-// stages 0-2 of the coming step (they read level n and the registers stage 0 rewrites, so
-// repeating them changes nothing the step itself does not overwrite) and keeps the fastest.
+// Autotuner of the RK4 stage: times the whole domain in one launch against the interior box in
+// a launch of its own on stages 0-2 of the coming step (they read level n and the registers
+// stage 0 rewrites, so repeating them changes nothing the step itself does not overwrite) and
+// keeps the faster; without an interior box there is one shape.
 template <typename T> int tune_rk(lee_ctx *c)
 {
     const Model &m = c->m;
-    if (m.opt.rk_tile > 0) {
-        c->rk_variant = std::min(m.opt.rk_tile, kRkVariants) - 1;
+    if (m.opt.rk_tile > 0 || !rk_rows(c) || !c->plan.has_in) {
+        c->rk_variant = m.opt.rk_tile > 0 ? std::min(m.opt.rk_tile, kRkVariants) - 1 : 0;
         return LEE_OK;
     }
-    const long long save = c->counter;
-    int J1, y1on;
-    gate_tick(c, J1, y1on);
-    c->counter = save;
-    // the air and boundary launches of stages 0, 1, 2 of the coming step: stage 0 rewrites the
-    // accumulators and the stage states that 1 and 2 read (from level n, which none of them
-    // writes), so the three can be repeated; stage 3 writes level n and is left out.  The
-    // boundary stage is timed with the air stage because its walks depend on the shape (the
-    // split shapes take the x-face nodes of the interior rows off it).
-    const int wind = rk_wind_mode(m);
-    RKArgs<T> r[3];
-    RKPoreArgs<T> pr;
-    RKBndArgs<T> b[3];
+    int rc = rk_args_peek<T>(c);
+    if (rc) return rc;
+    const int cand[2] = {0, kRkSplit};
+    float t[2] = {1e30f, 1e30f};
     // two passes over the shapes, each shape's best pass kept: shapes a few percent apart
     // are not ranked by one pass's noise
-    float t[kRkVariants];
-    for (int v = 0; v < kRkVariants; ++v) t[v] = 1e30f;
     for (int pass = 0; pass < 2; ++pass)
-        for (int v = 0; v < kRkVariants; ++v) {
-            c->rk_variant = v;  // the stage arguments of this shape (the boundary walks follow it)
-            for (int st = 0; st < 3; ++st) rk4_stage_args<T>(c, st, J1, y1on, r[st], pr, b[st]);
-            int rc = rk_args_sync<T>(c, J1, y1on);
-            if (rc) {
-                c->rk_variant = -1;
-                return rc;
-            }
-            const RKArgs<T> *rd = (const RKArgs<T> *)c->rk_args_dev;
-            const RKBndArgs<T> *bd =
-                (const RKBndArgs<T> *)((const unsigned char *)c->rk_args_dev + 4 * sizeof(RKArgs<T>));
+        for (int q = 0; q < 2; ++q) {
             auto stages = [&]() {
-                for (int st = 0; st < 3; ++st) {
-                    launch_rk_air_v<T>(r[st], rd + st, wind, m.terrain, v, c->stream);
-                    launch_rk_bnd<T>(b[st], bd + st, c->stream);
-                }
+                for (int st = 0; st < 3; ++st) rk_row_stage<T>(c, st, cand[q], c->rec_buf);
             };
             stages();  // warm-up
             HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1037,13 +1132,10 @@ template <typename T> int tune_rk(lee_ctx *c)
             HIPCHK(c, hipEventSynchronize(c->ev1));
             float ms = 0.f;
             HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
-            t[v] = std::min(t[v], ms);
+            t[q] = std::min(t[q], ms);
         }
     HIPCHK(c, hipGetLastError());
-    int pick = 0;
-    for (int v = 1; v < kRkVariants; ++v)
-        if (t[v] < t[pick]) pick = v;
-    c->rk_variant = pick;
+    c->rk_variant = cand[t[1] < t[0] ? 1 : 0];
     return LEE_OK;
 }
 
@@ -1212,7 +1304,7 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
             const long long e = (long long)mm.slab[2 * ax].count(mm.nx, mm.ny, mm.nz) + (long long)mm.slab[2 * ax + 1].count(mm.nx, mm.ny, mm.nz);
             fits = fits && e * (long long)(ax == 0 ? C->esz : 1) < (1LL << 31);
         }
-        C->row_ok = !mm.obstacle && apart && fits && (mm.nx + 63) / 64 < (1 << 16) && mm.ny / 4 < (1 << 14) &&
+        C->row_ok = !mm.obstacle && apart && fits && !(mm.rk4 && mm.south_porous && !mm.iface_copy) && (mm.nx + 63) / 64 < (1 << 16) && mm.ny / 4 < (1 << 14) &&
                     (long long)mm.nz + mm.pnz + 64 < 65536;
         // the boundary kernels decode node indices in 32 bits
         const long long nb = boundary_count<double>(mm.nx, mm.ny, mm.nz) +
@@ -1253,11 +1345,11 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
         C->plan.p.ring = C->plan.v.ring = C->ring;
         for (int q = 0; q < 3; ++q)
             if ((rc = dalloc(C, &C->xprof[q], (size_t)m.nx * es))) return rc;
-        if (!m.rk4) {
-            const size_t sz = C->prec == 64 ? sizeof(RowArgs<double>) : sizeof(RowArgs<float>);
-            const size_t sl = C->prec == 64 ? sizeof(RowLine<double>) : sizeof(RowLine<float>);
-            if ((rc = dalloc(C, &C->row_args, 2 * sz)) || (rc = dalloc(C, &C->row_lines, (size_t)(m.ny + m.nz) * sl))) return rc;
-        }
+        const bool f64 = C->prec == 64;
+        const size_t sz = m.rk4 ? 8 * (f64 ? sizeof(RkRowArgs<double>) : sizeof(RkRowArgs<float>))
+                                : 2 * (f64 ? sizeof(RowArgs<double>) : sizeof(RowArgs<float>));
+        const size_t sl = f64 ? sizeof(RowLine<double>) : sizeof(RowLine<float>);
+        if ((rc = dalloc(C, &C->row_args, sz)) || (rc = dalloc(C, &C->row_lines, (size_t)(m.ny + m.nz) * sl))) return rc;
     }
     int len[6] = {m.nx, m.nx, m.ny, m.ny, m.nz, m.nz};
     size_t qmax = 0;
@@ -1299,6 +1391,7 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
             for (int f = 0; f < 4; ++f) {
                 if ((rc = dalloc(C, &C->rk_sb[d][f], n * es)) || (d == 1 && (rc = dalloc(C, &C->rk_acc[d][f], n * es))))
                     return rc;
+                if (C->row_ok && (rc = dalloc(C, &C->rk_sc[d][f], n * es))) return rc;
                 // FP32: the carried state error; the low part of the accumulator only for the
                 // porous velocities (integrating-factor update)
                 if (C->prec == 32) {
@@ -1307,7 +1400,7 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
                 }
             }
         }
-        for (int s = 0; s < 6; ++s) {
+        for (int s = 0; s < 6 && !C->row_ok; ++s) {
             size_t cnt = m.slab[s].count(m.nx, m.ny, m.nz);
             for (int f = 0; f < 4; ++f)
                 if ((rc = dalloc(C, &C->rkq_sb[s][f], cnt * es))) return rc;
@@ -1716,6 +1809,7 @@ int lee_load_restart(lee_ctx *c, const char *path, int *index)
         for (int q = 0; q < 4; ++q)
             if ((rc = upload(c, c->Q[c->qcur][s][q], Q[q].data(), cnt))) return rc;
     }
+    if ((rc = sync_y1_sets(c))) return rc;
     const int b = c->cur * 4;
     for (int q = 0; q < 4; ++q)
         if ((rc = upload(c, c->air[b + q], f[q].data(), air_n(c)))) return rc;
@@ -1964,7 +2058,7 @@ int lee_kernel_stats(const lee_ctx *c, lee_kstat *out, int cap)
     // stage state, accumulator: stages read 4/12/12/8 and write 8/8/8/4 words); FP32 reads x_n
     // and the carried state error in the last stage and writes the error back (76 words); the
     // porous velocities keep a compensated accumulator (24 words each per step, the pressure
-    // 19); the auxiliaries 64 per slab element and step; the mean flow 1 (V only) or 3 words
+    // 19); the auxiliaries 64 per slab element and step (20 in row form); the mean flow 1 (V only) or 3 words
     // per point and stage; the faces write 4 words per boundary node from 4 source values.
     const double rkw = (c->prec == 32 ? 76.0 : 64.0) / 4.0;
     const double prkw = (c->prec == 32 ? 3 * 24.0 + 19.0 : 64.0) / 4.0;
@@ -1972,19 +2066,18 @@ int lee_kernel_stats(const lee_ctx *c, lee_kstat *out, int cap)
     for (int s = 0; s < 6; ++s) {
         double cnt = (double)m.slab[s].count(m.nx, m.ny, m.nz);
         if (!cnt || (s == 2 && m.J3 == 0)) continue;
-        qrk += cnt * 16.0;
+        qrk += cnt * (rk_rows(c) ? 5.0 : 16.0);
     }
     const double wrk = m.has_wind ? (m.wind_v_only ? 1.0 : 3.0) * m.nx * m.ny * m.nz : 0.0;
-    // x-face nodes of the interior rows, when the RK4 air stage's launch shape takes them
-    const double nxf = c->rk_xfaces ? 2.0 * (m.ny - 2) * (m.nz - 2) : 0.0;
+    const double rr = rk_rows(c) ? 1.0 : 0.0;  // the row form's stage holds the porous layer and the faces as well
     // the row form's FB phases hold the porous layer and the faces as well
     const double fr = !m.rk4 && fb_rows(c) ? 1.0 : 0.0;
     const char *names[KS_N] = {"air_p", "air_v", "pore_p", "pore_v", "air_fb", "bc_p", "bc_v", "rk_air", "rk_pore", "rk_bnd"};
     double bytes[KS_N] = {(5 * (inner + fr * pinner) + qp + wind + 2 * fr * nb) * es,
                           (7 * (inner + fr * pinner) + qv + wind + 6 * fr * nb) * es + fr * psi, 5 * pinner * es,
                           7 * pinner * es, (8 * inner + qf + wind) * es, 2 * nb * es, 6 * nb * es + psi,
-                          (rkw * inner + qrk + wrk + 8 * nxf) * es, prkw * pinner * es, 8 * (nb - nxf) * es};
-    double pts[KS_N] = {inner + fr * pinner, inner + fr * pinner, pinner, pinner, inner, nb, nb, inner, pinner, nb - nxf};
+                          (rkw * inner + qrk + wrk + rr * (prkw * pinner + 8 * nb)) * es, prkw * pinner * es, 8 * nb * es};
+    double pts[KS_N] = {inner + fr * pinner, inner + fr * pinner, pinner, pinner, inner, nb, nb, inner + rr * pinner, pinner, nb};
     int n = 0;
     for (int k = 0; k < KS_N && n < cap; ++k) {
         lee_kstat s = c->kstat[k];
@@ -2060,14 +2153,16 @@ struct lee_ensemble {
     std::string err;
     std::vector<void *> allocs;
     void *air_args[4] = {}, *pore_args[4] = {}, *bnd_args[4] = {};
-    // tile prefixes [air n+1 | pore np+1 | bnd n+1 | air n+1 | pore np+1] (np porous
-    // members): the last two with each member plane's tiles padded to a multiple of 8
-    // (launch form 1)
+    // block prefixes [air n+1 | pore np+1 | bnd n+1 | rows n+1] (np porous members)
     int *first = nullptr;
-    int air_blocks = 0, pore_blocks = 0, bnd_blocks = 0, n_pore = 0, air_blocks_pad = 0, pore_blocks_pad = 0;
-    int form = -1;       // launch form of the air stage (kEnsForms), -1 until tuned
-    int form_pore = -1;  // and of the porous stage (tuned on its own)
-    int form_pin = 0;    // lee_ensemble_set_launch: 0 autotune, 1 + form pinned for both
+    int air_blocks = 0, pore_blocks = 0, bnd_blocks = 0, n_pore = 0;
+    // row form (every member can run it): one launch per stage over all members' tiles, the
+    // arguments of both sets of auxiliaries and four stages, member by member
+    bool rows = false;
+    void *row_args = nullptr;
+    int row_blocks = 0, par = 0;  // par: set the coming step starts from, relative to the tables
+    int form = -1;      // launch form reported (1 + form), -1 before the first step
+    int form_pin = 0;   // lee_ensemble_set_launch
     std::vector<int> key;  // (J1, y1on) per member the tables hold
     int version = 0;
     void **rec_p = nullptr;
@@ -2075,7 +2170,7 @@ struct lee_ensemble {
     double *rec_buf = nullptr;
     int nrec = 0;
     std::vector<int> rec_off;
-    struct Graph { int n, version; hipGraphExec_t exec; };
+    struct Graph { int n, version, par; hipGraphExec_t exec; };
     std::vector<Graph> graphs;
 
     ~lee_ensemble()
@@ -2120,15 +2215,34 @@ template <typename T> int ens_tables(lee_ensemble *e, const std::vector<int> &J1
 {
     const int n = (int)e->m.size();
     EHIP(e, hipStreamSynchronize(e->stream));  // no launch may still read the old tables
-    for (int st = 0; st < 4; ++st) {
+    if (e->rows) {
+        std::vector<RkRowArgs<T>> t((size_t)8 * n);
+        int blocks = 0;
+        for (int d = 0; d < n; ++d) {
+            lee_ctx *c = e->m[d];
+            const std::vector<RowLine<T>> lines = row_lines_of<T>(c, J1[d], y1on[d]);
+            EHIP(e, hipMemcpy(c->row_lines, lines.data(), lines.size() * sizeof(RowLine<T>), hipMemcpyHostToDevice));
+            c->row_key.clear();
+            const int q = c->qcur;
+            for (int s = 0; s < 8; ++s) {
+                RkRowArgs<T> &r = t[(size_t)s * n + d];
+                c->qcur = q ^ (s / 4);
+                rk_row_args<T>(c, s % 4, J1[d], y1on[d], r);
+                r.first = blocks;
+            }
+            c->qcur = q;
+            blocks += (int)row_batch_blocks(c->plan);
+        }
+        e->par = 0;
+        EHIP(e, hipMemcpy(e->row_args, t.data(), t.size() * sizeof(RkRowArgs<T>), hipMemcpyHostToDevice));
+    }
+    for (int st = 0; st < 4 && !e->rows; ++st) {
         std::vector<RKArgs<T>> ra(n);
         std::vector<RKPoreArgs<T>> pa;
         std::vector<RKBndArgs<T>> ba(n);
         for (int d = 0; d < n; ++d) {
             RKPoreArgs<T> pr;
             rk4_stage_args<T>(e->m[d], st, J1[d], y1on[d], ra[d], pr, ba[d]);
-            // the batched air stage takes the x-face nodes whose neighbour is in its wavefront
-            ba[d].b.xring = 2;
             if (e->m[d]->m.south_porous) pa.push_back(pr);
         }
         EHIP(e, hipMemcpy(e->air_args[st], ra.data(), n * sizeof(RKArgs<T>), hipMemcpyHostToDevice));
@@ -2139,20 +2253,6 @@ template <typename T> int ens_tables(lee_ensemble *e, const std::vector<int> &J1
     for (int d = 0; d < n; ++d) { e->key[2 * d] = J1[d]; e->key[2 * d + 1] = y1on[d]; }
     e->version += 1;
     return LEE_OK;
-}
-
-// The air launch (form fa, -1 none) and the porous launch (form fp, -1 none) of RK4 stage st.
-template <typename T> void ens_stage_cells(lee_ensemble *e, int st, int fa, int fp, hipStream_t s)
-{
-    const int n = (int)e->m.size();
-    const int *pa = e->first + (fa == 1 ? 2 * (n + 1) + e->n_pore + 1 : 0);
-    const int *pp = e->first + (fp == 1 ? 3 * (n + 1) + e->n_pore + 1 : n + 1);
-    if (fa >= 0)
-        launch_rk_air_batch<T>((const RKArgs<T> *)e->air_args[st], pa, n, fa == 1 ? e->air_blocks_pad : e->air_blocks,
-                               e->wind, e->terrain, fa, s);
-    if (fp >= 0 && e->n_pore)
-        launch_rk_pore_batch<T>((const RKPoreArgs<T> *)e->pore_args[st], pp, e->n_pore,
-                                fp == 1 ? e->pore_blocks_pad : e->pore_blocks, e->terrain, fp, s);
 }
 
 // Tables current for the coming step (its gate states peeked, the counters left as they are).
@@ -2170,40 +2270,14 @@ template <typename T> int ens_tables_peek(lee_ensemble *e)
     return stale ? ens_tables<T>(e, J1, y1on) : LEE_OK;
 }
 
-// Autotuner of the launch forms: times stage 0's air launch, then its porous launch, of the
-// coming step in each form (stage 0 reads only level n, so repeating it changes nothing) and
-// keeps the fastest for each kind; every form gives the same bits.
-template <typename T> int ens_tune(lee_ensemble *e)
+// Host-side roles after n steps: the row form's auxiliaries alternate between their sets.
+void ens_advance(lee_ensemble *e, int n)
 {
-    if (e->form_pin > 0) {
-        e->form = e->form_pore = e->form_pin - 1;
-        return LEE_OK;
+    for (lee_ctx *c : e->m) {
+        c->steps += n;
+        if (e->rows && (n & 1)) c->qcur ^= 1;
     }
-    int rc = ens_tables_peek<T>(e);
-    if (rc) return rc;
-    int pick[2] = {0, 0};
-    for (int kind = 0; kind < (e->n_pore ? 2 : 1); ++kind) {
-        float t[kEnsForms];
-        for (int f = 0; f < kEnsForms; ++f) t[f] = 1e30f;
-        for (int pass = 0; pass < 2; ++pass)  // each form's best of two passes, as tune_rk
-            for (int f = 0; f < kEnsForms; ++f) {
-                const int fa = kind == 0 ? f : -1, fp = kind == 1 ? f : -1;
-                ens_stage_cells<T>(e, 0, fa, fp, e->stream);  // warm-up
-                EHIP(e, hipEventRecord(e->ev0, e->stream));
-                for (int rep = 0; rep < 4; ++rep) ens_stage_cells<T>(e, 0, fa, fp, e->stream);
-                EHIP(e, hipEventRecord(e->ev1, e->stream));
-                EHIP(e, hipEventSynchronize(e->ev1));
-                float ms = 0.f;
-                EHIP(e, hipEventElapsedTime(&ms, e->ev0, e->ev1));
-                t[f] = std::min(t[f], ms);
-            }
-        for (int f = 1; f < kEnsForms; ++f)
-            if (t[f] < t[pick[kind]]) pick[kind] = f;
-    }
-    EHIP(e, hipGetLastError());
-    e->form = pick[0];
-    e->form_pore = pick[1];
-    return LEE_OK;
+    if (e->rows && (n & 1)) e->par ^= 1;
 }
 
 // One ensemble RK4 step (launches only once the tables are current).
@@ -2222,12 +2296,20 @@ template <typename T> int ens_step(lee_ensemble *e, double *rec_slot)
     }
     hipStream_t s = e->stream;
     launch_sample_batch<T>((const T *const *)e->rec_p, e->rec_idx, e->nrec, rec_slot, s);
-    const int *fb = e->first + n + 1 + e->n_pore + 1;
+    const int *fb = e->first + n + 1 + e->n_pore + 1, *fr = fb + n + 1;
     for (int st = 0; st < 4; ++st) {
-        ens_stage_cells<T>(e, st, e->form, e->form_pore, s);
+        if (e->rows) {
+            launch_rk_row_batch<T>((const RkRowArgs<T> *)e->row_args + (size_t)(4 * e->par + st) * n, fr, n, e->row_blocks, st,
+                                   e->wind, e->terrain, s);
+            continue;
+        }
+        launch_rk_air_batch<T>((const RKArgs<T> *)e->air_args[st], e->first, n, e->air_blocks, e->wind, e->terrain, s);
+        if (e->n_pore)
+            launch_rk_pore_batch<T>((const RKPoreArgs<T> *)e->pore_args[st], e->first + n + 1, e->n_pore, e->pore_blocks,
+                                    e->terrain, s);
         launch_rk_bnd_batch<T>((const RKBndArgs<T> *)e->bnd_args[st], fb, n, e->bnd_blocks, s);
     }
-    for (lee_ctx *c : e->m) c->steps += 1;
+    ens_advance(e, 1);
     return LEE_OK;
 }
 
@@ -2242,10 +2324,7 @@ bool ens_gate_constant(const lee_ensemble *e, int n)
 template <typename T> int ens_run(lee_ensemble *e, int nsteps, double *rec_out, int use_graph)
 {
     hipStream_t s = e->stream;
-    if (e->form < 0) {
-        int rc = ens_tune<T>(e);
-        if (rc) return rc;
-    }
+    if (e->form < 0) e->form = e->form_pin > 0 ? e->form_pin - 1 : 0;
     EHIP(e, hipEventRecord(e->ev0, s));
     int done = 0;
     while (done < nsteps) {
@@ -2258,15 +2337,16 @@ template <typename T> int ens_run(lee_ensemble *e, int nsteps, double *rec_out, 
             if (rc) return rc;
             hipGraphExec_t exec = nullptr;
             for (auto &g : e->graphs)
-                if (g.n == n && g.version == e->version) exec = g.exec;
+                if (g.n == n && g.version == e->version && g.par == e->par) exec = g.exec;
             if (exec) {
                 EHIP(e, hipGraphLaunch(exec, s));
                 for (lee_ctx *c : e->m) {
                     const Model &m = c->m;
                     if (m.judge[1] == 1 || m.judge[1] == 3) c->counter += n;
-                    c->steps += n;
                 }
+                ens_advance(e, n);
             } else {
+                const int par = e->par;
                 EHIP(e, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
                 for (int t = 0; t < n; ++t) {
                     int rc = ens_step<T>(e, e->rec_buf + (size_t)t * e->nrec);
@@ -2274,7 +2354,7 @@ template <typename T> int ens_run(lee_ensemble *e, int nsteps, double *rec_out, 
                 }
                 hipGraph_t graph = nullptr;
                 EHIP(e, hipStreamEndCapture(s, &graph));
-                lee_ensemble::Graph g{n, e->version, nullptr};
+                lee_ensemble::Graph g{n, e->version, par, nullptr};
                 hipError_t ie = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(graph);
                 EHIP(e, ie);
@@ -2347,32 +2427,36 @@ int lee_ensemble_create(int n, const lee_deck *decks, const lee_options *opts, l
             (rc = ens_alloc(E, &E->bnd_args[st], n * sb)))
             return rc;
     }
-    // tile prefixes: interior columns of the air and porous grids in 256s per plane (and the
-    // same with each plane's tiles padded to a multiple of 8), boundary nodes in 256s
-    std::vector<int> fa(1, 0), fp(1, 0), fb(1, 0), fa8(1, 0), fp8(1, 0);
+    // block prefixes: interior columns of the air and porous grids in 256s per plane, boundary
+    // nodes in 256s, tiles of the row form
+    std::vector<int> fa(1, 0), fp(1, 0), fb(1, 0), fr(1, 0);
+    E->rows = true;
+    for (lee_ctx *c : E->m) E->rows = E->rows && c->row_ok;
     for (lee_ctx *c : E->m) {
         const Model &m = c->m;
-        long long ta = batch_blocks(m.nx, m.ny, m.nz), ta8 = batch_blocks(m.nx, m.ny, m.nz, true);
+        const long long ta = batch_blocks(m.nx, m.ny, m.nz), tr = E->rows ? row_batch_blocks(c->plan) : 0;
         long long nb = (c->prec == 64 ? boundary_count<double>(m.nx, m.ny, m.nz) : boundary_count<float>(m.nx, m.ny, m.nz));
         if (m.south_porous) {
             fp.push_back((int)(fp.back() + batch_blocks(m.pnx, m.pny, m.pnz)));
-            fp8.push_back((int)(fp8.back() + batch_blocks(m.pnx, m.pny, m.pnz, true)));
             nb += c->prec == 64 ? boundary_count<double>(m.pnx, m.pny, m.pnz) : boundary_count<float>(m.pnx, m.pny, m.pnz);
         }
-        if (fa8.back() + ta8 > INT_MAX / 2 || fp8.back() > INT_MAX / 2 || fb.back() + (nb + 255) / 256 > INT_MAX / 2)
+        if (fa.back() + ta > INT_MAX / 2 || fp.back() > INT_MAX / 2 || fb.back() + (nb + 255) / 256 > INT_MAX / 2 ||
+            fr.back() + tr > INT_MAX / 2)
             return ens_err(E, LEE_ERR_ARG, "ensemble too large for one launch");
         fa.push_back((int)(fa.back() + ta));
-        fa8.push_back((int)(fa8.back() + ta8));
         fb.push_back((int)(fb.back() + (nb + 255) / 256));
+        fr.push_back((int)(fr.back() + tr));
     }
-    E->air_blocks = fa.back(); E->pore_blocks = fp.back(); E->bnd_blocks = fb.back();
-    E->air_blocks_pad = fa8.back(); E->pore_blocks_pad = fp8.back();
+    E->air_blocks = fa.back(); E->pore_blocks = fp.back(); E->bnd_blocks = fb.back(); E->row_blocks = fr.back();
     E->n_pore = (int)fp.size() - 1;
     std::vector<int> first(fa);
     first.insert(first.end(), fp.begin(), fp.end());
     first.insert(first.end(), fb.begin(), fb.end());
-    first.insert(first.end(), fa8.begin(), fa8.end());
-    first.insert(first.end(), fp8.begin(), fp8.end());
+    first.insert(first.end(), fr.begin(), fr.end());
+    if (E->rows) {
+        const size_t sz = E->prec == 64 ? sizeof(RkRowArgs<double>) : sizeof(RkRowArgs<float>);
+        if ((rc = ens_alloc(E, &E->row_args, (size_t)8 * n * sz))) return rc;
+    }
     if ((rc = ens_alloc(E, (void **)&E->first, first.size() * sizeof(int)))) return rc;
     EHIP(E, hipMemcpy(E->first, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice));
     // receivers of all members, concatenated
@@ -2440,15 +2524,15 @@ int lee_ensemble_set_launch(lee_ensemble *e, int form)
     for (auto &g : e->graphs) (void)hipGraphExecDestroy(g.exec);  // captured with the old form
     e->graphs.clear();
     e->form_pin = form;
-    e->form = e->form_pore = -1;
+    e->form = -1;
     return LEE_OK;
 }
 
 int lee_ensemble_launch(const lee_ensemble *e, int porous)
 {
     if (!e) return 0;
-    const int f = porous ? e->form_pore : e->form;
-    return f >= 0 ? f + 1 : 0;
+    (void)porous;  // one form for both stages
+    return e->form >= 0 ? e->form + 1 : 0;
 }
 
 const char *lee_ensemble_error(const lee_ensemble *e) { return e ? e->err.c_str() : g_global_err.c_str(); }

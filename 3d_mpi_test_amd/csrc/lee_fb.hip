@@ -187,14 +187,14 @@ __global__ __launch_bounds__(RX * RY) void k_row_p(const RowArgs<T> *__restrict_
     const int jr = G.j0 + RY * t.ty + tj, k = t.k;
     const bool row_live = jr >= 1;
     const int j = row_live ? jr : 1;
-    const RowLane l = row_lane(t.tx * RX + lane, nx, row_live);
+    const RowLane l = row_lane(G.i0 + t.tx * RX + lane, nx, row_live);
     __shared__ T rows[RY][RX];
     const bool last = t.ty == L.nty - 1;  // holds rows ny-4 .. ny-2 (uniform over the block)
     T p;
     if (t.kind == RK_AIR) {
         const RowLine<T> yl = row_line(A.yl, j), zl = row_line(A.zl, k);
         const RowSlab<T> sy = row_slab_y(yl, nx, k), sz = row_slab_z(zl, nx, ny, j);
-        const bool mx = row_meets_x(G, t.tx * RX);
+        const bool mx = row_meets_x(G, G.i0 + t.tx * RX);
         const RowX xn = row_x<T>(G, l.in, j, k);
         T qx = T(0), qy = T(0), qz = T(0);
 #define LEE_BODY(X, Y, Z) p = fb_p_point<T, WM, TERRAIN, X, Y, Z>(A, G, l, j, k, yl, zl, sy, sz, xn, qx, qy, qz)
@@ -371,12 +371,12 @@ __global__ __launch_bounds__(RX * RY) void k_row_v(const RowArgs<T> *__restrict_
     const int jr = G.j0 + RY * t.ty + tj, k = t.k;
     if (jr < 1) return;
     const int j = jr;
-    const RowLane l = row_lane(t.tx * RX + lane, nx, true);
+    const RowLane l = row_lane(G.i0 + t.tx * RX + lane, nx, true);
     T f[3];
     if (t.kind == RK_AIR) {
         const RowLine<T> yl = row_line(A.yl, j), zl = row_line(A.zl, k);
         const RowSlab<T> sy = row_slab_y(yl, nx, k), sz = row_slab_z(zl, nx, ny, j);
-        const bool mx = row_meets_x(G, t.tx * RX);
+        const bool mx = row_meets_x(G, G.i0 + t.tx * RX);
         const RowX xn = row_x<T>(G, l.in, j, k);
         T qx[3], qy[3], qz[3];
 #define LEE_BODY(X, Y, Z) fb_v_point<T, WM, TERRAIN, X, Y, Z>(A, G, l, j, k, yl, zl, sy, sz, xn, f, qx, qy, qz)
@@ -498,7 +498,7 @@ __global__ __launch_bounds__(RX * RY) void k_row_in(const RowArgs<T> *__restrict
     const AirArgs<T> &a = A.a;
     const Grid<T> &g = a.g;
     const int tj = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-    const int i = (bx.tx + (int)blockIdx.x) * RX + (int)threadIdx.x, k = bx.k + (int)blockIdx.z;
+    const int i = bx.i0 + (bx.tx + (int)blockIdx.x) * RX + (int)threadIdx.x, k = bx.k + (int)blockIdx.z;
     const int j = bx.j0 + RY * (bx.ty + (int)blockIdx.y) + tj;
     const size_t snx = (size_t)g.nx * sizeof(T), sxy = snx * g.ny;
     const RowAt<T> at{snx * j + sxy * k, snx, sxy, (unsigned)i * (unsigned)sizeof(T)};
@@ -542,7 +542,7 @@ __global__ __launch_bounds__(256) void k_row_in_vec(const RowArgs<T> *__restrict
     const int per = bx.nbx * bx.nby, kk = t / per, c = t - kk * per, ty = c / bx.nbx, tx = c - ty * bx.nbx;
     constexpr int LR = RX / P;
     const int lane = (int)(threadIdx.x & 63), row = lane / LR;
-    const int i = (bx.tx + tx) * RX + (lane - row * LR) * P, j = bx.j0 + RY * (bx.ty + ty) + row, k = bx.k + kk;
+    const int i = bx.i0 + (bx.tx + tx) * RX + (lane - row * LR) * P, j = bx.j0 + RY * (bx.ty + ty) + row, k = bx.k + kk;
     const size_t nx = (size_t)g.nx, sxy = nx * g.ny, id = (size_t)i + nx * ((size_t)j + (size_t)g.ny * k);
     const V uc = ldv<T, P>(g.un, id), vc = ldv<T, P>(g.vn, id), wc = ldv<T, P>(g.wn, id);
     if constexpr (PRESSURE) {
@@ -635,7 +635,7 @@ template <typename T> void launch_row_v(const RowArgs<T> *ad, const RowPlan &pl,
 // every layer and not next to a face), that box and the ring of tiles around it.
 void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
 {
-    const int ntx = (m.nx + RX - 1) / RX, nty = row_tiles(m.ny), j0 = row_first(m.ny);
+    const int i0 = row_left(m.nx), j0 = row_first(m.ny), ntx = (m.nx - i0 + RX - 1) / RX, nty = row_tiles(m.ny);
     // first and one-past-last point of the interior along each axis
     auto span = [](int n, const int *qn, const int *qlo, int w1, int w2, int &a, int &b) {
         a = 2; b = n - 2;
@@ -648,12 +648,13 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
     span(m.nx, m.qn, m.qlo, m.w[0], m.w[1], xa, xb);
     span(m.ny, m.qn + 2, m.qlo + 2, m.w[2], m.w[3], ya, yb);
     span(m.nz, m.qn + 4, m.qlo + 4, m.w[4], m.w[5], za, zb);
-    const int tx0 = (xa + RX - 1) / RX, tx1 = xb / RX;
+    const int tx0 = (xa - i0 + RX - 1) / RX, tx1 = (xb - i0) / RX;
     const int ty0 = (ya - j0 + RY - 1) / RY, ty1 = (yb - j0) / RY;
     pl = RowPlan{};
+    pl.i0 = i0;
     pl.j0 = j0;
     pl.has_in = tx1 > tx0 && ty1 > ty0 && zb > za;
-    if (pl.has_in) pl.in = RowBox{tx0, tx1 - tx0, ty0, ty1 - ty0, za, zb - za, j0};
+    if (pl.has_in) pl.in = RowBox{tx0, tx1 - tx0, ty0, ty1 - ty0, za, zb - za, i0, j0};
     ring.clear();
     if (pl.has_in)
         for (int ty = 0; ty < nty; ++ty)

@@ -100,10 +100,6 @@ template <typename T> struct PoreArgs {
 template <typename T> struct BCArgs {
     Grid<T> air, pore;         // pore.nx == 0 without a porous ground
     int porous, iface, tdbc, y1on;
-    // the x planes' interior-row nodes the air stage takes: 0 none, 1 all (the split launches,
-    // rk_stage_takes_xfaces: the enumeration covers only the edge rings), 2 those of the
-    // batched stage (batch_takes_face; the enumeration skips them)
-    int xring;
     long long nb_air, nb_pore; // boundary nodes of each box
     gptr<const T> Qo[6][4];
     gptr<T> Qn[6][4];
@@ -142,7 +138,8 @@ template <typename T> struct RowLine {
     T s, c, d, m, t;
 };
 struct RowGeo {
-    int nx, ny, nz, pnz, j0, nty;  // j0: row of the first tile's first wavefront
+    int nx, ny, nz, pnz, nty;
+    int i0, j0;  // x and row of the first tile's first lane and wavefront
     int xa, xb, xi1, xi2;          // x1 holds i < xa, x2 i >= xb; terms apply for i < xi1, i >= xi2
     int n0, n1, d2;                // planes of the x slabs, element of (x2, i) minus i
     int porous, coupled, ground, tdbc, nrec;
@@ -161,8 +158,8 @@ template <typename T> struct RowArgs {
     BCArgs<T> b;
 };
 // A box of whole tiles (64 x 4 points) outside every layer: tile columns tx .. tx+nbx-1, tile
-// rows ty .. ty+nby-1 (points j0 + 4 ty ...), planes k .. k+nk-1.
-struct RowBox { int tx, nbx, ty, nby, k, nk, j0; };
+// rows ty .. ty+nby-1 (points i0 + 64 tx ..., rows j0 + 4 ty ...), planes k .. k+nk-1.
+struct RowBox { int tx, nbx, ty, nby, k, nk, i0, j0; };
 // Block ranges of one launch.  Whole domain: a grid of ntx x nty tiles over z = air planes, then
 // porous planes, the ground plane and the receivers.  Around an interior box: blocks first[q] ..
 // first[q+1]-1 of section q (planes 1 .. ka-1, planes kb .., the ring of planes ka .. kb-1 listed
@@ -175,7 +172,7 @@ struct RowLaunch {
 };
 struct RowPlan {
     bool has_in;
-    int j0;  // row of the first tile's first wavefront
+    int i0, j0;
     RowBox in;
     RowLaunch p, v;
 };
@@ -219,72 +216,65 @@ template <typename T> struct RKBndArgs {
     gptr<T> qacc[6][4], qdst[6][4];
     int stage;
 };
+// Row form of an RK4 stage (lee_rk.hip).  The auxiliaries' stage values are not stored: dQ/dt = f
+// is the field itself, so that of stage s at a node is Q_n + a_{s-1} dt y_{s-1} with the previous
+// stage's state there (pv), and Q_{n+1} follows in the last stage from Q_n and the four states
+// at the node -- the sums the stored form rounds the same way.  The three stage states keep a
+// buffer each (A, B, C) and the auxiliaries alternate between two sets.
+template <typename T> struct RkRowArgs {
+    RowGeo geo;
+    int first, ntile, zair;  // ensemble: the member's first block, tiles per plane, air planes
+    gptr<const RowLine<T>> yl, zl;
+    gptr<const T> xs, xc, xd;
+    RowQ<T> q[3];
+    gptr<const T> xn[4], pv[4], y1[4];
+    gptr<T> acc, err[4], dst[4];
+    T ca, cp;                    // a of this stage, a of the previous one
+    AirArgs<T> a;                // stage state in a.g.un .. a.g.pn (= a.g.pnn)
+    Grid<T> pore;                // the porous layer's
+    T pgama, peff, cf[5];
+    gptr<const T> pxn[4];
+    gptr<T> pacc[4], plo[4], perr[4], pdst[4];
+    gptr<const long long> rec_idx;
+};
+// One stage st of a domain: split = the interior box in a launch of its own and the rest in
+// another, else everything in one; stage 0 samples the receivers into rec.
+template <typename T> void launch_rk_row(const RkRowArgs<T> *ad, const RowPlan &pl, int st, int wind, bool terrain, bool split,
+                                         double *rec, hipStream_t s);
+// The same for n domains (their arguments one after the other), nblocks blocks in all.
+template <typename T> void launch_rk_row_batch(const RkRowArgs<T> *ad, const int *first, int n, int nblocks, int st, int wind,
+                                               bool terrain, hipStream_t s);
+inline long long row_batch_blocks(const RowPlan &p) { return (long long)p.v.ntx * p.v.nty * (p.v.zair + p.v.zpore); }
 // wind: 0 none, 1 U V W fields, 2 V only (U = W = 0: velocity_method 7)
 // r: the stage arguments on the host (grid shape), rd: the same in device memory (read by
 // the kernel)
 template <typename T>
 void launch_rk_air(const RKArgs<T> &r, const RKArgs<T> *rd, int wind, bool terrain, hipStream_t s);
-// Launch shapes of the RK4 air stage the autotuner chooses from (variant 0 = launch_rk_air).
-struct RkTile { int ty; bool columns; const char *name; };
-constexpr RkTile kRkTiles[11] = {{4, false, "64x4 planes"}, {4, true, "64x4 xcd-columns"}, {8, true, "64x8 xcd-columns"},
-                                {8, false, "64x8 planes"}, {16, true, "64x16 xcd-columns"},
-                                {4, false, "64x4 interior + layer shell"}, {4, false, "64x4 interior + layers by axis"},
-                                {4, false, "64x4 LDS-staged interior + layer shell"},
-                                {4, false, "64x4 LDS-staged interior + layers by axis"},
-                                {4, false, "64x4 LDS-staged interior + LDS-staged layer shell"},
-                                {4, false, "64x4 LDS-staged interior + LDS-staged layers by axis"}};
-constexpr int kRkVariants = 11;
-template <typename T>
-void launch_rk_air_v(const RKArgs<T> &r, const RKArgs<T> *rd, int wind, bool terrain, int v, hipStream_t s);
-// Whether shape v's air stage also takes the x-face nodes of the interior rows (the boundary
-// stage then walks only the x planes' edge rings: BCArgs::xring).
-template <typename T> bool rk_stage_takes_xfaces(const RKArgs<T> &r, int v);
+// Launch shapes of the RK4 stage (lee_options.rk_tile 1..11, identical bits): up to kRkSplit the
+// whole domain in one launch, above it the interior box in a launch of its own.
+constexpr int kRkVariants = 11, kRkSplit = 5;
 template <typename T> void launch_rk_pore(const RKPoreArgs<T> &r, bool terrain, hipStream_t s);
 // r: the stage arguments on the host (node count), rd: the same in device memory (read by the
 // kernel; by value the block was copied to scratch for the slab indexing)
 template <typename T> void launch_rk_bnd(const RKBndArgs<T> &r, const RKBndArgs<T> *rd, hipStream_t s);
-// Ensemble forms: args[d] in device memory for member d, first[d] = its first block
+// Ensemble, general form: args[d] in device memory for member d, first[d] = its first block
 // (first[n] = nblocks); 256 boundary nodes per block for bnd.  Air and porous blocks of 256
 // threads cover 256 consecutive columns i + nx*(j - 1) of the interior rows j = 1 .. ny-2 of
-// one plane (the member's rows are 64-128 points, so 64-wide tiles would leave about a
-// quarter of the lanes idle): batch_blocks of them per member.
+// one plane: batch_blocks of them per member.
 constexpr int kBatchBlock = 256;
-// Launch forms of the batched air and porous stages (same points, same arithmetic, identical
-// bits; the ensemble's autotuner keeps the fastest):
-//   0  one block per tile, member after member, plane after plane;
-//   1  as 0 with each member plane's tiles padded to a multiple of 8, so that a tile and the
-//      tiles above and below it run on one XCD under round-robin dispatch (padding tiles do
-//      nothing);
-//   2  persistent: as many blocks as the chip holds at once, each walking the tiles of form 0
-//      with a stride of the grid size.
-constexpr int kEnsForms = 3;
-inline long long batch_blocks(int nx, int ny, int nz, bool pad = false)
+constexpr int kEnsForms = 3;  // lee_ensemble_set_launch 1..3: one launch either way
+inline long long batch_blocks(int nx, int ny, int nz)
 {
-    long long per = ((long long)nx * (ny - 2) + kBatchBlock - 1) / kBatchBlock;
-    if (pad) per = (per + 7) & ~7LL;
-    return per * (nz - 2);
+    return ((long long)nx * (ny - 2) + kBatchBlock - 1) / kBatchBlock * (nz - 2);
 }
-// Whether node (i, j) of an interior row is an x-face node the batched air stage takes: its
-// interior neighbour (i + 1 or i - 1, the next or previous column) is in the same wavefront
-// of 64 consecutive columns (blocks start at multiples of 256 columns).  The boundary stage
-// skips exactly these (BCArgs::xring 2).
-__host__ __device__ inline bool batch_takes_face(int nx, int i, int j)
-{
-    if (i != 0 && i != nx - 1) return false;
-    const int c = (j - 1) * nx + i;
-    return i == 0 ? (c & 63) != 63 : (c & 63) != 0;
-}
-// form: kEnsForms; first and nblocks count the tiles of that form (padded for form 1)
 template <typename T>
-void launch_rk_air_batch(const RKArgs<T> *args, const int *first, int n, int nblocks, int wind, bool terrain, int form,
-                         hipStream_t s);
+void launch_rk_air_batch(const RKArgs<T> *args, const int *first, int n, int nblocks, int wind, bool terrain, hipStream_t s);
 template <typename T>
-void launch_rk_pore_batch(const RKPoreArgs<T> *args, const int *first, int n, int nblocks, bool terrain, int form,
-                          hipStream_t s);
+void launch_rk_pore_batch(const RKPoreArgs<T> *args, const int *first, int n, int nblocks, bool terrain, hipStream_t s);
 template <typename T> void launch_rk_bnd_batch(const RKBndArgs<T> *args, const int *first, int n, int nblocks, hipStream_t s);
 template <typename T> void launch_sample_batch(const T *const *p, const long long *idx, int n, double *out, hipStream_t s);
 
-template <typename T> long long boundary_count(int nx, int ny, int nz, bool xring = false);
+template <typename T> long long boundary_count(int nx, int ny, int nz);
 template <typename T> void launch_bc_p_all(const BCArgs<T> &a, hipStream_t s);
 template <typename T> void launch_bc_v_all(const BCArgs<T> &a, hipStream_t s);
 

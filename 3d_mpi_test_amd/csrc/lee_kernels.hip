@@ -36,56 +36,6 @@ __device__ __forceinline__ int xcd_tile(int b, int nb)
 }
 
 
-// A box of 64 x 4-point tiles: tile columns bx .. bx+nbx-1 (points i = 64 bx ...), tile
-// rows by .. by+nby-1 (points j = 4 by + 1 ...), planes k .. k+nk-1.  The split launches
-// cover the tile space of a domain with lists of such boxes, one list per set of slab axes
-// its points can meet (see split_regions).
-struct TileBox {
-    int bx, nbx, by, nby, k, nk;
-};
-constexpr int kMaxBoxes = 18;
-template <int NB> struct BoxList {
-    TileBox b[NB];
-    int first[NB + 1];  // first block of each box; first[n] = blocks in all, then INT_MAX
-    int n;
-    int pad;  // each plane of a box takes a multiple of 8 blocks (list_point)
-};
-
-// Point of block t of a list: thread (threadIdx.x, threadIdx.y) of the box's tiles, taken x
-// fastest, then y, then planes.  blockIdx is uniform, so this is scalar arithmetic on the
-// argument, read at constant offsets only: the box's fields as sums of products with 0/1
-// (selects between loaded values were merged into one load through a selected address,
-// which put the argument in private memory).  With pad each plane of a box takes a multiple
-// of 8 blocks (the extra ones get i = -1 and leave at the bounds check) and the boxes start at
-// multiples of 8: blocks are dealt to the 8 XCDs round-robin, so a tile column then stays on
-// one XCD through its planes, and the planes k - 1, k + 1 a tile reads come from that XCD's
-// L2 (on the 318-tile planes of the 512 x 256 x 128 interior, plane k + 1 of a column went to
-// another XCD and the RK4 stage fetched twice its compulsory reads).  It takes a third off
-// the RK4 stage's HBM reads at the same speed; the FB passes ran 2 % slower with it and
-// stay unpadded.
-template <int NB, int... Q>
-__device__ __forceinline__ void list_point_(const BoxList<NB> &l, int t, int &i, int &j, int &k,
-                                            std::integer_sequence<int, Q...>)
-{
-    const int q = (0 + ... + (int)(Q > 0 && t >= l.first[Q]));
-    const int bx = (0 + ... + ((q == Q) * l.b[Q].bx)), nbx = (0 + ... + ((q == Q) * l.b[Q].nbx));
-    const int by = (0 + ... + ((q == Q) * l.b[Q].by)), nby = (0 + ... + ((q == Q) * l.b[Q].nby));
-    const int k0 = (0 + ... + ((q == Q) * l.b[Q].k)), f = (0 + ... + ((q == Q) * l.first[Q]));
-    t -= f;
-    const int per = nbx * nby, pp = l.pad ? (per + 7) & ~7 : per, kk = t / pp, col = t - kk * pp, ry = col / nbx;
-    if (col >= per) {  // padding: leaves at the caller's bounds check
-        i = -1; j = 1; k = k0;
-        return;
-    }
-    k = k0 + kk;
-    i = (bx + (col - ry * nbx)) * 64 + threadIdx.x;
-    j = (by + ry) * BY + threadIdx.y + 1;
-}
-template <int NB> __device__ __forceinline__ void list_point(const BoxList<NB> &l, int t, int &i, int &j, int &k)
-{
-    list_point_(l, t, i, j, k, std::make_integer_sequence<int, NB>{});
-}
-
 __device__ __forceinline__ size_t qxi(int ii, int j, int k, int n, int ny) { return (size_t)ii + (size_t)n * ((size_t)j + (size_t)ny * k); }
 __device__ __forceinline__ size_t qyi(int i, int jj, int k, int nx, int n) { return (size_t)i + (size_t)nx * ((size_t)jj + (size_t)n * k); }
 __device__ __forceinline__ size_t qzi(int i, int j, int kk, int nx, int ny) { return (size_t)i + (size_t)nx * ((size_t)j + (size_t)ny * kk); }
@@ -95,17 +45,16 @@ template <typename T> struct OwnQ {
     size_t idx[6];
     bool in[6];
 };
-// L as for dp_layers: slabs of the axes left out are known not to hold the point.
-template <typename T, int L = 7> __device__ __forceinline__ OwnQ<T> own_slabs(const AirArgs<T> &a, int i, int j, int k)
+template <typename T> __device__ __forceinline__ OwnQ<T> own_slabs(const AirArgs<T> &a, int i, int j, int k)
 {
     const int nx = a.g.nx, ny = a.g.ny;
     OwnQ<T> o;
-    o.in[0] = (L & 1) && a.qn[0] && i < a.qlo[0] + a.qn[0];
-    o.in[1] = (L & 1) && a.qn[1] && i >= a.qlo[1];
-    o.in[2] = (L & 2) && a.qn[2] && a.y1on && j < a.qlo[2] + a.qn[2];
-    o.in[3] = (L & 2) && a.qn[3] && j >= a.qlo[3];
-    o.in[4] = (L & 4) && a.qn[4] && k < a.qlo[4] + a.qn[4];
-    o.in[5] = (L & 4) && a.qn[5] && k >= a.qlo[5];
+    o.in[0] = a.qn[0] && i < a.qlo[0] + a.qn[0];
+    o.in[1] = a.qn[1] && i >= a.qlo[1];
+    o.in[2] = a.qn[2] && a.y1on && j < a.qlo[2] + a.qn[2];
+    o.in[3] = a.qn[3] && j >= a.qlo[3];
+    o.in[4] = a.qn[4] && k < a.qlo[4] + a.qn[4];
+    o.in[5] = a.qn[5] && k >= a.qlo[5];
     o.idx[0] = o.in[0] ? qxi(i - a.qlo[0], j, k, a.qn[0], ny) : 0;
     o.idx[1] = o.in[1] ? qxi(i - a.qlo[1], j, k, a.qn[1], ny) : 0;
     o.idx[2] = o.in[2] ? qyi(i, j - a.qlo[2], k, nx, a.qn[2]) : 0;
@@ -164,9 +113,7 @@ __device__ __forceinline__ void load_nb(const AirArgs<T> &a, int i, int j, int k
 
 // The layer terms of the pressure increment (air.cpp:2044-2292): the x, y and z slabs with
 // their corner cross terms, added to r in the reference's order.  Reads the auxiliaries a.Qo.
-// L: the slab axes compiled in (bit 0 x, bit 1 y, bit 2 z), for launches whose tiles can only
-// meet those slabs; 7 compiles all.
-template <typename T, bool TERRAIN, int L = 7>
+template <typename T, bool TERRAIN>
 __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int k, T mX, T mY, T mZ, T zX, T zY, T pc,
                                           T ddx, T ddy, T dwz, T &r)
 {
@@ -189,7 +136,7 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
         return v;
     };
     // X1 (air.cpp:2044-2057)
-    if ((L & 1) && i < a.I1) {
+    if (i < a.I1) {
         const T sx = a.x1.s[i], cx = a.x1.c[i];
         const size_t q = qxi(i, j, k, n0, ny), sz = (size_t)n0 * ny;
         gptr<const T> Qv = a.Qo[0][1], Qw = a.Qo[0][2];
@@ -198,7 +145,7 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
         r += A - B;
     }
     // X2 (air.cpp:2059-2074)
-    if ((L & 1) && i >= nx - a.I2) {
+    if (i >= nx - a.I2) {
         const int ii = i - (nx - n1);
         const T sx = a.x2.s[i], cx = a.x2.c[i];
         const size_t q = qxi(ii, j, k, n1, ny), sz = (size_t)n1 * ny;
@@ -210,13 +157,13 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
     // cross term of a y or z layer with an x layer (air.cpp:2091-2115 and the like):
     //   -(Qp_x*sx*so + gP*((1/bx-1)*so*(dQu_x/dX) + (1/bo-1)*sx*(dQ_o/dO)))*dt
     auto xcross_y = [&](T so, T dom) {
-        if ((L & 1) && i < a.I1) {
+        if (i < a.I1) {
             const T sx = a.x1.s[i], dxm = a.x1.d[i];
             const size_t q = qxi(i, j, k, n0, ny), sz = (size_t)n0 * ny;
             const T t1 = (dxm * so) * fX(a.Qo[0][0], q, sz);
             const T t2 = (dom * sx) * fY(a.Qo[0][1], q, n0, sz);
             r += (-((a.Qo[0][3][q] * sx) * so + gP * (t1 + t2))) * dt;
-        } else if ((L & 1) && i >= nx - a.I2) {
+        } else if (i >= nx - a.I2) {
             const int ii = i - (nx - n1);
             const T sx = a.x2.s[i], dxm = a.x2.d[i];
             const size_t q = qxi(ii, j, k, n1, ny), sz = (size_t)n1 * ny;
@@ -226,13 +173,13 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
         }
     };
     auto xcross_z = [&](T so, T dom) {
-        if ((L & 1) && i < a.I1) {
+        if (i < a.I1) {
             const T sx = a.x1.s[i], dxm = a.x1.d[i];
             const size_t q = qxi(i, j, k, n0, ny), sz = (size_t)n0 * ny;
             const T t1 = (dxm * so) * fX(a.Qo[0][0], q, sz);
             const T t2 = (dom * sx) * ((mZ * (a.Qo[0][2][q + sz] - a.Qo[0][2][q])) * dzi);
             r += (-((a.Qo[0][3][q] * sx) * so + gP * (t1 + t2))) * dt;
-        } else if ((L & 1) && i >= nx - a.I2) {
+        } else if (i >= nx - a.I2) {
             const int ii = i - (nx - n1);
             const T sx = a.x2.s[i], dxm = a.x2.d[i];
             const size_t q = qxi(ii, j, k, n1, ny), sz = (size_t)n1 * ny;
@@ -242,7 +189,7 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
         }
     };
     // Y1 (air.cpp:2076-2116)
-    if ((L & 2) && j < a.J1) {
+    if (j < a.J1) {
         const T sy = a.y1.s[j], cy = a.y1.c[j];
         const size_t q = qyi(i, j, k, nx, n2), sz = (size_t)nx * n2;
         gptr<const T> Qu = a.Qo[2][0], Qw = a.Qo[2][2];
@@ -252,7 +199,7 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
         xcross_y(sy, a.y1.d[j]);
     }
     // Y2 (air.cpp:2118-2158)
-    if ((L & 2) && j >= ny - a.J2) {
+    if (j >= ny - a.J2) {
         const int jj = j - (ny - n3);
         const T sy = a.y2.s[j], cy = a.y2.c[j];
         const size_t q = qyi(i, jj, k, nx, n3), sz = (size_t)nx * n3;
@@ -264,13 +211,13 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
     }
     // y-z cross term (air.cpp:2200-2224)
     auto ycross_z = [&](T sz_, T dzm) {
-        if ((L & 2) && j < a.J1) {
+        if (j < a.J1) {
             const T sy = a.y1.s[j], dym = a.y1.d[j];
             const size_t q = qyi(i, j, k, nx, n2), sz = (size_t)nx * n2;
             const T t1 = (dym * sz_) * fY(a.Qo[2][1], q, nx, sz);
             const T t2 = (dzm * sy) * ((mZ * (a.Qo[2][2][q + sz] - a.Qo[2][2][q])) * dzi);
             r += (-((a.Qo[2][3][q] * sy) * sz_ + gP * (t1 + t2))) * dt;
-        } else if ((L & 2) && j >= ny - a.J2) {
+        } else if (j >= ny - a.J2) {
             const int jj = j - (ny - n3);
             const T sy = a.y2.s[j], dym = a.y2.d[j];
             const size_t q = qyi(i, jj, k, nx, n3), sz = (size_t)nx * n3;
@@ -294,14 +241,14 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
         r += A - B;
     };
     // Z1 (air.cpp:2160-2225)
-    if ((L & 4) && k < a.K1) {
+    if (k < a.K1) {
         const T sz = a.z1.s[k], cz = a.z1.c[k];
         zmain(sz, cz, a.Qo[4][0], a.Qo[4][1], qzi(i, j, k, nx, ny));
         xcross_z(sz, a.z1.d[k]);
         ycross_z(sz, a.z1.d[k]);
     }
     // Z2 (air.cpp:2227-2292)
-    if ((L & 4) && k >= nz - a.K2) {
+    if (k >= nz - a.K2) {
         const int kk = k - (nz - n5);
         const T sz = a.z2.s[k], cz = a.z2.c[k];
         zmain(sz, cz, a.Qo[5][0], a.Qo[5][1], qzi(i, j, kk, nx, ny));
@@ -314,7 +261,7 @@ __device__ __forceinline__ void dp_layers(const AirArgs<T> &a, int i, int j, int
 // The layer terms of the velocity increments (air.cpp:1579-1905): the x, y and z slabs with
 // their corner cross terms, added to du, dv, dw in the reference's order.  Reads the pressure
 // auxiliaries a.Qn[.][3] and the velocity auxiliaries a.Qo.
-template <typename T, bool TERRAIN, int L = 7>
+template <typename T, bool TERRAIN>
 __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, int k, T mX, T mY, T mZ, T zX, T zY,
                                             T uc, T vc, T wc, T gpx, T gpy, T gpz, T &du, T &dv, T &dw)
 {
@@ -337,7 +284,7 @@ __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, i
         return v;
     };
     // X1 / X2 (air.cpp:1579-1619)
-    if ((L & 1) && i < a.I1) {
+    if (i < a.I1) {
         const T sx = a.x1.s[i], cx = a.x1.c[i];
         const size_t q = qxi(i, j, k, n0, ny), sz = (size_t)n0 * ny;
         gptr<const T> Qp = a.Qn[0][3];
@@ -345,7 +292,7 @@ __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, i
         dv += ((-sx) * (vc + Aav * bY(Qp, q, n0, sz))) * dt;
         dw += ((-sx) * (wc + Aav * ((mZ * (Qp[q] - Qp[q - sz])) * dzi))) * dt;
     }
-    if ((L & 1) && i >= nx - a.I2) {
+    if (i >= nx - a.I2) {
         const int ii = i - (nx - n1);
         const T sx = a.x2.s[i], cx = a.x2.c[i];
         const size_t q = qxi(ii, j, k, n1, ny), sz = (size_t)n1 * ny;
@@ -360,14 +307,14 @@ __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, i
         du += ((-sy) * (uc + Aav * bX(Qp, qy, szy))) * dt;
         dv += ((cy * Aav) * gpy) * dt - (sy * vc) * dt;
         dw += ((-sy) * (wc + Aav * ((mZ * (Qp[qy] - Qp[qy - szy])) * dzi))) * dt;
-        if ((L & 1) && i < a.I1) {
+        if (i < a.I1) {
             const T sx = a.x1.s[i], dxm = a.x1.d[i];
             const size_t q = qxi(i, j, k, n0, ny), sz = (size_t)n0 * ny;
             gptr<const T> Xp = a.Qn[0][3];
             du += (-((a.Qo[0][0][q] * sx) * sy + ((dxm * sy) * Aav) * bX(Xp, q, sz))) * dt;
             dv += (-((a.Qo[0][1][q] * sx) * sy + ((dym * sx) * Aav) * bY(Xp, q, n0, sz))) * dt;
             dw += (((-a.Qo[0][2][q]) * sx) * sy) * dt;
-        } else if ((L & 1) && i >= nx - a.I2) {
+        } else if (i >= nx - a.I2) {
             const int ii = i - (nx - n1);
             const T sx = a.x2.s[i], dxm = a.x2.d[i];
             const size_t q = qxi(ii, j, k, n1, ny), sz = (size_t)n1 * ny;
@@ -377,21 +324,21 @@ __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, i
             dw += (((-a.Qo[1][2][q]) * sx) * sy) * dt;
         }
     };
-    if ((L & 2) && j < a.J1) ylayer(a.y1.s[j], a.y1.c[j], a.y1.d[j], a.Qn[2][3], qyi(i, j, k, nx, n2), n2);
-    if ((L & 2) && j >= ny - a.J2) ylayer(a.y2.s[j], a.y2.c[j], a.y2.d[j], a.Qn[3][3], qyi(i, j - (ny - n3), k, nx, n3), n3);
+    if (j < a.J1) ylayer(a.y1.s[j], a.y1.c[j], a.y1.d[j], a.Qn[2][3], qyi(i, j, k, nx, n2), n2);
+    if (j >= ny - a.J2) ylayer(a.y2.s[j], a.y2.c[j], a.y2.d[j], a.Qn[3][3], qyi(i, j - (ny - n3), k, nx, n3), n3);
     // z layer with x and y cross terms (air.cpp:1730-1905)
     auto zlayer = [&](T sz, T cz, T dzm, gptr<const T> Qp, size_t qz) {
         du += ((-sz) * (uc + Aav * bX(Qp, qz, sxy))) * dt;
         dv += ((-sz) * (vc + Aav * bY(Qp, qz, nx, sxy))) * dt;
         dw += ((cz * Aav) * gpz) * dt - (sz * wc) * dt;
-        if ((L & 1) && i < a.I1) {
+        if (i < a.I1) {
             const T sx = a.x1.s[i], dxm = a.x1.d[i];
             const size_t q = qxi(i, j, k, n0, ny), s0 = (size_t)n0 * ny;
             gptr<const T> Xp = a.Qn[0][3];
             du += (-((a.Qo[0][0][q] * sx) * sz + ((dxm * sz) * Aav) * bX(Xp, q, s0))) * dt;
             dv += (((-a.Qo[0][1][q]) * sx) * sz) * dt;
             dw += (-((a.Qo[0][2][q] * sx) * sz + ((dzm * sx) * Aav) * ((mZ * (Xp[q] - Xp[q - s0])) * dzi))) * dt;
-        } else if ((L & 1) && i >= nx - a.I2) {
+        } else if (i >= nx - a.I2) {
             const int ii = i - (nx - n1);
             const T sx = a.x2.s[i], dxm = a.x2.d[i];
             const size_t q = qxi(ii, j, k, n1, ny), s1 = (size_t)n1 * ny;
@@ -400,14 +347,14 @@ __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, i
             dv += (((-a.Qo[1][1][q]) * sx) * sz) * dt;
             dw += (-((a.Qo[1][2][q] * sx) * sz + ((dzm * sx) * Aav) * ((mZ * (Xp[q] - Xp[q - s1])) * dzi))) * dt;
         }
-        if ((L & 2) && j < a.J1) {
+        if (j < a.J1) {
             const T sy = a.y1.s[j], dym = a.y1.d[j];
             const size_t q = qyi(i, j, k, nx, n2), s2 = (size_t)nx * n2;
             gptr<const T> Yp = a.Qn[2][3];
             du += (((-a.Qo[2][0][q]) * sy) * sz) * dt;
             dv += (-((a.Qo[2][1][q] * sy) * sz + ((dym * sz) * Aav) * bY(Yp, q, nx, s2))) * dt;
             dw += (-((a.Qo[2][2][q] * sy) * sz + ((dzm * sy) * Aav) * ((mZ * (Yp[q] - Yp[q - s2])) * dzi))) * dt;
-        } else if ((L & 2) && j >= ny - a.J2) {
+        } else if (j >= ny - a.J2) {
             const int jj = j - (ny - n3);
             const T sy = a.y2.s[j], dym = a.y2.d[j];
             const size_t q = qyi(i, jj, k, nx, n3), s3 = (size_t)nx * n3;
@@ -417,8 +364,8 @@ __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, i
             dw += (-((a.Qo[3][2][q] * sy) * sz + ((dzm * sy) * Aav) * ((mZ * (Yp[q] - Yp[q - s3])) * dzi))) * dt;
         }
     };
-    if ((L & 4) && k < a.K1) zlayer(a.z1.s[k], a.z1.c[k], a.z1.d[k], a.Qn[4][3], qzi(i, j, k, nx, ny));
-    if ((L & 4) && k >= nz - a.K2) zlayer(a.z2.s[k], a.z2.c[k], a.z2.d[k], a.Qn[5][3], qzi(i, j, k - (nz - n5), nx, ny));
+    if (k < a.K1) zlayer(a.z1.s[k], a.z1.c[k], a.z1.d[k], a.Qn[4][3], qzi(i, j, k, nx, ny));
+    if (k >= nz - a.K2) zlayer(a.z2.s[k], a.z2.c[k], a.z2.d[k], a.Qn[5][3], qzi(i, j, k - (nz - n5), nx, ny));
 }
 
 // ------------------------------------------------------------------------------------
@@ -431,11 +378,7 @@ __device__ __forceinline__ void duvw_layers(const AirArgs<T> &a, int i, int j, i
 // of the reference's one-sided pair (backward for p, forward for u v w).  The one-sided pair
 // advects the velocity components across the flow with a downwind difference, whose modes
 // grow at up to 2|V|/dy; the central form is neutral.
-// L: the slab axes the point may lie in (bit 0 x, 1 y, 2 z; 7 all, 0 none): the launches over
-// the interior box and over the one-axis parts of the shell below know that the other
-// slabs hold no point of theirs, so those layer terms, which would add nothing, are not
-// compiled in.
-template <typename T, int WM, bool TERRAIN, bool CEN = false, int L = 7>
+template <typename T, int WM, bool TERRAIN, bool CEN = false>
 __device__ __forceinline__ T air_dp(const AirArgs<T> &a, int i, int j, int k)
 {
     const Grid<T> &g = a.g;
@@ -493,7 +436,7 @@ __device__ __forceinline__ T air_dp(const AirArgs<T> &a, int i, int j, int k)
             r += (((-a.gam) * pc) * dt) * ((UX + VY) + WZ);
             r += (((-a.gam) * a.Pav) * dt) * div;
     }
-    if constexpr (L != 0) dp_layers<T, TERRAIN, L>(a, i, j, k, mX, mY, mZ, zX, zY, pc, ddx, ddy, dwz, r);
+    dp_layers<T, TERRAIN>(a, i, j, k, mX, mY, mZ, zX, zY, pc, ddx, ddy, dwz, r);
     return r;
 }
 
@@ -544,7 +487,7 @@ __device__ __forceinline__ T air_p_point(const AirArgs<T> &a, int i, int j, int 
 // and the pressure auxiliaries in a.Qn[.][3] (FB: p^{n+1}; RK4: the stage state), the
 // velocity auxiliaries in a.Qo.
 // ------------------------------------------------------------------------------------
-template <typename T, int WM, bool TERRAIN, bool CEN = false, int L = 7>
+template <typename T, int WM, bool TERRAIN, bool CEN = false>
 __device__ __forceinline__ void air_duvw(const AirArgs<T> &a, int i, int j, int k, T &du_, T &dv_, T &dw_)
 {
     const Grid<T> &g = a.g;
@@ -611,7 +554,7 @@ __device__ __forceinline__ void air_duvw(const AirArgs<T> &a, int i, int j, int 
             dw += (((-uc) * WX) * dt - (vc * WY) * dt) - (wc * WZ) * dt;
             dw += ((-Aav) * dt) * gpz;
     }
-    if constexpr (L != 0) duvw_layers<T, TERRAIN, L>(a, i, j, k, mX, mY, mZ, zX, zY, uc, vc, wc, gpx, gpy, gpz, du, dv, dw);
+    duvw_layers<T, TERRAIN>(a, i, j, k, mX, mY, mZ, zX, zY, uc, vc, wc, gpx, gpy, gpz, du, dv, dw);
     du_ = du; dv_ = dv; dw_ = dw;
 }
 
@@ -907,12 +850,12 @@ __device__ __forceinline__ T rk_update_if(int st, T xn, T k, gptr<T> acc, gptr<T
 
 // Auxiliaries of the point's own slabs: dQ/dt = f (air.cpp:2323-2439 as an ODE) with the RK4
 // register update, f the stage state xc at the point; each slab's reads before its stores.
-template <typename T, int L>
+template <typename T>
 __device__ __forceinline__ void rk_aux_point(const RKArgs<T> &r, int i, int j, int k, const T (&xc)[4])
 {
     const AirArgs<T> &a = r.a;
     const int st = r.stage;
-    const OwnQ<T> own = own_slabs<T, L>(a, i, j, k);
+    const OwnQ<T> own = own_slabs<T>(a, i, j, k);
     const T dt = a.g.dt;
 #pragma unroll
     for (int s = 0; s < 6; ++s)
@@ -931,54 +874,35 @@ __device__ __forceinline__ void rk_aux_point(const RKArgs<T> &r, int i, int j, i
         }
 }
 
-// XF: the lanes on the x faces (i = 0 and nx - 1, rows and planes of the interior) take
-// their face node of the destination state -- u = 0, v, w, p copied from the interior
-// neighbour (calculation_2D.cpp:696-725, 784-864, the values the boundary stage's walks give
-// such a node) -- and the node's auxiliaries, in place of the boundary stage: the lines of
-// those nodes are streamed by this pass anyway, and one node per row costs a line per array
-// in the boundary stage.  The lane is idle otherwise; the neighbour's values come across the
-// wavefront (the face's neighbour lane is in the same 64-point row).
-template <typename T, int WM, bool TERRAIN, bool COMP, int L = 7, bool XF = false>
+template <typename T, int WM, bool TERRAIN, bool COMP>
 __device__ __forceinline__ void rk_air_point(const RKArgs<T> &r, int i, int j, int k)
 {
     const AirArgs<T> &a = r.a;
     const size_t id = (size_t)i + (size_t)a.g.nx * ((size_t)j + (size_t)a.g.ny * k);
     const int st = r.stage;
-    const bool face = XF && (i == 0 || i == a.g.nx - 1);
-    T kf[4] = {T(0), T(0), T(0), T(0)};
-    if (!face) {
-        kf[3] = air_dp<T, WM, TERRAIN, true, L>(a, i, j, k);
-        air_duvw<T, WM, TERRAIN, true, L>(a, i, j, k, kf[0], kf[1], kf[2]);
-    }
+    T kf[4];
+    kf[3] = air_dp<T, WM, TERRAIN, true>(a, i, j, k);
+    air_duvw<T, WM, TERRAIN, true>(a, i, j, k, kf[0], kf[1], kf[2]);
     const T xc[4] = {a.g.un[id], a.g.vn[id], a.g.wn[id], a.g.pn[id]};  // stage state at the point
     // every register read of the point first, then the arithmetic, then the stores
     T xn[4], ac[4] = {T(0), T(0), T(0), T(0)}, er[4];
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
         // level n: the stage state itself at stage 0; not needed by the last FP64 stage
-        xn[f] = (st == 0 || face) ? xc[f] : (!COMP && st == 3) ? T(0) : r.xn[f][id];
-        er[f] = (COMP && st == 3 && !face) ? r.err[f][id] : T(0);
+        xn[f] = st == 0 ? xc[f] : (!COMP && st == 3) ? T(0) : r.xn[f][id];
+        er[f] = (COMP && st == 3) ? r.err[f][id] : T(0);
     }
-    if (st != 0 && !face) acc4_load(r.acc[0], id, ac);
+    if (st != 0) acc4_load(r.acc[0], id, ac);
     T d[4], ao[4], eo[4];
 #pragma unroll
     for (int f = 0; f < 4; ++f) d[f] = rk_regs<T, COMP>(st, xn[f], kf[f], ac[f], er[f], ao[f], eo[f]);
-    if constexpr (XF) {
-        const int lane = (int)threadIdx.x;
-        const int from = i == 0 ? lane + 1 : i == a.g.nx - 1 ? lane - 1 : lane;
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            const T v = __shfl(d[f], from, 64);
-            if (face) d[f] = f == 0 ? T(0) : v;
-        }
-    }
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
         r.dst[f][id] = d[f];
-        if (COMP && st == 3 && !face) r.err[f][id] = eo[f];
+        if (COMP && st == 3) r.err[f][id] = eo[f];
     }
-    if (st < 3 && !face) acc4_store(r.acc[0], id, ao);
-    if constexpr (L != 0) rk_aux_point<T, L>(r, i, j, k, xc);
+    if (st < 3) acc4_store(r.acc[0], id, ao);
+    rk_aux_point<T>(r, i, j, k, xc);
 }
 
 // The stage arguments (some 200 pointers) live in device memory: passed by value they
@@ -990,268 +914,6 @@ __global__ __launch_bounds__(BX * BY) void k_rk_air(const RKArgs<T> *__restrict_
     const int i = blockIdx.x * BX + threadIdx.x, j = blockIdx.y * BY + threadIdx.y + 1, k = blockIdx.z + 1;
     if (i < 1 || i >= r.a.g.nx - 1 || j >= r.a.g.ny - 1) return;
     rk_air_point<T, WM, TERRAIN, COMP>(r, i, j, k);
-}
-
-// Tuned forms of the RK4 air stage: tiles of 64 x TY points and a flat grid.  COLUMNS orders
-// the tiles plane-fastest (a tile's column of planes one after another) and hands each XCD a
-// contiguous run of columns, so the planes k-1 and k+1 a tile reads were loaded into the same
-// XCD's L2 by the tiles just before and after it; otherwise the order is plane by plane.
-template <typename T, int WM, bool TERRAIN, bool COMP, int TY, bool COLUMNS>
-__global__ __launch_bounds__(BX * TY) void k_rk_air_t(const RKArgs<T> *__restrict__ rp)
-{
-    const RKArgs<T> &r = *rp;
-    const int nx = r.a.g.nx, ny = r.a.g.ny, K = r.a.g.nz - 2;
-    const int tx = (nx + BX - 1) / BX, ty = (ny - 2 + TY - 1) / TY;
-    int bx, by, k;
-    if constexpr (COLUMNS) {
-        const int t = xcd_tile(blockIdx.x, gridDim.x);
-        k = t % K + 1;
-        const int col = t / K;
-        bx = col % tx;
-        by = col / tx;
-    } else {
-        const int b = blockIdx.x;
-        bx = b % tx;
-        by = (b / tx) % ty;
-        k = b / (tx * ty) + 1;
-    }
-    const int i = bx * BX + threadIdx.x, j = by * TY + threadIdx.y + 1;
-    if (i < 1 || i >= nx - 1 || j >= ny - 1) return;
-    rk_air_point<T, WM, TERRAIN, COMP>(r, i, j, k);
-}
-
-// Split form of the RK4 air stage (64 x 4 tiles), as k_air_p_box.  The FP32 interior kernel
-// is held to 72 registers (7 waves per SIMD at least): left free it took 77 and ran 6; the
-// FP64 one, and the FP32 one with a uniform mean flow (WM 1), would spill there.
-template <typename T, int WM, bool TERRAIN, bool COMP, int L, int NB, bool XF = false>
-__global__ __launch_bounds__(BX * BY) __attribute__((amdgpu_waves_per_eu((COMP && L == 0 && WM != 1) ? 7 : 1, 8))) void k_rk_air_box(
-    const RKArgs<T> *__restrict__ rp, const BoxList<NB> l)
-{
-    const RKArgs<T> &r = *rp;
-    int i, j, k;
-    list_point(l, blockIdx.x, i, j, k);
-    if (i < (XF ? 0 : 1) || i >= r.a.g.nx - (XF ? 0 : 1) || j >= r.a.g.ny - 1) return;
-    rk_air_point<T, WM, TERRAIN, COMP, L, XF>(r, i, j, k);
-}
-
-// Interior RK4 air stage with the stage state staged through LDS.  Each block copies the
-// fields its 64 x 4 tile reads -- u, v, w, p (and the mean flow V) on plane k with a halo of a
-// 16-byte chunk in x and a row in y, and on planes k - 1, k + 1 the tile's own points -- into
-// LDS with global_load_lds (16 bytes per lane, no registers held while the loads are in
-// flight, so a block has its whole stencil input in flight at once), then every point takes
-// its neighbours from LDS and runs the same dp_core / duvw_core and register update as
-// rk_air_point: the same bits.  Mean flows of velocity_method 0 and 7; rows a multiple of 16
-// bytes (nx % (16 / sizeof(T)) == 0), so every chunk is aligned.
-template <typename T> struct Stage {
-    static constexpr int H = 16 / (int)sizeof(T);   // elements per chunk, the x halo
-    static constexpr int W = BX + 2 * H;            // a plane-k row: i0 - H .. i0 + 63 + H
-    static constexpr int PK = (BY + 2) * W;         // plane k: rows j0 - 1 .. j0 + BY
-    static constexpr int PS = BY * BX;              // planes k -+ 1: the tile's own points
-    static constexpr int SZ = PK + 2 * PS;          // one field
-    static constexpr int CK = PK / H, CS = PS / H;  // 16-byte chunks
-    static constexpr int GK = (CK + 63) / 64, GS = CS / 64;  // wave loads per part
-    static constexpr int G = GK + 2 * GS;           // wave loads per field
-    static_assert(CS % 64 == 0, "side planes are whole wave loads");
-};
-typedef __attribute__((address_space(3))) void lds_void;
-
-// Only grid points are loaded: chunks outside x = 0 .. nx - 1 or rows outside 0 .. ny - 1 (the
-// planes k -+ 1: 0 .. ny - 2, the rows of points) are left out, which no point of the grid
-// reads (tiles of the layer shell reach past the faces); the caller keeps nx a multiple of H.
-template <typename T, int NF>
-__device__ __forceinline__ void stage_fields(gptr<const T> const (&F)[5], T *lds, int nx, int ny, size_t sxy, int i0,
-                                             int j0, int k)
-{
-    using S = Stage<T>;
-    const int lane = threadIdx.x;
-    // wave w (= threadIdx.y) issues the loads g = f * G + part with g % BY == w; the loops run
-    // at compile time so that every field pointer is read at a constant index
-#pragma unroll
-    for (int f = 0; f < NF; ++f)
-#pragma unroll
-        for (int part = 0; part < S::G; ++part) {
-            if ((f * S::G + part) % BY != (int)threadIdx.y) continue;
-            int c, limit, off, x, y, ylim;
-            size_t e;
-            if (part < S::GK) {  // plane k, row by row of W elements
-                c = part * 64 + lane;
-                const int r = c / (S::W / S::H), cc = c - r * (S::W / S::H);
-                x = i0 - S::H + cc * S::H;
-                y = j0 - 1 + r;
-                ylim = ny;
-                e = sxy * (size_t)k;
-                limit = S::CK;
-                off = f * S::SZ + part * 64 * S::H;
-            } else {  // plane k - 1 (side 0) or k + 1 (side 1), the tile's rows
-                const int q = part - S::GK, side = q / S::GS, gq = q - side * S::GS;
-                c = gq * 64 + lane;
-                const int r = c / (BX / S::H), cc = c - r * (BX / S::H);
-                x = i0 + cc * S::H;
-                y = j0 + r;
-                ylim = ny - 1;
-                e = sxy * (size_t)(side ? k + 1 : k - 1);
-                limit = S::CS;
-                off = f * S::SZ + S::PK + side * S::PS + gq * 64 * S::H;
-            }
-            if (x < 0 || x >= nx || y >= ylim) continue;
-            e += (size_t)x + (size_t)nx * (size_t)y;
-            if (c < limit)
-                __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) const void *)(F[f] + e),
-                                                 (lds_void *)(lds + off), 16, 0, 0);
-        }
-}
-
-template <typename T, int WM, bool TERRAIN, bool COMP>
-__global__ __launch_bounds__(BX * BY) void k_rk_air_lds(const RKArgs<T> *__restrict__ rp, const BoxList<1> l)
-{
-    static_assert(WM == 0 || WM == 2, "uniform mean flows take the register path");
-    using S = Stage<T>;
-    constexpr int NF = WM == 2 ? 5 : 4;
-    __shared__ T lds[NF * S::SZ];
-    const RKArgs<T> &r = *rp;
-    const AirArgs<T> &a = r.a;
-    const Grid<T> &g = a.g;
-    int i, j, k;
-    list_point(l, blockIdx.x, i, j, k);
-    if (i < 1) return;  // a padding block (uniform over the block: no barrier is left waiting)
-    const int ti = threadIdx.x, tj = threadIdx.y;
-    const size_t nx = (size_t)g.nx, sxy = (size_t)g.nx * g.ny;
-    const size_t id = (size_t)i + nx * ((size_t)j + (size_t)g.ny * k);
-    {
-        gptr<const T> const F[5] = {g.un, g.vn, g.wn, g.pn, a.V};
-        stage_fields<T, NF>(F, lds, g.nx, g.ny, sxy, i - ti, j - tj, k);
-    }
-    // the point's registers while the stage state is in flight
-    const int st = r.stage;
-    T xn[4], ac[4] = {T(0), T(0), T(0), T(0)}, er[4];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        xn[f] = (st == 0 || (!COMP && st == 3)) ? T(0) : r.xn[f][id];
-        er[f] = (COMP && st == 3) ? r.err[f][id] : T(0);
-    }
-    if (st != 0) acc4_load(r.acc[0], id, ac);
-    Nb<T> n;
-    n.zX = T(0); n.zY = T(0);
-    if constexpr (TERRAIN) metric_terrain(g, i, j, k, n.mX, n.mY, n.mZ, n.zX, n.zY);
-    else metric(g, i, j, k, n.mX, n.mY, n.mZ);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    auto K = [&](int f, int di, int dj) { return lds[f * S::SZ + (tj + 1 + dj) * S::W + (ti + S::H + di)]; };
-    auto M = [&](int f) { return lds[f * S::SZ + S::PK + tj * BX + ti]; };
-    auto P = [&](int f) { return lds[f * S::SZ + S::PK + S::PS + tj * BX + ti]; };
-    n.uc = K(0, 0, 0); n.u_ip = K(0, 1, 0); n.u_jp = K(0, 0, 1); n.u_jm = K(0, 0, -1); n.u_kp = P(0); n.u_km = M(0);
-    n.vc = K(1, 0, 0); n.v_jp = K(1, 0, 1); n.v_jm = K(1, 0, -1); n.v_kp = P(1); n.v_km = M(1);
-    n.wc = K(2, 0, 0); n.w_jp = K(2, 0, 1); n.w_jm = K(2, 0, -1); n.w_kp = P(2); n.w_km = M(2);
-    n.pc = K(3, 0, 0); n.p_im = K(3, -1, 0); n.p_jp = K(3, 0, 1); n.p_jm = K(3, 0, -1); n.p_kp = P(3); n.p_km = M(3);
-    if constexpr (WM == 2) {
-        n.Vc = K(4, 0, 0); n.V_ip = K(4, 1, 0); n.V_im = K(4, -1, 0); n.V_jp = K(4, 0, 1); n.V_jm = K(4, 0, -1);
-        n.V_kp = P(4); n.V_km = M(4);
-    }
-    T kf[4], ddx, ddy, dwz, gpx, gpy, gpz;
-    kf[3] = dp_core<T, WM, TERRAIN, true>(a, n, ddx, ddy, dwz);
-    duvw_core<T, WM, TERRAIN, true>(a, n, gpx, gpy, gpz, kf[0], kf[1], kf[2]);
-    const T xc[4] = {n.uc, n.vc, n.wc, n.pc};
-    if (st == 0) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) xn[f] = xc[f];
-    }
-    T d[4], ao[4], eo[4];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) d[f] = rk_regs<T, COMP>(st, xn[f], kf[f], ac[f], er[f], ao[f], eo[f]);
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        r.dst[f][id] = d[f];
-        if (COMP && st == 3) r.err[f][id] = eo[f];
-    }
-    if (st < 3) acc4_store(r.acc[0], id, ao);
-}
-
-// The layer shell (or one part of it, L its slab axes) with the stage state staged through LDS
-// as k_rk_air_lds stages the interior's: the same core on LDS operands, then the layer terms,
-// the register update, the x-face lanes (XF) and the auxiliaries exactly as rk_air_point has
-// them, so the bits are the same.  Every thread of a block stages and meets the barrier; the
-// points outside the grid's interior rows leave after it.
-template <typename T, int WM, bool TERRAIN, bool COMP, int L, int NB, bool XF>
-__global__ __launch_bounds__(BX * BY) __attribute__((amdgpu_waves_per_eu(COMP ? 7 : 1, 8))) void k_rk_air_lds_box(const RKArgs<T> *__restrict__ rp, const BoxList<NB> l)
-{
-    static_assert(WM == 0 || WM == 2, "uniform mean flows take the register path");
-    using S = Stage<T>;
-    constexpr int NF = WM == 2 ? 5 : 4;
-    __shared__ T lds[NF * S::SZ];
-    const RKArgs<T> &r = *rp;
-    const AirArgs<T> &a = r.a;
-    const Grid<T> &g = a.g;
-    int i, j, k;
-    list_point(l, blockIdx.x, i, j, k);
-    if (i < 0) return;  // a padding block (uniform over the block)
-    const int ti = threadIdx.x, tj = threadIdx.y, nx = g.nx;
-    const size_t sxy = (size_t)nx * g.ny;
-    {
-        gptr<const T> const F[5] = {g.un, g.vn, g.wn, g.pn, a.V};
-        stage_fields<T, NF>(F, lds, nx, g.ny, sxy, i - ti, j - tj, k);
-    }
-    const bool live = i >= (XF ? 0 : 1) && i < nx - (XF ? 0 : 1) && j < g.ny - 1;
-    const bool face = XF && (i == 0 || i == nx - 1);
-    const size_t id = live ? (size_t)i + (size_t)nx * ((size_t)j + (size_t)g.ny * k) : 0;
-    const int st = r.stage;
-    T xn[4], ac[4] = {T(0), T(0), T(0), T(0)}, er[4];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        xn[f] = (!live || st == 0 || face || (!COMP && st == 3)) ? T(0) : r.xn[f][id];
-        er[f] = (live && COMP && st == 3 && !face) ? r.err[f][id] : T(0);
-    }
-    if (live && st != 0 && !face) acc4_load(r.acc[0], id, ac);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (!live) return;
-    auto K = [&](int f, int di, int dj) { return lds[f * S::SZ + (tj + 1 + dj) * S::W + (ti + S::H + di)]; };
-    auto M = [&](int f) { return lds[f * S::SZ + S::PK + tj * BX + ti]; };
-    auto P = [&](int f) { return lds[f * S::SZ + S::PK + S::PS + tj * BX + ti]; };
-    const T xc[4] = {K(0, 0, 0), K(1, 0, 0), K(2, 0, 0), K(3, 0, 0)};  // stage state at the point
-    T kf[4] = {T(0), T(0), T(0), T(0)};
-    if (!face) {
-        Nb<T> n;
-        n.zX = T(0); n.zY = T(0);
-        if constexpr (TERRAIN) metric_terrain(g, i, j, k, n.mX, n.mY, n.mZ, n.zX, n.zY);
-        else metric(g, i, j, k, n.mX, n.mY, n.mZ);
-        n.uc = xc[0]; n.u_ip = K(0, 1, 0); n.u_jp = K(0, 0, 1); n.u_jm = K(0, 0, -1); n.u_kp = P(0); n.u_km = M(0);
-        n.vc = xc[1]; n.v_jp = K(1, 0, 1); n.v_jm = K(1, 0, -1); n.v_kp = P(1); n.v_km = M(1);
-        n.wc = xc[2]; n.w_jp = K(2, 0, 1); n.w_jm = K(2, 0, -1); n.w_kp = P(2); n.w_km = M(2);
-        n.pc = xc[3]; n.p_im = K(3, -1, 0); n.p_jp = K(3, 0, 1); n.p_jm = K(3, 0, -1); n.p_kp = P(3); n.p_km = M(3);
-        if constexpr (WM == 2) {
-            n.Vc = K(4, 0, 0); n.V_ip = K(4, 1, 0); n.V_im = K(4, -1, 0); n.V_jp = K(4, 0, 1); n.V_jm = K(4, 0, -1);
-            n.V_kp = P(4); n.V_km = M(4);
-        }
-        T ddx, ddy, dwz, gpx, gpy, gpz;
-        kf[3] = dp_core<T, WM, TERRAIN, true>(a, n, ddx, ddy, dwz);
-        if constexpr (L != 0) dp_layers<T, TERRAIN, L>(a, i, j, k, n.mX, n.mY, n.mZ, n.zX, n.zY, n.pc, ddx, ddy, dwz, kf[3]);
-        duvw_core<T, WM, TERRAIN, true>(a, n, gpx, gpy, gpz, kf[0], kf[1], kf[2]);
-        if constexpr (L != 0)
-            duvw_layers<T, TERRAIN, L>(a, i, j, k, n.mX, n.mY, n.mZ, n.zX, n.zY, n.uc, n.vc, n.wc, gpx, gpy, gpz, kf[0],
-                                       kf[1], kf[2]);
-    }
-    if (st == 0 || face) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) xn[f] = xc[f];
-    }
-    T d[4], ao[4], eo[4];
-#pragma unroll
-    for (int f = 0; f < 4; ++f) d[f] = rk_regs<T, COMP>(st, xn[f], kf[f], ac[f], er[f], ao[f], eo[f]);
-    if constexpr (XF) {
-        const int from = i == 0 ? ti + 1 : i == nx - 1 ? ti - 1 : ti;
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            const T v = __shfl(d[f], from, 64);
-            if (face) d[f] = f == 0 ? T(0) : v;
-        }
-    }
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        r.dst[f][id] = d[f];
-        if (COMP && st == 3 && !face) r.err[f][id] = eo[f];
-    }
-    if (st < 3 && !face) acc4_store(r.acc[0], id, ao);
-    if constexpr (L != 0) rk_aux_point<T, L>(r, i, j, k, xc);
 }
 
 // Ensemble form: one launch steps every member.  The flat block index selects the member by
@@ -1268,13 +930,11 @@ __device__ __forceinline__ int batch_member(const int *first, int n, int b)
 }
 
 // Point of thread (threadIdx.x, threadIdx.y) in tile `local` of a member: tiles of 256
-// consecutive columns c = i + nx*(j - 1) over the interior rows, plane after plane (a plane's
-// tile count rounded up to a multiple of 8 when `pad`); false for a face column (i = 0,
-// nx - 1) or past the last row (every point of a padding tile).
-__device__ __forceinline__ bool batch_point(int nx, int ny, bool pad, int local, int &i, int &j, int &k)
+// consecutive columns c = i + nx*(j - 1) over the interior rows, plane after plane; false for a
+// face column (i = 0, nx - 1) or past the last row.
+__device__ __forceinline__ bool batch_point(int nx, int ny, int local, int &i, int &j, int &k)
 {
-    int per = (nx * (ny - 2) + kBatchBlock - 1) / kBatchBlock;
-    if (pad) per = (per + 7) & ~7;
+    const int per = (nx * (ny - 2) + kBatchBlock - 1) / kBatchBlock;
     const int c = (local % per) * kBatchBlock + threadIdx.x + BX * threadIdx.y;
     k = local / per + 1;
     j = c / nx + 1;
@@ -1282,31 +942,13 @@ __device__ __forceinline__ bool batch_point(int nx, int ny, bool pad, int local,
     return j < ny - 1 && i >= 1 && i < nx - 1;
 }
 
-// The batched stage also takes the x-face nodes of the interior rows whose interior neighbour
-// is in the same wavefront (batch_takes_face), as the split single-domain launches do
-// (rk_air_point with XF): the face lane runs the same code as the others and takes the
-// neighbour's values across the wavefront.
 template <typename T, int WM, bool TERRAIN, bool COMP>
-__device__ __forceinline__ void rk_air_tile(const RKArgs<T> *__restrict__ args, const int *__restrict__ first, int n,
-                                            int tile, bool pad)
+__global__ __launch_bounds__(BX * BY) void k_rk_air_batch(const RKArgs<T> *__restrict__ args, const int *__restrict__ first, int n)
 {
-    const int d = batch_member(first, n, tile);
+    const int tile = blockIdx.x, d = batch_member(first, n, tile);
     const RKArgs<T> &r = args[d];
-    const int nx = r.a.g.nx, ny = r.a.g.ny;
     int i, j, k;
-    const bool in = batch_point(nx, ny, pad, tile - first[d], i, j, k);
-    if (in || (j < ny - 1 && batch_takes_face(nx, i, j))) rk_air_point<T, WM, TERRAIN, COMP, 7, true>(r, i, j, k);
-}
-template <typename T, int WM, bool TERRAIN, bool COMP, int FORM>
-__global__ __launch_bounds__(BX * BY) void k_rk_air_batch(const RKArgs<T> *__restrict__ args, const int *__restrict__ first,
-                                                         int n, int ntiles)
-{
-    if constexpr (FORM == 2) {
-        // the tile index is uniform over the block, so every wave of it takes the same trips
-        for (int t = blockIdx.x; t < ntiles; t += gridDim.x) rk_air_tile<T, WM, TERRAIN, COMP>(args, first, n, t, false);
-    } else {
-        rk_air_tile<T, WM, TERRAIN, COMP>(args, first, n, blockIdx.x, FORM == 1);
-    }
+    if (batch_point(r.a.g.nx, r.a.g.ny, tile - first[d], i, j, k)) rk_air_point<T, WM, TERRAIN, COMP>(r, i, j, k);
 }
 
 // Porous layer: dt*R_p = -gama div u (porous.cpp:77-95); dt*R_u = -dt eff grad p, with the
@@ -1361,24 +1003,12 @@ __global__ __launch_bounds__(BX * BY) void k_rk_pore(const RKPoreArgs<T> r)
 }
 
 template <typename T, bool TERRAIN, bool COMP>
-__device__ __forceinline__ void rk_pore_tile(const RKPoreArgs<T> *__restrict__ args, const int *__restrict__ first, int n,
-                                             int tile, bool pad)
+__global__ __launch_bounds__(BX * BY) void k_rk_pore_batch(const RKPoreArgs<T> *__restrict__ args, const int *__restrict__ first, int n)
 {
-    const int d = batch_member(first, n, tile);
+    const int tile = blockIdx.x, d = batch_member(first, n, tile);
     const RKPoreArgs<T> &r = args[d];
-    const int nx = r.g.nx, ny = r.g.ny;
     int i, j, k;
-    if (batch_point(nx, ny, pad, tile - first[d], i, j, k)) rk_pore_point<T, TERRAIN, COMP>(r, i, j, k);
-}
-template <typename T, bool TERRAIN, bool COMP, int FORM>
-__global__ __launch_bounds__(BX * BY) void k_rk_pore_batch(const RKPoreArgs<T> *__restrict__ args,
-                                                          const int *__restrict__ first, int n, int ntiles)
-{
-    if constexpr (FORM == 2) {
-        for (int t = blockIdx.x; t < ntiles; t += gridDim.x) rk_pore_tile<T, TERRAIN, COMP>(args, first, n, t, false);
-    } else {
-        rk_pore_tile<T, TERRAIN, COMP>(args, first, n, blockIdx.x, FORM == 1);
-    }
+    if (batch_point(r.g.nx, r.g.ny, tile - first[d], i, j, k)) rk_pore_point<T, TERRAIN, COMP>(r, i, j, k);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1592,84 +1222,6 @@ __global__ __launch_bounds__(256) void k_stream_words(StreamPtrs p, size_t n)
 // face threads i = 0 and i = nx - 1 return at once); y and z start at the first interior plane.
 dim3 interior_grid(int nx, int ny, int nz) { return dim3((nx + BX - 1) / BX, (ny - 2 + BY - 1) / BY, nz - 2); }
 
-// The split of a domain's tile space by the slab axes its tiles can meet.  Along each axis the
-// tiles fall in three ranges: before, inside and after the range wholly outside that axis's
-// layers (the terms of dp_layers / duvw_layers and the auxiliaries of own_slabs).  A box of
-// three inside ranges is the interior (no layer terms), one with a single outside range meets
-// only that axis's slabs, the rest (edges and corners of the shell) may meet any.  False when
-// the interior is empty or an obstacle is embedded: the full launch then covers the domain.
-struct Regions {
-    BoxList<1> in;        // the interior
-    BoxList<2> ax[3];     // the shell's parts that meet only x, only y, only z slabs
-    BoxList<12> edge;     // the rest of the shell (edges and corners)
-    BoxList<6> shell;     // the whole shell: planes below and above the interior, then rows
-                          // before and after it, then columns left and right of it
-};
-template <int NB> void pack(BoxList<NB> &l, const std::vector<TileBox> &v, bool pad)
-{
-    l.n = (int)v.size();
-    l.pad = pad ? 1 : 0;
-    l.first[0] = 0;
-    for (int q = 0; q < NB; ++q) {
-        const int per = q < l.n ? v[q].nbx * v[q].nby : 0;
-        l.b[q] = q < l.n ? v[q] : TileBox{0, 1, 0, 1, 1, 1};
-        l.first[q + 1] = q < l.n ? l.first[q] + (pad ? (per + 7) & ~7 : per) * v[q].nk : INT_MAX;
-    }
-}
-template <typename T> bool split_regions(const AirArgs<T> &a, Regions &R, bool pad)
-{
-    const int nx = a.g.nx, ny = a.g.ny, nz = a.g.nz;
-    if (a.omask) return false;
-    int xa = std::max(1, a.I1), xb = std::min(nx - 1, nx - a.I2);
-    int ya = std::max(1, a.J1), yb = std::min(ny - 1, ny - a.J2);
-    int za = std::max(1, a.K1), zb = std::min(nz - 1, nz - a.K2);
-    if (a.qn[0]) xa = std::max(xa, a.qlo[0] + a.qn[0]);
-    if (a.qn[1]) xb = std::min(xb, a.qlo[1]);
-    if (a.qn[2]) ya = std::max(ya, a.qlo[2] + a.qn[2]);
-    if (a.qn[3]) yb = std::min(yb, a.qlo[3]);
-    if (a.qn[4]) za = std::max(za, a.qlo[4] + a.qn[4]);
-    if (a.qn[5]) zb = std::min(zb, a.qlo[5]);
-    const int bx0 = (xa + BX - 1) / BX, bx1 = xb / BX;            // tiles [64 bx, 64 bx + 64) in [xa, xb)
-    const int by0 = (ya - 1 + BY - 1) / BY, by1 = (yb - 1) / BY;  // rows [BY by + 1, BY by + BY + 1) in [ya, yb)
-    if (bx1 <= bx0 || by1 <= by0 || zb <= za) return false;
-    const int TX = (nx + BX - 1) / BX, TYt = (ny - 2 + BY - 1) / BY;
-    // ranges (start, count) before / inside / after, per axis
-    const int X[3][2] = {{0, bx0}, {bx0, bx1 - bx0}, {bx1, TX - bx1}};
-    const int Y[3][2] = {{0, by0}, {by0, by1 - by0}, {by1, TYt - by1}};
-    const int Z[3][2] = {{1, za - 1}, {za, zb - za}, {zb, nz - 1 - zb}};
-    std::vector<TileBox> in, ax[3], edge, shell;
-    auto add = [](std::vector<TileBox> &l, int x0, int nbx, int y0, int nby, int z0, int nk) {
-        if (nbx > 0 && nby > 0 && nk > 0) l.push_back(TileBox{x0, nbx, y0, nby, z0, nk});
-    };
-    for (int cz = 0; cz < 3; ++cz)
-        for (int cy = 0; cy < 3; ++cy) {
-            const int outs = (cy != 1) + (cz != 1);
-            if (outs == 2) {  // an edge for every x range: one box across x
-                add(edge, 0, TX, Y[cy][0], Y[cy][1], Z[cz][0], Z[cz][1]);
-                continue;
-            }
-            for (int cx = 0; cx < 3; ++cx) {
-                const int o = outs + (cx != 1);
-                std::vector<TileBox> &l = o == 0 ? in : o == 2 ? edge : cx != 1 ? ax[0] : cy != 1 ? ax[1] : ax[2];
-                add(l, X[cx][0], X[cx][1], Y[cy][0], Y[cy][1], Z[cz][0], Z[cz][1]);
-            }
-        }
-    const int nk = zb - za;
-    add(shell, 0, TX, 0, TYt, 1, za - 1);
-    add(shell, 0, TX, 0, TYt, zb, nz - 1 - zb);
-    add(shell, 0, TX, 0, by0, za, nk);
-    add(shell, 0, TX, by1, TYt - by1, za, nk);
-    add(shell, 0, bx0, by0, by1 - by0, za, nk);
-    add(shell, bx1, TX - bx1, by0, by1 - by0, za, nk);
-    pack(R.in, in, pad);
-    for (int q = 0; q < 3; ++q) pack(R.ax[q], ax[q], pad);
-    pack(R.edge, edge, pad);
-    pack(R.shell, shell, pad);
-    return true;
-}
-template <int NB> unsigned list_blocks(const BoxList<NB> &l) { return (unsigned)l.first[l.n]; }
-
-
 unsigned flat_blocks(size_t total)
 {
     size_t b = (total + 255) / 256;
@@ -1715,151 +1267,13 @@ void launch_rk_air(const RKArgs<T> &r, const RKArgs<T> *rd, int wind, bool terra
 #undef LEE_RK
 }
 
-// Variant v of the tuned stage launch (lee_ctx keeps the autotuner's choice): v = 0 the
-// plane-by-plane 64x4 grid, 1..4 the flat grids of kRkTiles, 5 and 6 the split launches of
-// split_regions: the interior and the shell, or the interior and the shell by slab axes; 7 and
-// 8 as 5 and 6 with the interior staged through LDS, 9 and 10 with the shell staged as well
-// (5 and 6 for a uniform mean flow or rows not a multiple of 16 bytes).  v = 0 when the
-// interior is empty.
-// Whether launch shape v of the stage takes the x-face nodes of the interior rows (the split
-// shapes, when the interior is not empty and the East face lane has its neighbour in its own
-// 64-point row); the boundary stage then walks only the x planes' edge rings.
-template <typename T> bool rk_stage_takes_xfaces(const RKArgs<T> &r, int v)
-{
-    Regions R;
-    return v >= 5 && v <= 10 && r.a.g.nx % BX != 1 && split_regions(r.a, R, true);
-}
-
 template <typename T>
-void launch_rk_air_v(const RKArgs<T> &r, const RKArgs<T> *rd, int wind, bool terrain, int v, hipStream_t s)
-{
-    // the layer shell by slab axes: x, y, z layers and the edges (Regions R, block b, C, xf)
-#define LEE_RK_AXES(WM, TER)                                                                                      \
-    do {                                                                                                        \
-        if (R.ax[0].n && xf) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 1, 2, true>), dim3(list_blocks(R.ax[0])), b, 0, s, rd, R.ax[0]); \
-        else if (R.ax[0].n) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 1, 2>), dim3(list_blocks(R.ax[0])), b, 0, s, rd, R.ax[0]); \
-        if (R.ax[1].n) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 2, 2>), dim3(list_blocks(R.ax[1])), b, 0, s, rd, R.ax[1]); \
-        if (R.ax[2].n) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 4, 2>), dim3(list_blocks(R.ax[2])), b, 0, s, rd, R.ax[2]); \
-        if (R.edge.n && xf) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 7, 12, true>), dim3(list_blocks(R.edge)), b, 0, s, rd, R.edge); \
-        else if (R.edge.n) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 7, 12>), dim3(list_blocks(R.edge)), b, 0, s, rd, R.edge); \
-    } while (0)
-    Regions R;
-    if (v <= 0 || (v >= 5 && !split_regions(r.a, R, true))) { launch_rk_air<T>(r, rd, wind, terrain, s); return; }
-    const bool xf = rk_stage_takes_xfaces<T>(r, v);
-    constexpr bool C = std::is_same<T, float>::value;
-    if (v >= 7 && v <= 10 && wind != 1 && r.a.g.nx % Stage<T>::H == 0) {
-        // the interior staged through LDS; the shell as v 5 (whole) or v 6 (by slab axes),
-        // from registers (v 7, 8) or staged through LDS as well (v 9, 10)
-        const dim3 b(BX, BY);
-#define LEE_RKLS(WM, TER, LL, NB, LIST)                                                                            \
-    do {                                                                                                        \
-        if (LIST.n && xf) hipLaunchKernelGGL((k_rk_air_lds_box<T, WM, TER, C, LL, NB, true>), dim3(list_blocks(LIST)), b, 0, s, rd, LIST); \
-        else if (LIST.n) hipLaunchKernelGGL((k_rk_air_lds_box<T, WM, TER, C, LL, NB, false>), dim3(list_blocks(LIST)), b, 0, s, rd, LIST); \
-    } while (0)
-#define LEE_RKL(WM, TER)                                                                                          \
-    do {                                                                                                        \
-        if (R.in.n) hipLaunchKernelGGL((k_rk_air_lds<T, WM, TER, C>), dim3(list_blocks(R.in)), b, 0, s, rd, R.in); \
-        if (v == 9) { LEE_RKLS(WM, TER, 7, 6, R.shell); break; }                                                \
-        if (v == 10) {                                                                                          \
-            LEE_RKLS(WM, TER, 1, 2, R.ax[0]);                                                                   \
-            if (R.ax[1].n) hipLaunchKernelGGL((k_rk_air_lds_box<T, WM, TER, C, 2, 2, false>), dim3(list_blocks(R.ax[1])), b, 0, s, rd, R.ax[1]); \
-            if (R.ax[2].n) hipLaunchKernelGGL((k_rk_air_lds_box<T, WM, TER, C, 4, 2, false>), dim3(list_blocks(R.ax[2])), b, 0, s, rd, R.ax[2]); \
-            LEE_RKLS(WM, TER, 7, 12, R.edge);                                                                   \
-            break;                                                                                              \
-        }                                                                                                       \
-        if (v == 7) {                                                                                           \
-            if (R.shell.n && xf) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 7, 6, true>), dim3(list_blocks(R.shell)), b, 0, s, rd, R.shell); \
-            else if (R.shell.n) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 7, 6>), dim3(list_blocks(R.shell)), b, 0, s, rd, R.shell); \
-            break;                                                                                              \
-        }                                                                                                       \
-        LEE_RK_AXES(WM, TER);                                                                                   \
-    } while (0)
-        if (terrain) { if (wind == 2) LEE_RKL(2, true); else LEE_RKL(0, true); }
-        else { if (wind == 2) LEE_RKL(2, false); else LEE_RKL(0, false); }
-#undef LEE_RKL
-#undef LEE_RKLS
-        return;
-    }
-    if (v == 7 || v == 9) v = 5;
-    if (v == 8 || v == 10) v = 6;
-    if (v >= 5) {
-        const dim3 b(BX, BY);
-#define LEE_RKS(WM, TER)                                                                                          \
-    do {                                                                                                        \
-        if (R.in.n) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 0, 1>), dim3(list_blocks(R.in)), b, 0, s, rd, R.in); \
-        if (v == 5) {                                                                                           \
-            if (R.shell.n && xf) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 7, 6, true>), dim3(list_blocks(R.shell)), b, 0, s, rd, R.shell); \
-            else if (R.shell.n) hipLaunchKernelGGL((k_rk_air_box<T, WM, TER, C, 7, 6>), dim3(list_blocks(R.shell)), b, 0, s, rd, R.shell); \
-            break;                                                                                              \
-        }                                                                                                       \
-        LEE_RK_AXES(WM, TER);                                                                                   \
-    } while (0)
-        if (terrain) {
-            if (wind == 1) LEE_RKS(1, true); else if (wind == 2) LEE_RKS(2, true); else LEE_RKS(0, true);
-        } else {
-            if (wind == 1) LEE_RKS(1, false); else if (wind == 2) LEE_RKS(2, false); else LEE_RKS(0, false);
-        }
-#undef LEE_RKS
-        return;
-    }
-    const int nx = r.a.g.nx, ny = r.a.g.ny, K = r.a.g.nz - 2;
-    const int TYv = kRkTiles[v].ty;
-    const unsigned nb = (unsigned)(((nx + BX - 1) / BX) * ((ny - 2 + TYv - 1) / TYv) * K);
-#define LEE_RKT(TY, COL)                                                                              \
-    do {                                                                                              \
-        if (terrain) {                                                                                \
-            if (wind == 1) hipLaunchKernelGGL((k_rk_air_t<T, 1, true, C, TY, COL>), dim3(nb), dim3(BX, TY), 0, s, rd);  \
-            else if (wind == 2) hipLaunchKernelGGL((k_rk_air_t<T, 2, true, C, TY, COL>), dim3(nb), dim3(BX, TY), 0, s, rd); \
-            else hipLaunchKernelGGL((k_rk_air_t<T, 0, true, C, TY, COL>), dim3(nb), dim3(BX, TY), 0, s, rd); \
-        } else {                                                                                      \
-            if (wind == 1) hipLaunchKernelGGL((k_rk_air_t<T, 1, false, C, TY, COL>), dim3(nb), dim3(BX, TY), 0, s, rd); \
-            else if (wind == 2) hipLaunchKernelGGL((k_rk_air_t<T, 2, false, C, TY, COL>), dim3(nb), dim3(BX, TY), 0, s, rd); \
-            else hipLaunchKernelGGL((k_rk_air_t<T, 0, false, C, TY, COL>), dim3(nb), dim3(BX, TY), 0, s, rd); \
-        }                                                                                             \
-    } while (0)
-    switch (v) {
-    case 1: LEE_RKT(4, true); break;
-    case 2: LEE_RKT(8, true); break;
-    case 3: LEE_RKT(8, false); break;
-    default: LEE_RKT(16, true); break;
-    }
-#undef LEE_RKT
-#undef LEE_RK_AXES
-}
-
-// Blocks of `kernel` (256 threads) the chip holds at once: the grid of a persistent form.
-template <typename K> unsigned resident_blocks(K kernel)
-{
-    int dev = 0, cus = 0, per = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, BX * BY, 0) != hipSuccess)
-        return 0;
-    return (unsigned)std::max(1, cus * per);
-}
-// One launch of a batched kernel in form `form` over `nblocks` tiles: a block per tile, or
-// (form 2) the resident grid walking them.
-template <typename K, typename... A>
-void launch_form(K kernel, int form, int nblocks, hipStream_t s, A... args)
-{
-    unsigned g = (unsigned)nblocks;
-    if (form == 2) {
-        static const unsigned cap = resident_blocks(kernel);  // one per instantiation (one device)
-        if (cap) g = std::min(g, cap);
-    }
-    hipLaunchKernelGGL(kernel, dim3(g), dim3(BX, BY), 0, s, args...);
-}
-template <typename T>
-void launch_rk_air_batch(const RKArgs<T> *args, const int *first, int n, int nblocks, int wind, bool terrain, int form,
-                         hipStream_t s)
+void launch_rk_air_batch(const RKArgs<T> *args, const int *first, int n, int nblocks, int wind, bool terrain, hipStream_t s)
 {
     constexpr bool C = std::is_same<T, float>::value;
     if (nblocks <= 0) return;
-#define LEE_RKF(WM, TER)                                                                                       \
-    do {                                                                                                     \
-        if (form == 2) launch_form(k_rk_air_batch<T, WM, TER, C, 2>, 2, nblocks, s, args, first, n, nblocks);    \
-        else if (form == 1) launch_form(k_rk_air_batch<T, WM, TER, C, 1>, 1, nblocks, s, args, first, n, nblocks); \
-        else launch_form(k_rk_air_batch<T, WM, TER, C, 0>, 0, nblocks, s, args, first, n, nblocks);             \
-    } while (0)
+#define LEE_RKF(WM, TER) \
+    hipLaunchKernelGGL((k_rk_air_batch<T, WM, TER, C>), dim3((unsigned)nblocks), dim3(BX, BY), 0, s, args, first, n)
     if (terrain) {
         if (wind == 1) LEE_RKF(1, true); else if (wind == 2) LEE_RKF(2, true); else LEE_RKF(0, true);
     } else {
@@ -1868,19 +1282,13 @@ void launch_rk_air_batch(const RKArgs<T> *args, const int *first, int n, int nbl
 #undef LEE_RKF
 }
 template <typename T>
-void launch_rk_pore_batch(const RKPoreArgs<T> *args, const int *first, int n, int nblocks, bool terrain, int form,
-                          hipStream_t s)
+void launch_rk_pore_batch(const RKPoreArgs<T> *args, const int *first, int n, int nblocks, bool terrain, hipStream_t s)
 {
     constexpr bool C = std::is_same<T, float>::value;
     if (nblocks <= 0) return;
-#define LEE_RPF(TER)                                                                                           \
-    do {                                                                                                     \
-        if (form == 2) launch_form(k_rk_pore_batch<T, TER, C, 2>, 2, nblocks, s, args, first, n, nblocks);       \
-        else if (form == 1) launch_form(k_rk_pore_batch<T, TER, C, 1>, 1, nblocks, s, args, first, n, nblocks);  \
-        else launch_form(k_rk_pore_batch<T, TER, C, 0>, 0, nblocks, s, args, first, n, nblocks);                \
-    } while (0)
-    if (terrain) LEE_RPF(true); else LEE_RPF(false);
-#undef LEE_RPF
+    const dim3 g((unsigned)nblocks), b(BX, BY);
+    if (terrain) hipLaunchKernelGGL((k_rk_pore_batch<T, true, C>), g, b, 0, s, args, first, n);
+    else hipLaunchKernelGGL((k_rk_pore_batch<T, false, C>), g, b, 0, s, args, first, n);
 }
 template <typename T> void launch_sample_batch(const T *const *p, const long long *idx, int n, double *out, hipStream_t s)
 {
@@ -1997,10 +1405,8 @@ void launch_copy_words(float *dst, const float *src, size_t n, hipStream_t s)
     template bool fused_fits<T>(int);                                                                        \
     template void launch_rk_air<T>(const RKArgs<T> &, const RKArgs<T> *, int, bool, hipStream_t);            \
     template void launch_rk_pore<T>(const RKPoreArgs<T> &, bool, hipStream_t);                               \
-    template void launch_rk_air_batch<T>(const RKArgs<T> *, const int *, int, int, int, bool, int, hipStream_t); \
-    template void launch_rk_air_v<T>(const RKArgs<T> &, const RKArgs<T> *, int, bool, int, hipStream_t);     \
-    template bool rk_stage_takes_xfaces<T>(const RKArgs<T> &, int);                                           \
-    template void launch_rk_pore_batch<T>(const RKPoreArgs<T> *, const int *, int, int, bool, int, hipStream_t); \
+    template void launch_rk_air_batch<T>(const RKArgs<T> *, const int *, int, int, int, bool, hipStream_t);  \
+    template void launch_rk_pore_batch<T>(const RKPoreArgs<T> *, const int *, int, int, bool, hipStream_t);   \
     template void launch_sample_batch<T>(const T *const *, const long long *, int, double *, hipStream_t);     \
     template void launch_air_fb<T>(const AirArgs<T> &, bool, hipStream_t, int);                              \
     template void launch_pore_p<T>(const PoreArgs<T> &, hipStream_t);                                        \

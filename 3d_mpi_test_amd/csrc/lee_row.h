@@ -41,8 +41,12 @@ template <typename T> __device__ __forceinline__ T lds_(gptr<const T> f, int i)
 // The rows of a block: tile row ty covers j0 + 4 ty .. + 3, anchored at the high end so that the
 // last tile row holds the interior rows ny - 4, ny - 3, ny - 2 the East face's pressure is
 // extrapolated from; rows below 1 of the first tile row idle (clamped to row 1, nothing stored).
-__host__ __device__ inline int row_tiles(int ny) { return (ny - 2 + RY - 1) / RY; }
-__host__ __device__ inline int row_first(int ny) { return ny - 1 - RY * row_tiles(ny); }
+inline int row_tiles(int ny) { return (ny - 2 + RY - 1) / RY; }
+inline int row_first(int ny) { return ny - 1 - RY * row_tiles(ny); }
+// x of a row's first lane: 0, or -1 where the last face would otherwise stand alone in its
+// wavefront (the RK4 registers are updated in place, so the point a face lane computes must
+// belong to its own wavefront).
+inline int row_left(int nx) { return nx % RX == 1 ? -1 : 0; }
 
 // Where a lane stands.  A lane on an x face (or past the row's end) computes the interior
 // neighbour's point (ip) and stores it as its own node (in): the value the face's copy gives.
@@ -56,7 +60,7 @@ __device__ __forceinline__ RowLane row_lane(int i, int nx, bool row_live)
     RowLane l;
     l.in = i;
     l.ip = i < 1 ? 1 : i > nx - 2 ? nx - 2 : i;
-    l.live = row_live && i < nx;
+    l.live = row_live && i >= 0 && i < nx;
     l.face = i == 0 || i == nx - 1;
     return l;
 }
