@@ -69,6 +69,7 @@ struct lee_ctx {
     // the frame change, never inside a capture)
     bool row_ok = false;
     RowPlan plan{};
+    ColPlan col{};  // several FB_p_v steps per launch (steps 0: not this deck)
     int *ring = nullptr;
     void *xprof[3] = {};
     void *row_args = nullptr, *row_lines = nullptr;       // lines: ny rows, then nz planes
@@ -1027,6 +1028,26 @@ template <typename T> void enqueue_fb_step(lee_ctx *c, double *rec_slot)
     c->steps += 1;
 }
 
+// n steps of a narrow column, several per launch; the buffer roles change once a launch.
+template <typename T> int col_steps(lee_ctx *c, int n)
+{
+    const Model &m = c->m;
+    const size_t nr = m.ri.size();
+    for (int t = 0; t < n;) {
+        const int s = std::min(n - t, c->col.steps);
+        int J1 = 0, y1on = 0;
+        for (int q = 0; q < s; ++q) gate_tick(c, J1, y1on);  // (no layer here opens with the gate)
+        if (int rc = row_args_sync<T>(c, J1, y1on)) return rc;
+        launch_col<T>(row_args_now<T>(c), c->col, s, c->rec_buf + (size_t)t * nr, c->stream);
+        if (m.ground) std::swap(c->gpsi, c->gpsi2);
+        c->cur ^= 1;
+        c->qcur ^= 1;
+        c->steps += s;
+        t += s;
+    }
+    return LEE_OK;
+}
+
 template <typename T> void enqueue_step(lee_ctx *c, double *rec_slot)
 {
     if (c->m.rk4) enqueue_rk4_step<T>(c, rec_slot);
@@ -1217,7 +1238,11 @@ template <typename T> int run_steps(lee_ctx *c, int nsteps, double *rec_out)
     while (done < nsteps) {
         int n = std::min(nsteps - done, kRecChunk);
         const long long before = c->steps;
-        if (m.opt.use_graph && !c->profile && c->src_ps.empty()) {
+        if (c->col.steps && !c->profile && c->src_ps.empty()) {
+            if (m.opt.use_graph && m.opt.health_every > 0) n = std::min(n, kGraphSteps);  // (checked between chunks)
+            int rc = col_steps<T>(c, n);
+            if (rc) return rc;
+        } else if (m.opt.use_graph && !c->profile && c->src_ps.empty()) {
             n = std::min(n, kGraphSteps);
             if (gate_constant(c, n)) {
                 int rc = graph_steps<T>(c, n);
@@ -1343,6 +1368,11 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
             HIPCHK(C, hipStreamSynchronize(C->stream));
         }
         C->plan.p.ring = C->plan.v.ring = C->ring;
+        // narrow columns without a flow, hills, the East impedance or a layer along x or y; a
+        // launch form that the caller names is the one that runs
+        if (!m.rk4 && o.fb_form == 0 && o.path != LEE_PATH_FUSED && !m.has_wind && !m.terrain && !m.east_tdbc &&
+            !m.slab[0].n && !m.slab[1].n && !m.slab[2].n && !m.slab[3].n && !(m.south_porous && !m.iface_copy))
+            C->col = col_plan(m.nx, m.ny, m.nz, rg.pnz);
         for (int q = 0; q < 3; ++q)
             if ((rc = dalloc(C, &C->xprof[q], (size_t)m.nx * es))) return rc;
         const bool f64 = C->prec == 64;

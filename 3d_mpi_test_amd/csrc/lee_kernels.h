@@ -188,6 +188,14 @@ template <typename T> void launch_row_p(const RowArgs<T> *ad, const RowPlan &pl,
 template <typename T> void launch_row_v(const RowArgs<T> *ad, const RowPlan &pl, bool wind, bool terrain, bool split,
                                         bool vec, hipStream_t s);
 
+// Several steps in one launch over a narrow column (lee_col.hip): planes a workgroup owns, halo
+// planes on either side, steps a launch can take (0: not this grid).
+constexpr int kColPlane = 64;  // nodes of a plane at most
+struct ColPlan { int own, halo, steps, blocks; };
+ColPlan col_plan(int nx, int ny, int nz, int pnz);
+// rec: the first step's receiver row, the others follow it.
+template <typename T> void launch_col(const RowArgs<T> *ad, const ColPlan &p, int nsteps, double *rec, hipStream_t s);
+
 // ---- RK4 (extension) ------------------------------------------------------------------
 // Registers: level n (xn), the accumulator acc = xn + sum_s b_s k_s, and the destination
 // (the next stage state xn + a_s k_s, or level n+1 = acc + b_4 k_4 after the last stage).
