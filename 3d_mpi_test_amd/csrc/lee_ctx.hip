@@ -649,10 +649,11 @@ RowGeo row_geo(const lee_ctx *c)
 }
 
 // Arguments of RK4 stage st in row form, from the context's buffer roles: the stages run
-// X -> A -> B -> C -> X, the auxiliaries from set qcur to the other one.
-template <typename T> void rk_row_args(lee_ctx *c, int st, int J1, int y1on, RkRowArgs<T> &r)
+// X -> A -> B -> C -> A (in place: -> X), the auxiliaries from set qcur to the other one.
+template <typename T> void rk_row_args(lee_ctx *c, int st, int J1, int y1on, bool in_place, RkRowArgs<T> &r)
 {
     const Model &m = c->m;
+    const int to = st < 3 ? st + 1 : in_place ? 0 : 1;
     std::memset(&r, 0, sizeof r);
     T *buf[2][4][4];  // air, porous: X A B C
     for (int d = 0; d < 2; ++d)
@@ -680,10 +681,10 @@ template <typename T> void rk_row_args(lee_ctx *c, int st, int J1, int y1on, RkR
     for (int f = 0; f < 4; ++f) {
         r.xn[f] = buf[0][0][f]; r.y1[f] = buf[0][1][f];
         r.pv[f] = buf[0][st ? st - 1 : 0][f];
-        r.dst[f] = buf[0][(st + 1) % 4][f];
+        r.dst[f] = buf[0][to][f];
         r.err[f] = (T *)c->rk_err[0][f];
         r.pxn[f] = buf[1][0][f];
-        r.pdst[f] = buf[1][(st + 1) % 4][f];
+        r.pdst[f] = buf[1][to][f];
         r.pacc[f] = (T *)c->rk_acc[1][f]; r.plo[f] = (T *)c->rk_lo[1][f]; r.perr[f] = (T *)c->rk_err[1][f];
     }
     r.acc = (T *)c->rk_acc[0][0];
@@ -701,24 +702,24 @@ template <typename T> void rk_row_args(lee_ctx *c, int st, int J1, int y1on, RkR
     r.rec_idx = c->rec_idx;
 }
 
-// The eight blocks (set qcur 0 and 1, four stages each) of the row kernels' arguments and the
+// The eight blocks (level cur 0 and 1, four stages each) of the row kernels' arguments and the
 // rows' records, for the gate state (J1, y1on), uploaded when the buffer roles, the gate or the
-// frame change: a step alternates the auxiliaries' sets and uploads nothing.
+// frame change: a step alternates the levels and the auxiliaries' sets and uploads nothing.
 template <typename T> int rk_rows_sync(lee_ctx *c, int J1, int y1on)
 {
-    const std::vector<uintptr_t> key = {(uintptr_t)J1, (uintptr_t)y1on, (uintptr_t)c->cur, c->frame_gen};
+    const int cur = c->cur, qcur = c->qcur, rel = cur ^ qcur;
+    const std::vector<uintptr_t> key = {(uintptr_t)J1, (uintptr_t)y1on, (uintptr_t)rel, c->frame_gen};
     if (key == c->row_key) return LEE_OK;
     if (c->capturing) return set_err(c, LEE_ERR_STATE, "step arguments changed inside a captured chunk");
     const std::vector<RowLine<T>> lines = row_lines_of<T>(c, J1, y1on);
     std::vector<unsigned char> host(8 * sizeof(RkRowArgs<T>));
-    const int q = c->qcur;
     for (int n = 0; n < 8; ++n) {
         RkRowArgs<T> r;
-        c->qcur = n / 4;
-        rk_row_args<T>(c, n % 4, J1, y1on, r);
+        c->cur = n / 4; c->qcur = c->cur ^ rel;
+        rk_row_args<T>(c, n % 4, J1, y1on, false, r);
         std::memcpy(host.data() + n * sizeof r, &r, sizeof r);
     }
-    c->qcur = q;
+    c->cur = cur; c->qcur = qcur;
     HIPCHK(c, hipMemcpyAsync(c->row_args, host.data(), host.size(), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->row_lines, lines.data(), lines.size() * sizeof(RowLine<T>), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -838,7 +839,7 @@ template <typename T> int rk_args_peek(lee_ctx *c)
 // Stage st in row form, launch shape v.
 template <typename T> void rk_row_stage(lee_ctx *c, int st, int v, double *rec)
 {
-    launch_rk_row<T>((const RkRowArgs<T> *)c->row_args + 4 * c->qcur + st, c->plan, st, rk_wind_mode(c->m), c->m.terrain,
+    launch_rk_row<T>((const RkRowArgs<T> *)c->row_args + 4 * c->cur + st, c->plan, st, rk_wind_mode(c->m), c->m.terrain,
                      c->plan.has_in && v >= kRkSplit, rec, c->stream);
 }
 
@@ -856,6 +857,7 @@ template <typename T> void enqueue_rk4_step(lee_ctx *c, double *rec_slot)
             rk_row_stage<T>(c, st, c->rk_variant, rec_slot);
             prof_mark(c, KS_RK_AIR, false);
         }
+        c->cur ^= 1;
         c->qcur ^= 1;
     } else {
         const int nr = (int)m.ri.size();
@@ -1092,7 +1094,7 @@ template <typename T> int graph_steps(lee_ctx *c, int n)
                     if (m.east_tdbc) std::swap(c->psi, c->psi2);
                     if (m.ground) std::swap(c->gpsi, c->gpsi2);
                 } else if (rk_rows(c)) {
-                    c->qcur ^= 1;
+                    c->cur ^= 1; c->qcur ^= 1;
                 }
             }
             if (gate) c->counter += n;
@@ -1124,10 +1126,10 @@ template <typename T> int graph_steps(lee_ctx *c, int n)
     return LEE_OK;
 }
 
-// Autotuner of the RK4 stage: times the whole domain in one launch against the interior box in
-// a launch of its own on stages 0-2 of the coming step (they read level n and the registers
-// stage 0 rewrites, so repeating them changes nothing the step itself does not overwrite) and
-// keeps the faster; without an interior box there is one shape.
+// Autotuner of the RK4 stage: times the whole domain in one launch a stage against the interior's
+// two stages a launch on stages 0 and 1 of the coming step (they read level n and write the
+// registers that the step itself rewrites) and keeps the faster; without an interior there is one
+// shape.
 template <typename T> int tune_rk(lee_ctx *c)
 {
     const Model &m = c->m;
@@ -1144,7 +1146,7 @@ template <typename T> int tune_rk(lee_ctx *c)
     for (int pass = 0; pass < 2; ++pass)
         for (int q = 0; q < 2; ++q) {
             auto stages = [&]() {
-                for (int st = 0; st < 3; ++st) rk_row_stage<T>(c, st, cand[q], c->rec_buf);
+                for (int st = 0; st < 2; ++st) rk_row_stage<T>(c, st, cand[q], c->rec_buf);
             };
             stages();  // warm-up
             HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1357,7 +1359,7 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
         if ((rc = dalloc(C, &C->pmx, m.pnx * es)) || (rc = dalloc(C, &C->pmy, m.pny * es)) || (rc = dalloc(C, &C->pmz, m.pnz * es)))
             return rc;
     if (C->row_ok) {
-        RowGeom rg{m.nx, m.ny, m.nz, m.south_porous ? m.pnz : 0, m.iface_copy, m.ground, (int)m.ri.size(), {}, {},
+        RowGeom rg{m.nx, m.ny, m.nz, m.south_porous ? m.pnz : 0, m.iface_copy, m.ground, (int)m.ri.size(), m.rk4, es, {}, {},
                    {m.I1, m.I2, m.J3, m.J2, m.K1, m.K2}};
         for (int s = 0; s < 6; ++s) { rg.qn[s] = m.slab[s].n; rg.qlo[s] = m.slab[s].lo; }
         std::vector<int> ring;
@@ -2257,7 +2259,7 @@ template <typename T> int ens_tables(lee_ensemble *e, const std::vector<int> &J1
             for (int s = 0; s < 8; ++s) {
                 RkRowArgs<T> &r = t[(size_t)s * n + d];
                 c->qcur = q ^ (s / 4);
-                rk_row_args<T>(c, s % 4, J1[d], y1on[d], r);
+                rk_row_args<T>(c, s % 4, J1[d], y1on[d], true, r);
                 r.first = blocks;
             }
             c->qcur = q;

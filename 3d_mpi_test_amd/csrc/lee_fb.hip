@@ -138,7 +138,7 @@ __device__ __forceinline__ T fb_p_point(const RowArgs<T> &A, const RowGeo &G, co
         qz = ldr<T>(Q.o[3], sz.row, on);
     }
     T ddx, ddy, dwz;
-    T r = row_dp<T, WM, TERRAIN, false>(a, at, n, ddx, ddy, dwz);
+    T r = row_dp<T, WM, TERRAIN, false>(a, at, RowState<T>{g, at}, n, ddx, ddy, dwz);
     r = row_dp_layers<T, TERRAIN, X, Y, Z>(a, n, lx, ly, lz, x, y, z, n.pc, ddx, ddy, dwz, r);
     return n.pc + r;
 }
@@ -336,7 +336,7 @@ __device__ __forceinline__ void fb_v_point(const RowArgs<T> &A, const RowGeo &G,
         for (int c = 0; c < 3; ++c) qz[c] = ldr<T>(Q.o[c], sz.row, on);
     }
     T gpx, gpy, gpz, du, dv, dw;
-    row_duvw<T, WM, TERRAIN, false>(a, at, n, gpx, gpy, gpz, du, dv, dw);
+    row_duvw<T, WM, TERRAIN, false>(a, at, RowState<T>{g, at}, n, gpx, gpy, gpz, du, dv, dw);
     row_duvw_layers<T, TERRAIN, X, Y, Z>(a, n, lx, ly, lz, x, y, z, n.uc, n.vc, n.wc, gpx, gpy, gpz, du, dv, dw);
     out[0] = n.uc + du; out[1] = n.vc + dv; out[2] = n.wc + dw;
 }
@@ -506,11 +506,11 @@ __global__ __launch_bounds__(RX * RY) void k_row_in(const RowArgs<T> *__restrict
     row_metric<T, TERRAIN>(g, g.nx, i, j, lds_<T>(g.my, j), lds_<T>(g.mz, k), TERRAIN ? lds_<T>(g.ttk, k) : T(0), n);
     if constexpr (PRESSURE) {
         T ddx, ddy, dwz;
-        const T r = row_dp<T, WM, TERRAIN, false>(a, at, n, ddx, ddy, dwz);
+        const T r = row_dp<T, WM, TERRAIN, false>(a, at, RowState<T>{g, at}, n, ddx, ddy, dwz);
         str<T>(g.pnn, at.row, at.o, n.pc + r);
     } else {
         T gpx, gpy, gpz, du, dv, dw;
-        row_duvw<T, WM, TERRAIN, false>(a, at, n, gpx, gpy, gpz, du, dv, dw);
+        row_duvw<T, WM, TERRAIN, false>(a, at, RowState<T>{g, at}, n, gpx, gpy, gpz, du, dv, dw);
         str<T>(g.unn, at.row, at.o, n.uc + du); str<T>(g.vnn, at.row, at.o, n.vc + dv); str<T>(g.wnn, at.row, at.o, n.wc + dw);
     }
 }
@@ -631,8 +631,8 @@ template <typename T> void launch_row_v(const RowArgs<T> *ad, const RowPlan &pl,
 #undef LEE_RV
 }
 
-// Launch plan of a domain: tile counts and, over a grid with an interior (whole tiles outside
-// every layer and not next to a face), that box and the ring of tiles around it.
+// Launch plan of a domain: tile counts and, over a grid with an interior (outside every layer and
+// not next to a face; FB: whole tiles of it), that box and the ring of tiles around it.
 void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
 {
     const int i0 = row_left(m.nx), j0 = row_first(m.ny), ntx = (m.nx - i0 + RX - 1) / RX, nty = row_tiles(m.ny);
@@ -655,11 +655,39 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
     pl.j0 = j0;
     pl.has_in = tx1 > tx0 && ty1 > ty0 && zb > za;
     if (pl.has_in) pl.in = RowBox{tx0, tx1 - tx0, ty0, ty1 - ty0, za, zb - za, i0, j0};
+    if (m.rk4) {
+        // any points, except the rows of the last tile row (it extrapolates the East pressure);
+        // two tiles wide at least, so that no tile meets both ends
+        RowPair &b = pl.pair;
+        b.xa = xa; b.xb = xb; b.ya = ya; b.yb = std::min(yb, j0 + RY * (nty - 1)); b.za = za; b.zb = zb;
+        const int wx = b.xb - b.xa, wy = b.yb - b.ya, wz = b.zb - b.za;
+        pl.has_in = wx >= 2 * RX && wy >= 16 && wz >= 8;
+        if (pl.has_in) {
+            auto cut = [](int n, int most, int &parts, int &width) {
+                parts = (n + most - 1) / most;
+                width = (n + parts - 1) / parts;
+                parts = (n + width - 1) / width;
+            };
+            cut(wx, RX - 2, b.nbx, b.wx);
+            cut(wy, pair_rows(m.esz) - 2, b.nby, b.wy);
+            // planes per block: one block a CU at a time, each with two planes more than its own
+            const int cols = b.nbx * b.nby;
+            long long best = -1;
+            for (int nz = 1; nz <= 16 && nz * 4 <= wz; ++nz) {
+                const int w = (wz + nz - 1) / nz;
+                const long long cost = (long long)((cols * nz + 255) / 256) * (w + 2);
+                if (best < 0 || cost < best) { best = cost; b.wz = w; b.nbz = (wz + w - 1) / w; }
+            }
+        }
+    }
     ring.clear();
     if (pl.has_in)
         for (int ty = 0; ty < nty; ++ty)
             for (int tx = 0; tx < ntx; ++tx)
-                if (tx < tx0 || tx >= tx1 || ty < ty0 || ty >= ty1) ring.push_back(tx | (ty << 16));
+                if (m.rk4 ? i0 + RX * tx < pl.pair.xa || i0 + RX * (tx + 1) > pl.pair.xb || j0 + RY * ty < pl.pair.ya ||
+                                j0 + RY * (ty + 1) > pl.pair.yb
+                          : tx < tx0 || tx >= tx1 || ty < ty0 || ty >= ty1)
+                    ring.push_back(tx | (ty << 16));
     const int full = ntx * nty, nrp = (m.nrec + full * RX * RY - 1) / (full * RX * RY);
     for (int ph = 0; ph < 2; ++ph) {
         RowLaunch &l = ph ? pl.v : pl.p;
@@ -670,6 +698,7 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
         l.zground = m.ground || (m.pnz > 0 && !m.coupled) ? 1 : 0;
         l.z = l.zair + l.zpore + l.zground + (ph ? 0 : nrp);
         l.ka = za; l.kb = zb;
+        l.xa = pl.pair.xa; l.xb = pl.pair.xb; l.ya = pl.pair.ya; l.yb = pl.pair.yb;
         l.nring = (int)ring.size() ? (int)ring.size() : 1;
         if (pl.has_in) {
             const int per[6] = {full * (za - 1), full * (m.nz - 1 - zb), (int)ring.size() * (zb - za), full * l.zpore,

@@ -167,17 +167,26 @@ struct RowBox { int tx, nbx, ty, nby, k, nk, i0, j0; };
 struct RowLaunch {
     int ntx, nty, z, zair, zpore, zground;
     int ka, kb, nring;
+    int xa, xb, ya, yb;  // RK4: the interior's points, which the ring's tiles leave out
     int first[7];
     const int *ring;
 };
+// The interior of an RK4 domain, points [xa, xb) x [ya, yb) x [za, zb) outside every layer and
+// away from every face, in nbx x nby x nbz blocks of wx x wy columns and wz planes.
+// Rows of such a block with the two around its own: 16 waves leave 128 registers a lane, FP64 needs
+// up to 199 (12 rows and 168 registers spilled 92 to 168 B a lane and took twice as long).
+constexpr int pair_rows(size_t esz) { return esz == 8 ? 8 : 16; }
+struct RowPair { int xa, xb, ya, yb, za, zb, nbx, wx, nby, wy, nbz, wz; };
 struct RowPlan {
     bool has_in;
     int i0, j0;
-    RowBox in;
+    RowBox in;     // FB
+    RowPair pair;  // RK4
     RowLaunch p, v;
 };
 struct RowGeom {
-    int nx, ny, nz, pnz, coupled, ground, nrec;
+    int nx, ny, nz, pnz, coupled, ground, nrec, rk4;
+    size_t esz;
     int qn[6], qlo[6], w[6];  // slabs and layer widths, x1 x2 y1 y2 z1 z2
 };
 void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m);
@@ -228,7 +237,9 @@ template <typename T> struct RKBndArgs {
 // is the field itself, so that of stage s at a node is Q_n + a_{s-1} dt y_{s-1} with the previous
 // stage's state there (pv), and Q_{n+1} follows in the last stage from Q_n and the four states
 // at the node -- the sums the stored form rounds the same way.  The three stage states keep a
-// buffer each (A, B, C) and the auxiliaries alternate between two sets.
+// buffer each (A, B, C) and the auxiliaries alternate between two sets; level n+1 takes A's place
+// (a block of the interior still reads level n around it when a neighbour stores), or level n's in
+// an ensemble, which has no interior kernel.
 template <typename T> struct RkRowArgs {
     RowGeo geo;
     int first, ntile, zair;  // ensemble: the member's first block, tiles per plane, air planes
@@ -245,8 +256,9 @@ template <typename T> struct RkRowArgs {
     gptr<T> pacc[4], plo[4], perr[4], pdst[4];
     gptr<const long long> rec_idx;
 };
-// One stage st of a domain: split = the interior box in a launch of its own and the rest in
-// another, else everything in one; stage 0 samples the receivers into rec.
+// One stage st of a domain, everything in one launch; or split: the rest of the domain, and with
+// stages 0 and 2 the interior's stages st and st + 1 in a launch after it (ad + 1: the arguments of
+// stage st + 1).  Stage 0 samples the receivers into rec.
 template <typename T> void launch_rk_row(const RkRowArgs<T> *ad, const RowPlan &pl, int st, int wind, bool terrain, bool split,
                                          double *rec, hipStream_t s);
 // The same for n domains (their arguments one after the other), nblocks blocks in all.

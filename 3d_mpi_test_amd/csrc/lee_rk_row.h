@@ -169,10 +169,11 @@ __device__ __forceinline__ void rk_row_point(const RkRowArgs<T> &A, const RowGeo
         if constexpr (TERRAIN) vz.pk = s(ldr<T>(Q.o[3], sz.row - sz.dk, op), e.pk);
     }
     T ddx, ddy, dwz, gpx, gpy, gpz;
-    T r = row_dp<T, WM, TERRAIN, true>(a, at, n, ddx, ddy, dwz);
+    const RowState<T> st{g, at};
+    T r = row_dp<T, WM, TERRAIN, true>(a, at, st, n, ddx, ddy, dwz);
     kf[3] = row_dp_layers<T, TERRAIN, X, Y, Z>(a, n, lx, ly, lz, px, py, pz, n.pc, ddx, ddy, dwz, r);
     T du, dv, dw;
-    row_duvw<T, WM, TERRAIN, true>(a, at, n, gpx, gpy, gpz, du, dv, dw);
+    row_duvw<T, WM, TERRAIN, true>(a, at, st, n, gpx, gpy, gpz, du, dv, dw);
     row_duvw_layers<T, TERRAIN, X, Y, Z>(a, n, lx, ly, lz, vx, vy, vz, n.uc, n.vc, n.wc, gpx, gpy, gpz, du, dv, dw);
     kf[0] = du; kf[1] = dv; kf[2] = dw;
     xc[0] = n.uc; xc[1] = n.vc; xc[2] = n.wc; xc[3] = n.pc;
@@ -300,7 +301,7 @@ __device__ __forceinline__ void rk_row_pore(const RkRowArgs<T> &A, const RowGeo 
 // MODE 0: the whole domain, 1: around the interior box, 2: an ensemble.
 template <typename T, int WM, bool TERRAIN, int ST, int MODE>
 __device__ __forceinline__ void rk_row_block(const RkRowArgs<T> &A, int st, int kind, int k, int tx, int ty, long long rec,
-                                             double *__restrict__ rec_out, T (&rows)[RY][RX])
+                                             double *__restrict__ rec_out, T (&rows)[RY][RX], const int (&box)[4])
 {
     constexpr bool COMP = std::is_same<T, float>::value;
     const RowGeo G = A.geo;
@@ -321,8 +322,15 @@ __device__ __forceinline__ void rk_row_block(const RkRowArgs<T> &A, int st, int 
     const bool row_live = jr >= 1;
     const int j = row_live ? jr : 1;
     const int i0 = G.i0 + tx * RX;
-    const RowLane l = row_lane(i0 + lane, nx, row_live);
+    RowLane l = row_lane(i0 + lane, nx, row_live);
     const bool last = ty == G.nty - 1;
+    if (MODE == 1 && j >= box[2] && j < box[3]) {
+        // the interior's points [box 0, box 1) of this row belong to its own kernel: their lanes
+        // repeat the nearest other point (a tile never meets both ends of the interior)
+        if (i0 >= box[0] && i0 + RX <= box[1]) return;  // (never in the last tile row)
+        if (l.in >= box[0] && l.in < box[1]) l.live = false;
+        l.ip = i0 < box[0] ? min(l.ip, box[0] - 1) : max(l.ip, box[1]);
+    }
     T d[4];
     if (kind == RK_AIR) {
         const RowLine<T> yl = row_line(A.yl, j), zl = row_line(A.zl, k);
@@ -408,6 +416,7 @@ __global__ __launch_bounds__(RX * RY) void k_rk_row(const RkRowArgs<T> *__restri
 {
     __shared__ T rows[RY][RX];
     int kind, k, tx, ty;
+    int box[4] = {0, 0, 0, 0};
     long long rec = 0;
     if constexpr (!RING) {
         const int z = blockIdx.z;
@@ -429,12 +438,13 @@ __global__ __launch_bounds__(RX * RY) void k_rk_row(const RkRowArgs<T> *__restri
         if (s == 2) {
             const int e = ((const __attribute__((address_space(4))) int *)L.ring)[idx];
             tx = e & 0xffff; ty = e >> 16;
+            box[0] = L.xa; box[1] = L.xb; box[2] = L.ya; box[3] = L.yb;
         } else {
             ty = idx / L.ntx;
             tx = idx - ty * L.ntx;
         }
     }
-    rk_row_block<T, WM, TERRAIN, ST, RING ? 1 : 0>(*ap, st, kind, k, tx, ty, rec, rec_out, rows);
+    rk_row_block<T, WM, TERRAIN, ST, RING ? 1 : 0>(*ap, st, kind, k, tx, ty, rec, rec_out, rows, box);
 }
 
 // Ensemble: the block's member by binary search over the block prefix, then its plane and tile.
@@ -450,45 +460,209 @@ __global__ __launch_bounds__(RX * RY) void k_rk_row_batch(const RkRowArgs<T> *__
     }
     const RkRowArgs<T> &A = ap[lo];
     const int t = b - A.first, z = t / A.ntile, idx = t - z * A.ntile, ntx = A.ntile / A.geo.nty, ty = idx / ntx;
-    const int kind = z < A.zair ? RK_AIR : RK_PORE;
-    rk_row_block<T, WM, TERRAIN, ST, 2>(A, st, kind, kind == RK_AIR ? z + 1 : z - A.zair + 1, idx - ty * ntx, ty, 0, nullptr, rows);
+    const int kind = z < A.zair ? RK_AIR : RK_PORE, box[4] = {0, 0, 0, 0};
+    rk_row_block<T, WM, TERRAIN, ST, 2>(A, st, kind, kind == RK_AIR ? z + 1 : z - A.zair + 1, idx - ty * ntx, ty, 0, nullptr, rows, box);
 }
 
-// The interior outside every layer and away from every face, a point per lane.
-template <typename T, int WM, bool TERRAIN, int ST>
-__global__ __launch_bounds__(RX * RY) void k_rk_in(const RkRowArgs<T> *__restrict__ ap, RowBox bx)
+// ---- the interior outside every layer and away from every face: two stages per launch ------
+// A stage of the interior reads and writes 13 to 25 words a point at 4.2 of the 4.7 TB/s a copy
+// reaches, so only fewer passes make it faster.  Here a block marches up its columns and keeps
+// stage s's state y of four planes in LDS: plane k + 1 of y from the state in memory, then stage
+// s + 1 of plane k from y.  Two stages move 13 + 25 words (FP32; 13 + 17 in FP64) instead of 34 +
+// 46 (34 + 34).  Per step, 512 x 256 x 128 with wind over a hill: the interior 702 us by single
+// stages (8.8 M points, whole tiles) and 578 us so (10.7 M points, any), the step 1779 -> 1570 us in
+// FP32 and 3476 -> 3046 us in FP64; 768 x 384 x 192 FP32 4860 -> 4217 us.  At 2.7 to 3.5 TB/s it is
+// bound by the latency of its loads and the barrier between the stages.  The y around a block's columns is computed by the neighbours as well; next to the
+// interior it is read from the buffer stage s left it in, and the interior's outermost points
+// store theirs there for the ring's stage s + 1.
+//
+// The lane's own column (state, mean flow along y, and in the second pair level n, accumulator
+// and error) is loaded a plane ahead into registers, so that loads from memory are in flight all
+// through a plane.  Loads and stores are waited for in order, so the neighbours' values of the
+// next plane, which the caches hold by then, are requested before stage s + 1 stores.  Without the
+// column loaded ahead the pairs took 741 us (FP32) and 1182 us (FP64: 1002 us so), with the
+// neighbours requested after the column's next plane 655 us, after the stores 580 us; FP32 blocks
+// of 8 rows 635 us; nontemporal stores the same as plain ones.
+template <typename T> constexpr int kPR = pair_rows(sizeof(T));  // rows of a block with the two around its own
+
+// Readers around the lane's point: the state with the lane's column and its four neighbours (x + 1,
+// x - 1, y + 1, y - 1) in registers, ...
+template <typename T> struct PairColumn {
+    const T (&r)[3][4], (&nb)[4][4];
+    template <int C> __device__ __forceinline__ T get(int di, int dj, int dk) const
+    {
+        constexpr int f = C > 3 ? 3 : C;
+        return di ? nb[di > 0 ? 0 : 1][f] : dj ? nb[dj > 0 ? 2 : 3][f] : r[dk + 1][f];
+    }
+};
+// ... the mean flow (V alone: in registers too), ...
+template <typename T, int WM> struct PairWind {
+    const RowAt<T> &at;
+    const T *r, *nb;
+    __device__ __forceinline__ T operator()(gptr<const T> f, int di, int dj, int dk) const
+    {
+        if constexpr (WM == 2) return di ? nb[di > 0 ? 0 : 1] : dj ? nb[dj > 0 ? 2 : 3] : r[dk + 1];
+        else return at(f, di, dj, dk);
+    }
+};
+// ... and y from LDS planes k - 1, k, k + 1.
+template <typename T> struct PairState {
+    const T *y[3];  // the lane's value of field 0
+    template <int C> __device__ __forceinline__ T get(int di, int dj, int dk) const
+    {
+        return y[dk + 1][(C > 3 ? 3 : C) * kPR<T> * RX + dj * RX + di];
+    }
+};
+template <typename T> struct PairPoint {
+    T xn[4], acc[4];  // level n, accumulator after stage s
+    T V[4];           // mean flow at the four neighbours
+};
+
+template <typename T, int WM, bool TERRAIN, bool LAST>
+__global__ __launch_bounds__(RX * kPR<T>) void k_rk_pair(const RkRowArgs<T> *__restrict__ ap, RowPair bx)
 {
     constexpr bool COMP = std::is_same<T, float>::value;
-    const RkRowArgs<T> &A = *ap;
+    constexpr int SA = LAST ? 1 : 0, SB = LAST ? 3 : 1;
+    __shared__ T Y[4][4][kPR<T>][RX];
+    const RkRowArgs<T> &A = ap[0], &B = ap[1];
     const AirArgs<T> &a = A.a;
     const Grid<T> &g = a.g;
-    const int tj = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-    const int i = bx.i0 + (bx.tx + (int)blockIdx.x) * RX + (int)threadIdx.x, k = bx.k + (int)blockIdx.z;
-    const int j = bx.j0 + RY * (bx.ty + (int)blockIdx.y) + tj;
+    const int lane = threadIdx.x, row = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    // blocks that follow one another in a plane share an XCD (and the columns around them its L2)
+    const int blocks = gridDim.x, b = blockIdx.x, xcd = b & 7, per = blocks >> 3, more = blocks & 7;
+    const int t = xcd * per + min(xcd, more) + (b >> 3);
+    const int plane = bx.nbx * bx.nby, tz = t / plane, tp = t - tz * plane, ty = tp / bx.nbx, tx = tp - ty * bx.nbx;
+    const int x0 = bx.xa + tx * bx.wx, x1 = min(x0 + bx.wx, bx.xb), y0 = bx.ya + ty * bx.wy, y1 = min(y0 + bx.wy, bx.yb);
+    const int k0 = bx.za + tz * bx.wz, k1 = min(k0 + bx.wz, bx.zb);
+    // lanes and rows past the block's last repeat the one after it
+    const int i = min(x0 - 1 + lane, x1), j = min(y0 - 1 + row, y1);
+    const bool own = lane >= 1 && x0 - 1 + lane < x1 && row >= 1 && y0 - 1 + row < y1;
+    const bool in = i >= bx.xa && i < bx.xb && j >= bx.ya && j < bx.yb;
+    const bool rim = i == bx.xa || i == bx.xb - 1 || j == bx.ya || j == bx.yb - 1;
     const size_t snx = (size_t)g.nx * sizeof(T), sxy = snx * g.ny;
-    const RowAt<T> at{snx * j + sxy * k, snx, sxy, (unsigned)i * (unsigned)sizeof(T)};
-    const size_t e = (size_t)i + (size_t)g.nx * ((size_t)j + (size_t)g.ny * k);
-    Nb<T> n;
-    row_metric<T, TERRAIN>(g, g.nx, i, j, lds_<T>(g.my, j), lds_<T>(g.mz, k), TERRAIN ? lds_<T>(g.ttk, k) : T(0), n);
-    T xn[4], ac[4] = {T(0), T(0), T(0), T(0)}, er[4];
+    const unsigned o = (unsigned)i * (unsigned)sizeof(T);
+    auto at_plane = [&](int k) { return RowAt<T>{snx * j + sxy * k, snx, sxy, o}; };
+    auto elem = [&](int k) { return (size_t)i + (size_t)g.nx * ((size_t)j + (size_t)g.ny * k); };
+    // planes k - 1, k, k + 1 of the state, k - 2 .. k + 1 of V; level n, accumulator of plane k,
+    // error of plane k - 1
+    T r[3][4], v[4] = {}, xn[4] = {}, ac[4] = {}, er[4] = {};
+    T r2[4], v2 = T(0), xn2[4] = {}, ac2[4] = {}, er2[4] = {};  // the next plane's
+    const RowColumn<T> col = row_column<T, TERRAIN>(g, g.nx, i, j);
+    const T my = lds_<T>(g.my, j);
+    auto column = [&](int k, T(&q)[4]) {
+        const RowAt<T> at = at_plane(k);
+        q[0] = at(g.un, 0, 0, 0); q[1] = at(g.vn, 0, 0, 0); q[2] = at(g.wn, 0, 0, 0); q[3] = at(g.pn, 0, 0, 0);
+    };
+    auto level = [&](int k, T(&q)[4]) {
+        const RowAt<T> at = at_plane(k);
 #pragma unroll
-    for (int f = 0; f < 4; ++f) {
-        xn[f] = ST == 0 || (ST == 3 && !COMP) ? T(0) : at(A.xn[f], 0, 0, 0);
-        er[f] = ST == 3 && COMP ? at(A.err[f], 0, 0, 0) : T(0);
+        for (int f = 0; f < 4; ++f) q[f] = at(A.xn[f], 0, 0, 0);
+    };
+    column(k0 - 2, r[1]);
+    column(k0 - 1, r[2]);
+    column(k0, r2);
+    if constexpr (WM == 2) {
+        v[2] = at_plane(k0 - 2)(a.V, 0, 0, 0);
+        v[3] = at_plane(k0 - 1)(a.V, 0, 0, 0);
+        v2 = at_plane(k0)(a.V, 0, 0, 0);
     }
-    if constexpr (ST != 0) acc4_load(A.acc, e, ac);
-    T kf[4], ddx, ddy, dwz, gpx, gpy, gpz;
-    kf[3] = row_dp<T, WM, TERRAIN, true>(a, at, n, ddx, ddy, dwz);
-    row_duvw<T, WM, TERRAIN, true>(a, at, n, gpx, gpy, gpz, kf[0], kf[1], kf[2]);
-    const T xc[4] = {n.uc, n.vc, n.wc, n.pc};
-    T d[4], ao[4], eo[4];
+    if constexpr (LAST) level(k0 - 1, xn2);
+    // the neighbours' values of plane k, or the plane's own y outside the interior
+    T nb[4][4] = {}, vn[4] = {};
+    auto inside = [&](int k) { return in && k >= bx.za && k < bx.zb; };
+    auto neighbours = [&](int k) {
+        const RowAt<T> at = at_plane(k);
+        if (inside(k)) {
+            constexpr int D[4][2] = {{1, 0}, {-1, 0}, {0, 1}, {0, -1}};
+            const RowState<T> st{g, at};
 #pragma unroll
-    for (int f = 0; f < 4; ++f) d[f] = rk_point<T, ST>(ST == 0 ? xc[f] : xn[f], kf[f], ac[f], er[f], A.ca, ao[f], eo[f]);
-    rk_store4(A.dst, at.row, at.o, d);
-    if constexpr (ST != 3) acc4_store(A.acc, e, ao);
-    if constexpr (ST == 3 && COMP) {
+            for (int q = 0; q < 4; ++q) {
+                nb[q][0] = st.template get<0>(D[q][0], D[q][1], 0);
+                nb[q][1] = st.template get<1>(D[q][0], D[q][1], 0);
+                nb[q][2] = st.template get<2>(D[q][0], D[q][1], 0);
+                nb[q][3] = st.template get<3>(D[q][0], D[q][1], 0);
+                if constexpr (WM == 2) vn[q] = at(a.V, D[q][0], D[q][1], 0);
+            }
+        } else {
+            nb[0][0] = at(A.dst[0], 0, 0, 0); nb[1][3] = at(A.dst[1], 0, 0, 0);
+            nb[2][1] = at(A.dst[2], 0, 0, 0); nb[3][3] = at(A.dst[3], 0, 0, 0);
+        }
+    };
+    neighbours(k0 - 1);
+    PairPoint<T> c{}, n{};
+#pragma unroll 1
+    for (int k = k0 - 1; k <= k1; ++k) {
+        const RowAt<T> at = at_plane(k);
+        T y[4];
+        // what the previous plane asked for, then the next plane's
 #pragma unroll
-        for (int f = 0; f < 4; ++f) str<T>(A.err[f], at.row, at.o, eo[f]);
+        for (int f = 0; f < 4; ++f) {
+            r[0][f] = r[1][f]; r[1][f] = r[2][f]; r[2][f] = r2[f];
+            xn[f] = xn2[f]; ac[f] = ac2[f]; er[f] = er2[f];
+        }
+        v[0] = v[1]; v[1] = v[2]; v[2] = v[3]; v[3] = v2;
+        __builtin_amdgcn_sched_barrier(0);
+        const int k2 = min(k + 2, k1 + 1), kn = min(k + 1, k1);
+        column(k2, r2);
+        if constexpr (WM == 2) v2 = at_plane(k2)(a.V, 0, 0, 0);
+        if constexpr (LAST) {
+            level(kn, xn2);
+            if (own && kn < k1) acc4_load(A.acc, elem(kn), ac2);
+            if constexpr (COMP) {
+                const RowAt<T> ak = at_plane(min(k, k1 - 1));
+                if (own && k >= k0)
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) er2[f] = ak(B.err[f], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (inside(k)) {
+            Nb<T> q;
+            row_metric<T, TERRAIN>(col, my, lds_<T>(g.mz, k), TERRAIN ? lds_<T>(g.ttk, k) : T(0), q);
+            T kf[4], ddx, ddy, dwz, gpx, gpy, gpz, e;
+            const PairColumn<T> st{r, nb};
+            const PairWind<T, WM> wind{at, v + 1, vn};
+            kf[3] = row_dp<T, WM, TERRAIN, true>(a, wind, st, q, ddx, ddy, dwz);
+            row_duvw<T, WM, TERRAIN, true>(a, wind, st, q, gpx, gpy, gpz, kf[0], kf[1], kf[2]);
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                n.xn[f] = LAST ? xn[f] : r[1][f];
+                y[f] = rk_point<T, SA>(n.xn[f], kf[f], ac[f], T(0), A.ca, n.acc[f], e);
+            }
+            if (own && k >= k0 && k < k1 && (rim || k == bx.za || k == bx.zb - 1)) rk_store4(A.dst, at.row, o, y);
+#pragma unroll
+            for (int f = 0; f < 4; ++f) n.V[f] = vn[f];
+        } else {
+            y[0] = nb[0][0]; y[1] = nb[1][3]; y[2] = nb[2][1]; y[3] = nb[3][3];
+        }
+#pragma unroll
+        for (int f = 0; f < 4; ++f) Y[k & 3][f][row][lane] = y[f];
+        // the plane written next was last read before the previous barrier
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        neighbours(min(k + 1, k1));
+        __builtin_amdgcn_sched_barrier(0);
+        if (own && k > k0) {
+            const int kc = k - 1;
+            const RowAt<T> ac1 = at_plane(kc);
+            Nb<T> q;
+            row_metric<T, TERRAIN>(col, my, lds_<T>(g.mz, kc), TERRAIN ? lds_<T>(g.ttk, kc) : T(0), q);
+            const PairState<T> st{{&Y[(kc - 1) & 3][0][row][lane], &Y[kc & 3][0][row][lane], &Y[(kc + 1) & 3][0][row][lane]}};
+            const PairWind<T, WM> wind{ac1, v, c.V};
+            T kf[4], ddx, ddy, dwz, gpx, gpy, gpz, d[4], ao[4], eo[4];
+            kf[3] = row_dp<T, WM, TERRAIN, true>(a, wind, st, q, ddx, ddy, dwz);
+            row_duvw<T, WM, TERRAIN, true>(a, wind, st, q, gpx, gpy, gpz, kf[0], kf[1], kf[2]);
+#pragma unroll
+            for (int f = 0; f < 4; ++f) d[f] = rk_point<T, SB>(c.xn[f], kf[f], c.acc[f], er[f], B.ca, ao[f], eo[f]);
+            rk_store4(B.dst, ac1.row, o, d);
+            if constexpr (!LAST) acc4_store(B.acc, elem(kc), ao);
+            if constexpr (LAST && COMP) {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) str<T>(B.err[f], ac1.row, o, eo[f]);
+            }
+        }
+        c = n;
     }
 }
 
@@ -497,14 +671,17 @@ __global__ __launch_bounds__(RX * RY) void k_rk_in(const RkRowArgs<T> *__restric
 template <typename T>
 void launch_rk_row(const RkRowArgs<T> *ad, const RowPlan &pl, int st, int wind, bool terrain, bool split, double *rec, hipStream_t s)
 {
-    const dim3 blk(RX, RY), box((unsigned)pl.in.nbx, (unsigned)pl.in.nby, (unsigned)pl.in.nk);
+    const dim3 blk(RX, RY);
+    const RowPair &bx = pl.pair;
     RowLaunch L = pl.v;
     if (st == 0) L = pl.p;  // with the receivers
 #define LEE_RS(WM, TER, ST)                                                                                            \
     do {                                                                                                               \
         if (split) {                                                                                                   \
-            hipLaunchKernelGGL((k_rk_in<T, WM, TER, ST>), box, blk, 0, s, ad, pl.in);                                  \
             hipLaunchKernelGGL((k_rk_row<T, WM, TER, ST, true>), dim3((unsigned)L.first[6]), blk, 0, s, ad, L, st, rec); \
+            if (st == 0 || st == 2)                                                                                    \
+                hipLaunchKernelGGL((k_rk_pair<T, WM, TER, ST != 0>), dim3((unsigned)(bx.nbx * bx.nby * bx.nbz)),        \
+                                   dim3(RX, kPR<T>), 0, s, ad, bx);                                                        \
         } else {                                                                                                       \
             hipLaunchKernelGGL((k_rk_row<T, WM, TER, ST, false>), dim3((unsigned)L.ntx, (unsigned)L.nty, (unsigned)L.z), blk, 0, s, \
                                ad, L, st, rec);                                                                        \

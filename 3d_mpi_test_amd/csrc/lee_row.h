@@ -248,18 +248,28 @@ __device__ __forceinline__ void row_duvw_layers(const AirArgs<T> &a, const Nb<T>
     }
 }
 
-// Inverse metric at point i of row j from the row's and the plane's values: metric /
-// metric_terrain.
-template <typename T, bool TERRAIN>
-__device__ __forceinline__ void row_metric(const Grid<T> &g, int nx, int i, int j, T yy, T zk, T tk, Nb<T> &n)
+// The column's part of the metric at point i of row j: x, and over terrain sh, hx, hy.
+template <typename T> struct RowColumn { T x, sh, hx, hy; };
+template <typename T, bool TERRAIN> __device__ __forceinline__ RowColumn<T> row_column(const Grid<T> &g, int nx, int i, int j)
 {
     const unsigned o = (unsigned)i * (unsigned)sizeof(T);
-    n.zX = T(0); n.zY = T(0);
-    const T xx = ldr<T>(g.mx, 0, o);
+    RowColumn<T> c{ldr<T>(g.mx, 0, o), T(0), T(0), T(0)};
     if constexpr (TERRAIN) {
-        const size_t c = (size_t)nx * j * sizeof(T);
-        const T zz = zk * ldr<T>(g.tsh, c, o);
-        const T Zx = ldr<T>(g.thx, c, o) * tk, Zy = ldr<T>(g.thy, c, o) * tk;
+        const size_t r = (size_t)nx * j * sizeof(T);
+        c.sh = ldr<T>(g.tsh, r, o);
+        c.hx = ldr<T>(g.thx, r, o);
+        c.hy = ldr<T>(g.thy, r, o);
+    }
+    return c;
+}
+// Inverse metric from the column's, the row's and the plane's values: metric / metric_terrain.
+template <typename T, bool TERRAIN> __device__ __forceinline__ void row_metric(const RowColumn<T> &c, T yy, T zk, T tk, Nb<T> &n)
+{
+    n.zX = T(0); n.zY = T(0);
+    const T xx = c.x;
+    if constexpr (TERRAIN) {
+        const T zz = zk * c.sh;
+        const T Zx = c.hx * tk, Zy = c.hy * tk;
         const T J = T(1) / (xx * yy * zz);
         n.mX = (yy * zz) * J;
         n.mY = (xx * zz) * J;
@@ -275,6 +285,11 @@ __device__ __forceinline__ void row_metric(const Grid<T> &g, int nx, int i, int 
         n.mX = xx; n.mY = yy; n.mZ = zk;
     }
 }
+template <typename T, bool TERRAIN>
+__device__ __forceinline__ void row_metric(const Grid<T> &g, int nx, int i, int j, T yy, T zk, T tk, Nb<T> &n)
+{
+    row_metric<T, TERRAIN>(row_column<T, TERRAIN>(g, nx, i, j), yy, zk, tk, n);
+}
 
 // Reader of a field at offsets (di, dj, dk) from the lane's point.
 template <typename T> struct RowAt {
@@ -286,26 +301,37 @@ template <typename T> struct RowAt {
     }
 };
 
+// Reader of the state around a point: field C (0 .. 3: u v w p, 4: the pressure the velocities
+// read, of level n+1 in the FB step) at an offset.
+template <typename T> struct RowState {
+    const Grid<T> &g;
+    const RowAt<T> &at;
+    template <int C> __device__ __forceinline__ T get(int di, int dj, int dk) const
+    {
+        return at(C == 0 ? g.un : C == 1 ? g.vn : C == 2 ? g.wn : C == 3 ? g.pn : g.pnn, di, dj, dk);
+    }
+};
+
 // The pressure increment without the layer terms, with the damped terms they use: dp_core for
 // no mean flow and the log wind (WM 0, 2), the three-component mean flow (WM 1) in the form of
-// air_dp.  n holds the metric; CEN: central convective differences (RK4).
-template <typename T, int WM, bool TERRAIN, bool CEN>
-__device__ __forceinline__ T row_dp(const AirArgs<T> &a, const RowAt<T> &at, Nb<T> &n, T &ddx, T &ddy, T &dwz)
+// air_dp.  n holds the metric; CEN: central convective differences (RK4).  The state comes
+// from st, the mean flow from at.
+template <typename T, int WM, bool TERRAIN, bool CEN, typename W, typename S>
+__device__ __forceinline__ T row_dp(const AirArgs<T> &a, const W &at, const S &st, Nb<T> &n, T &ddx, T &ddy, T &dwz)
 {
     const Grid<T> &g = a.g;
-    gptr<const T> u = g.un, v = g.vn, w = g.wn, p = g.pn;
-    n.pc = at(p, 0, 0, 0);
-    n.uc = at(u, 0, 0, 0); n.vc = at(v, 0, 0, 0); n.wc = at(w, 0, 0, 0);
-    n.u_ip = at(u, 1, 0, 0); n.v_jp = at(v, 0, 1, 0); n.w_kp = at(w, 0, 0, 1);
-    if constexpr (TERRAIN) { n.u_kp = at(u, 0, 0, 1); n.v_kp = at(v, 0, 0, 1); }
+    n.pc = st.template get<3>(0, 0, 0);
+    n.uc = st.template get<0>(0, 0, 0); n.vc = st.template get<1>(0, 0, 0); n.wc = st.template get<2>(0, 0, 0);
+    n.u_ip = st.template get<0>(1, 0, 0); n.v_jp = st.template get<1>(0, 1, 0); n.w_kp = st.template get<2>(0, 0, 1);
+    if constexpr (TERRAIN) { n.u_kp = st.template get<0>(0, 0, 1); n.v_kp = st.template get<1>(0, 0, 1); }
     if constexpr (WM == 2) {
         n.Vc = at(a.V, 0, 0, 0); n.V_jp = at(a.V, 0, 1, 0); n.V_jm = at(a.V, 0, -1, 0);
-        n.p_jm = at(p, 0, -1, 0);
-        if constexpr (CEN) n.p_jp = at(p, 0, 1, 0);
+        n.p_jm = st.template get<3>(0, -1, 0);
+        if constexpr (CEN) n.p_jp = st.template get<3>(0, 1, 0);
         if constexpr (TERRAIN) {
             n.V_kp = at(a.V, 0, 0, 1); n.V_km = at(a.V, 0, 0, -1);
-            n.p_km = at(p, 0, 0, -1);
-            if constexpr (CEN) n.p_kp = at(p, 0, 0, 1);
+            n.p_km = st.template get<3>(0, 0, -1);
+            if constexpr (CEN) n.p_kp = st.template get<3>(0, 0, 1);
         }
     }
     if constexpr (WM != 1) {
@@ -329,35 +355,33 @@ __device__ __forceinline__ T row_dp(const AirArgs<T> &a, const RowAt<T> &at, Nb<
         }
         T r;
         if constexpr (CEN)
-            r = ((-c1) * ((at(p, 1, 0, 0) - at(p, -1, 0, 0)) * T(0.5)) - c2 * ((at(p, 0, 1, 0) - at(p, 0, -1, 0)) * T(0.5))) -
-                c3 * ((at(p, 0, 0, 1) - at(p, 0, 0, -1)) * T(0.5));
+            r = ((-c1) * ((st.template get<3>(1, 0, 0) - st.template get<3>(-1, 0, 0)) * T(0.5)) - c2 * ((st.template get<3>(0, 1, 0) - st.template get<3>(0, -1, 0)) * T(0.5))) -
+                c3 * ((st.template get<3>(0, 0, 1) - st.template get<3>(0, 0, -1)) * T(0.5));
         else
-            r = ((-c1) * (pc - at(p, -1, 0, 0)) - c2 * (pc - at(p, 0, -1, 0))) - c3 * (pc - at(p, 0, 0, -1));
+            r = ((-c1) * (pc - st.template get<3>(-1, 0, 0)) - c2 * (pc - st.template get<3>(0, -1, 0))) - c3 * (pc - st.template get<3>(0, 0, -1));
         r += (((-a.gam) * pc) * dt) * ((UX + VY) + WZ);
         return r + r0;
     }
 }
 
 // The velocity increments without the layer terms, with the pressure gradients they use:
-// duvw_core (WM 0, 2), or the form of air_duvw (WM 1).  The pressure is read from g.pnn.
-template <typename T, int WM, bool TERRAIN, bool CEN>
-__device__ __forceinline__ void row_duvw(const AirArgs<T> &a, const RowAt<T> &at, Nb<T> &n, T &gpx, T &gpy, T &gpz, T &du,
+// duvw_core (WM 0, 2), or the form of air_duvw (WM 1).
+template <typename T, int WM, bool TERRAIN, bool CEN, typename W, typename S>
+__device__ __forceinline__ void row_duvw(const AirArgs<T> &a, const W &at, const S &st, Nb<T> &n, T &gpx, T &gpy, T &gpz, T &du,
                                          T &dv, T &dw)
 {
-    const Grid<T> &g = a.g;
-    gptr<const T> u = g.un, v = g.vn, w = g.wn, p = g.pnn;
-    n.uc = at(u, 0, 0, 0); n.vc = at(v, 0, 0, 0); n.wc = at(w, 0, 0, 0);
-    n.pc = at(p, 0, 0, 0);
-    n.p_im = at(p, -1, 0, 0); n.p_jm = at(p, 0, -1, 0); n.p_km = at(p, 0, 0, -1);
+    n.uc = st.template get<0>(0, 0, 0); n.vc = st.template get<1>(0, 0, 0); n.wc = st.template get<2>(0, 0, 0);
+    n.pc = st.template get<4>(0, 0, 0);
+    n.p_im = st.template get<4>(-1, 0, 0); n.p_jm = st.template get<4>(0, -1, 0); n.p_km = st.template get<4>(0, 0, -1);
     if constexpr (WM == 2) {
         n.Vc = at(a.V, 0, 0, 0);
         n.V_ip = at(a.V, 1, 0, 0); n.V_im = at(a.V, -1, 0, 0); n.V_jp = at(a.V, 0, 1, 0); n.V_jm = at(a.V, 0, -1, 0);
         n.V_kp = at(a.V, 0, 0, 1); n.V_km = at(a.V, 0, 0, -1);
-        n.u_jp = at(u, 0, 1, 0); n.v_jp = at(v, 0, 1, 0); n.w_jp = at(w, 0, 1, 0);
-        if constexpr (CEN) { n.u_jm = at(u, 0, -1, 0); n.v_jm = at(v, 0, -1, 0); n.w_jm = at(w, 0, -1, 0); }
+        n.u_jp = st.template get<0>(0, 1, 0); n.v_jp = st.template get<1>(0, 1, 0); n.w_jp = st.template get<2>(0, 1, 0);
+        if constexpr (CEN) { n.u_jm = st.template get<0>(0, -1, 0); n.v_jm = st.template get<1>(0, -1, 0); n.w_jm = st.template get<2>(0, -1, 0); }
         if constexpr (TERRAIN) {
-            n.u_kp = at(u, 0, 0, 1); n.v_kp = at(v, 0, 0, 1); n.w_kp = at(w, 0, 0, 1);
-            if constexpr (CEN) { n.u_km = at(u, 0, 0, -1); n.v_km = at(v, 0, 0, -1); n.w_km = at(w, 0, 0, -1); }
+            n.u_kp = st.template get<0>(0, 0, 1); n.v_kp = st.template get<1>(0, 0, 1); n.w_kp = st.template get<2>(0, 0, 1);
+            if constexpr (CEN) { n.u_km = st.template get<0>(0, 0, -1); n.v_km = st.template get<1>(0, 0, -1); n.w_km = st.template get<2>(0, 0, -1); }
         }
     }
     if constexpr (WM != 1) {
@@ -365,7 +389,7 @@ __device__ __forceinline__ void row_duvw(const AirArgs<T> &a, const RowAt<T> &at
     } else {
         T d0, d1, d2;
         duvw_core<T, 0, TERRAIN, CEN>(a, n, gpx, gpy, gpz, d0, d1, d2);  // (-Aav dt) grad p
-        const T dxi = g.dxi, dyi = g.dyi, dzi = g.dzi, dt = g.dt;
+        const T dxi = a.g.dxi, dyi = a.g.dyi, dzi = a.g.dzi, dt = a.g.dt;
         const T mX = n.mX, mY = n.mY, mZ = n.mZ, zX = n.zX, zY = n.zY, uc = n.uc, vc = n.vc, wc = n.wc;
         const T Uc = at(a.U, 0, 0, 0), Vc = at(a.V, 0, 0, 0), Wc = at(a.W, 0, 0, 0);
         const T c1 = ((Uc * mX) * dxi) * dt, c2 = ((Vc * mY) * dyi) * dt;
@@ -383,21 +407,22 @@ __device__ __forceinline__ void row_duvw(const AirArgs<T> &a, const RowAt<T> &at
             return q;
         };
         auto gz = [&](gptr<const T> F) { return ((mZ * (at(F, 0, 0, 1) - at(F, 0, 0, -1))) * dzi) * T(0.5); };
-        auto cv = [&](gptr<const T> F, T fc) {
+        auto cv = [&](auto C, T fc) {
+            constexpr int F = decltype(C)::value;
             if constexpr (CEN)
-                return ((-c1) * ((at(F, 1, 0, 0) - at(F, -1, 0, 0)) * T(0.5)) -
-                        c2 * ((at(F, 0, 1, 0) - at(F, 0, -1, 0)) * T(0.5))) -
-                       c3 * ((at(F, 0, 0, 1) - at(F, 0, 0, -1)) * T(0.5));
+                return ((-c1) * ((st.template get<F>(1, 0, 0) - st.template get<F>(-1, 0, 0)) * T(0.5)) -
+                        c2 * ((st.template get<F>(0, 1, 0) - st.template get<F>(0, -1, 0)) * T(0.5))) -
+                       c3 * ((st.template get<F>(0, 0, 1) - st.template get<F>(0, 0, -1)) * T(0.5));
             else
-                return ((-c1) * (at(F, 1, 0, 0) - fc) - c2 * (at(F, 0, 1, 0) - fc)) - c3 * (at(F, 0, 0, 1) - fc);
+                return ((-c1) * (st.template get<F>(1, 0, 0) - fc) - c2 * (st.template get<F>(0, 1, 0) - fc)) - c3 * (st.template get<F>(0, 0, 1) - fc);
         };
-        du = cv(u, uc);
+        du = cv(std::integral_constant<int, 0>{}, uc);
         du += (((-uc) * gx(a.U)) * dt - (vc * gy(a.U)) * dt) - (wc * gz(a.U)) * dt;
         du += d0;
-        dv = cv(v, vc);
+        dv = cv(std::integral_constant<int, 1>{}, vc);
         dv += (((-uc) * gx(a.V)) * dt - (vc * gy(a.V)) * dt) - (wc * gz(a.V)) * dt;
         dv += d1;
-        dw = cv(w, wc);
+        dw = cv(std::integral_constant<int, 2>{}, wc);
         dw += (((-uc) * gx(a.W)) * dt - (vc * gy(a.W)) * dt) - (wc * gz(a.W)) * dt;
         dw += d2;
     }
