@@ -665,8 +665,7 @@ template <typename T> void rk_row_args(lee_ctx *c, int st, int J1, int y1on, boo
             buf[d][3][f] = (T *)c->rk_sc[d][f];
         }
     r.geo = row_geo(c);
-    r.ntile = c->plan.p.ntx * c->plan.p.nty;
-    r.zair = m.nz - 2;
+    r.whole = c->plan.w[1];
     r.yl = (const RowLine<T> *)c->row_lines;
     r.zl = (const RowLine<T> *)c->row_lines + m.ny;
     r.xs = (const T *)c->xprof[0]; r.xc = (const T *)c->xprof[1]; r.xd = (const T *)c->xprof[2];
@@ -1364,12 +1363,15 @@ int create_impl(const lee_deck *deck, const lee_options *opt, lee_ctx **out)
         for (int s = 0; s < 6; ++s) { rg.qn[s] = m.slab[s].n; rg.qlo[s] = m.slab[s].lo; }
         std::vector<int> ring;
         row_plan(C->plan, ring, rg);
+        const size_t nring = ring.size();
+        ring.insert(ring.end(), C->plan.list.begin(), C->plan.list.end());
         if (!ring.empty()) {
             if ((rc = dalloc(C, (void **)&C->ring, ring.size() * sizeof(int)))) return rc;
             HIPCHK(C, hipMemcpyAsync(C->ring, ring.data(), ring.size() * sizeof(int), hipMemcpyHostToDevice, C->stream));
             HIPCHK(C, hipStreamSynchronize(C->stream));
         }
         C->plan.p.ring = C->plan.v.ring = C->ring;
+        C->plan.w[0].ring = C->plan.w[1].ring = C->ring + nring;
         // narrow columns without a flow, hills, the East impedance or a layer along x or y; a
         // launch form that the caller names is the one that runs
         if (!m.rk4 && o.fb_form == 0 && o.path != LEE_PATH_FUSED && !m.has_wind && !m.terrain && !m.east_tdbc &&
@@ -2185,7 +2187,8 @@ struct lee_ensemble {
     std::string err;
     std::vector<void *> allocs;
     void *air_args[4] = {}, *pore_args[4] = {}, *bnd_args[4] = {};
-    // block prefixes [air n+1 | pore np+1 | bnd n+1 | rows n+1] (np porous members)
+    // block prefixes [air n+1 | pore np+1 | bnd n+1] (np porous members), then the member of each
+    // block of the row form
     int *first = nullptr;
     int air_blocks = 0, pore_blocks = 0, bnd_blocks = 0, n_pore = 0;
     // row form (every member can run it): one launch per stage over all members' tiles, the
@@ -2328,10 +2331,10 @@ template <typename T> int ens_step(lee_ensemble *e, double *rec_slot)
     }
     hipStream_t s = e->stream;
     launch_sample_batch<T>((const T *const *)e->rec_p, e->rec_idx, e->nrec, rec_slot, s);
-    const int *fb = e->first + n + 1 + e->n_pore + 1, *fr = fb + n + 1;
+    const int *fb = e->first + n + 1 + e->n_pore + 1, *member = fb + n + 1;
     for (int st = 0; st < 4; ++st) {
         if (e->rows) {
-            launch_rk_row_batch<T>((const RkRowArgs<T> *)e->row_args + (size_t)(4 * e->par + st) * n, fr, n, e->row_blocks, st,
+            launch_rk_row_batch<T>((const RkRowArgs<T> *)e->row_args + (size_t)(4 * e->par + st) * n, member, e->row_blocks, st,
                                    e->wind, e->terrain, s);
             continue;
         }
@@ -2484,7 +2487,7 @@ int lee_ensemble_create(int n, const lee_deck *decks, const lee_options *opts, l
     std::vector<int> first(fa);
     first.insert(first.end(), fp.begin(), fp.end());
     first.insert(first.end(), fb.begin(), fb.end());
-    first.insert(first.end(), fr.begin(), fr.end());
+    for (int d = 0; d < n && E->rows; ++d) first.insert(first.end(), (size_t)(fr[d + 1] - fr[d]), d);
     if (E->rows) {
         const size_t sz = E->prec == 64 ? sizeof(RkRowArgs<double>) : sizeof(RkRowArgs<float>);
         if ((rc = ens_alloc(E, &E->row_args, (size_t)8 * n * sz))) return rc;

@@ -680,15 +680,27 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
             }
         }
     }
-    ring.clear();
-    if (pl.has_in)
-        for (int ty = 0; ty < nty; ++ty)
-            for (int tx = 0; tx < ntx; ++tx)
-                if (m.rk4 ? i0 + RX * tx < pl.pair.xa || i0 + RX * (tx + 1) > pl.pair.xb || j0 + RY * ty < pl.pair.ya ||
-                                j0 + RY * (ty + 1) > pl.pair.yb
-                          : tx < tx0 || tx >= tx1 || ty < ty0 || ty >= ty1)
-                    ring.push_back(tx | (ty << 16));
     const int full = ntx * nty, nrp = (m.nrec + full * RX * RY - 1) / (full * RX * RY);
+    // tile rows outside the y layers, neither the first (face row) nor the last (East extrapolation)
+    const int jy0 = m.qn[2] ? m.qlo[2] + m.qn[2] : 0, jy1 = m.qn[3] ? m.qlo[3] : m.ny;
+    auto packs = [&](RowLaunch &l, int most, int xlo, int xhi, int ya, int yb) {  // strips [0, xlo) and [xhi, nx)
+        const int ta = std::max(1, (std::max(ya, jy0) - j0 + RY - 1) / RY), tb = std::min(nty - 1, (std::min(yb, jy1) - j0) / RY);
+        if (tb <= ta) return;
+        for (int q = 0; q < 2; ++q) {
+            const int x0 = q ? xhi : 0, n = q ? m.nx - xhi : xlo;
+            if (n >= 1 && n <= most) l.strip[l.nstrip++] = RowStrip{x0, n, RX / n, 65536 / n + 1};
+        }
+        l.ja = j0 + RY * ta; l.jb = j0 + RY * tb;
+    };
+    auto packed = [&](const RowLaunch &l, int tx, int ty) {  // the tile's points are strips' (or the interior's)
+        if (!l.nstrip || j0 + RY * ty < l.ja || j0 + RY * (ty + 1) > l.jb) return false;
+        const int x0 = i0 + RX * tx, x1 = std::min(x0 + RX, m.nx);
+        for (int q = 0; q < l.nstrip; ++q) {
+            const int a = l.strip[q].x0, b = a + l.strip[q].n;
+            if (std::max(a, x0) < std::min(b, x1)) return true;
+        }
+        return false;
+    };
     for (int ph = 0; ph < 2; ++ph) {
         RowLaunch &l = ph ? pl.v : pl.p;
         l.ntx = ntx; l.nty = nty;
@@ -699,13 +711,52 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
         l.z = l.zair + l.zpore + l.zground + (ph ? 0 : nrp);
         l.ka = za; l.kb = zb;
         l.xa = pl.pair.xa; l.xb = pl.pair.xb; l.ya = pl.pair.ya; l.yb = pl.pair.yb;
-        l.nring = (int)ring.size() ? (int)ring.size() : 1;
-        if (pl.has_in) {
-            const int per[6] = {full * (za - 1), full * (m.nz - 1 - zb), (int)ring.size() * (zb - za), full * l.zpore,
-                                full * l.zground, ph ? 0 : (m.nrec + RX * RY - 1) / (RX * RY)};
-            l.first[0] = 0;
-            for (int q = 0; q < 6; ++q) l.first[q + 1] = l.first[q] + per[q];
+        RowLaunch &w = pl.w[ph];
+        if (m.rk4) {
+            w = l;
+            w.xa = w.xb = w.ya = w.yb = 0;
+            w.ka = 2; w.kb = std::max(2, m.nz - 2);
+            const int tail = i0 + RX * (ntx - 1);
+            packs(w, RX / 3, 0, ntx > 1 ? tail : m.nx, 0, m.ny);
+            w.grid = !w.nstrip;
+            if (w.grid) w.ka = w.kb = 1;  // (an ensemble's blocks: whole planes)
+            if (pl.has_in) packs(l, RX / 2, l.xa, l.xb, l.ya, l.yb);
         }
+        auto sections = [&](RowLaunch &r, int tiles) {
+            r.nring = tiles ? tiles : 1;
+            auto inverse = [](int d) { return d > 1 ? (unsigned)(((1ULL << 32) + d - 1) / d) : ~0u; };
+            r.by_full = inverse(full); r.by_ntx = inverse(ntx); r.by_ring = inverse(r.nring);
+            const int per[6] = {full * (r.ka - 1), full * (m.nz - 1 - r.kb), tiles * (r.kb - r.ka), full * r.zpore, full * r.zground,
+                                ph ? 0 : (m.nrec + RX * RY - 1) / (RX * RY)};
+            r.first[0] = 0;
+            for (int q = 0; q < 6; ++q) r.first[q + 1] = r.first[q] + per[q];
+        };
+        if (!ph) {
+            ring.clear();
+            pl.list.clear();
+            auto strips = [&](std::vector<int> &list, const RowLaunch &r, int ty) {  // those that start in tile row ty
+                for (int q = 0; q < r.nstrip; ++q)
+                    for (int b = 0; r.ja + RY * r.strip[q].rows * b < r.jb; ++b)
+                        if ((r.ja + RY * r.strip[q].rows * b - j0) / RY == ty) list.push_back(kStripBlock | q << 20 | b);
+            };
+            for (int ty = 0; ty < nty; ++ty) {
+                for (int tx = 0; tx < ntx; ++tx) {
+                    const int e = tx | (ty << 16);
+                    const bool in = m.rk4 ? i0 + RX * tx >= pl.pair.xa && i0 + RX * (tx + 1) <= pl.pair.xb &&
+                                                j0 + RY * ty >= pl.pair.ya && j0 + RY * (ty + 1) <= pl.pair.yb
+                                          : tx >= tx0 && tx < tx1 && ty >= ty0 && ty < ty1;
+                    if (pl.has_in && !in && !packed(l, tx, ty)) ring.push_back(e);
+                    if (m.rk4 && !packed(w, tx, ty)) pl.list.push_back(e);
+                }
+                if (m.rk4) {
+                    if (pl.has_in) strips(ring, l, ty);
+                    strips(pl.list, w, ty);
+                }
+            }
+        }
+        if (pl.has_in) sections(l, (int)ring.size());
+        else l.nring = 1;
+        if (m.rk4) sections(w, (int)pl.list.size());
     }
 }
 

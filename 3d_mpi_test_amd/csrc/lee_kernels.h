@@ -164,10 +164,21 @@ struct RowBox { int tx, nbx, ty, nby, k, nk, i0, j0; };
 // porous planes, the ground plane and the receivers.  Around an interior box: blocks first[q] ..
 // first[q+1]-1 of section q (planes 1 .. ka-1, planes kb .., the ring of planes ka .. kb-1 listed
 // in `ring` as tx | ty << 16, porous, ground, receivers).
+// RK4: strips of n <= 32 columns from x0, which whole tiles would leave mostly empty (what an
+// interior leaves of the outer tiles, or a row's narrow last tile): `rows` rows per wavefront, on
+// the rows [ja, jb) outside the y layers, in the planes ka .. kb - 1.  Their blocks stand in the
+// list of those planes' tiles as kStripBlock | strip << 20 | block; the list is in the order of the
+// rows.
+constexpr int kStripBlock = 1 << 30;
+struct RowStrip { int x0, n, rows, inv; };  // inv: lane / n = lane * inv >> 16
 struct RowLaunch {
     int ntx, nty, z, zair, zpore, zground;
     int ka, kb, nring;
     int xa, xb, ya, yb;  // RK4: the interior's points, which the ring's tiles leave out
+    int ja, jb, nstrip;
+    int grid;  // RK4: a grid of tiles and planes after all
+    RowStrip strip[2];
+    unsigned by_full, by_ntx, by_ring;  // 2^32 / divisor, rounded up
     int first[7];
     const int *ring;
 };
@@ -183,6 +194,8 @@ struct RowPlan {
     RowBox in;     // FB
     RowPair pair;  // RK4
     RowLaunch p, v;
+    RowLaunch w[2];        // RK4, the whole domain: stage 0 (with the receivers), the others
+    std::vector<int> list; // and the tiles of its planes ka .. kb - 1, as the ring's
 };
 struct RowGeom {
     int nx, ny, nz, pnz, coupled, ground, nrec, rk4;
@@ -242,7 +255,8 @@ template <typename T> struct RKBndArgs {
 // an ensemble, which has no interior kernel.
 template <typename T> struct RkRowArgs {
     RowGeo geo;
-    int first, ntile, zair;  // ensemble: the member's first block, tiles per plane, air planes
+    int first;                   // ensemble: the member's first block
+    RowLaunch whole;             // and its blocks
     gptr<const RowLine<T>> yl, zl;
     gptr<const T> xs, xc, xd;
     RowQ<T> q[3];
@@ -261,10 +275,11 @@ template <typename T> struct RkRowArgs {
 // stage st + 1).  Stage 0 samples the receivers into rec.
 template <typename T> void launch_rk_row(const RkRowArgs<T> *ad, const RowPlan &pl, int st, int wind, bool terrain, bool split,
                                          double *rec, hipStream_t s);
-// The same for n domains (their arguments one after the other), nblocks blocks in all.
-template <typename T> void launch_rk_row_batch(const RkRowArgs<T> *ad, const int *first, int n, int nblocks, int st, int wind,
+// The same for n domains (their arguments one after the other), nblocks blocks in all; member:
+// the domain of each block.
+template <typename T> void launch_rk_row_batch(const RkRowArgs<T> *ad, const int *member, int nblocks, int st, int wind,
                                                bool terrain, hipStream_t s);
-inline long long row_batch_blocks(const RowPlan &p) { return (long long)p.v.ntx * p.v.nty * (p.v.zair + p.v.zpore); }
+inline long long row_batch_blocks(const RowPlan &p) { return p.w[1].first[6]; }
 // wind: 0 none, 1 U V W fields, 2 V only (U = W = 0: velocity_method 7)
 // r: the stage arguments on the host (grid shape), rd: the same in device memory (read by
 // the kernel)

@@ -90,19 +90,25 @@ __device__ __forceinline__ T rk_point_if(int st, T xn, T k, T acc, T lo, T err, 
 // layer terms read.
 template <typename T> struct RkE { T u0, ui, uk, v0, vj, vk, w0, wk, p0, pi, pj, pk; };
 
+// Where a wavefront's lanes stand: a row jb (uniform) that addresses start from, the lane's row j
+// (jb, or one of the next ones) and the byte offsets of its point and node from row jb's first.
+struct RowPos {
+    int jb, j;
+    unsigned op, on;
+};
 // dt R of the four fields at the lane's point; xc: the stage state there.
 template <typename T, int WM, bool TERRAIN, int ST, bool X, bool Y, bool Z>
-__device__ __forceinline__ void rk_row_point(const RkRowArgs<T> &A, const RowGeo &G, const RowLane &l, int j, int k,
+__device__ __forceinline__ void rk_row_point(const RkRowArgs<T> &A, const RowGeo &G, const RowLane &l, const RowPos &ps, int k,
                                              const RowLine<T> &yl, const RowLine<T> &zl, const RowSlab<T> &sy,
                                              const RowSlab<T> &sz, T (&xc)[4], T (&kf)[4])
 {
     const AirArgs<T> &a = A.a;
     const Grid<T> &g = a.g;
     const size_t snx = (size_t)G.nx * sizeof(T), sxy = snx * G.ny;
-    const unsigned op = (unsigned)l.ip * (unsigned)sizeof(T);
-    const RowAt<T> at{snx * j + sxy * k, snx, sxy, op};
+    const unsigned op = ps.op, ox = (unsigned)l.ip * (unsigned)sizeof(T);
+    const RowAt<T> at{snx * ps.jb + sxy * k, snx, sxy, op};
     Nb<T> n;
-    row_metric<T, TERRAIN>(g, G.nx, l.ip, j, yl.m, zl.m, zl.t, n);
+    row_metric<T, TERRAIN>(row_column<T, TERRAIN>(g, G.nx, l.ip, ps.jb, op), yl.m, zl.m, zl.t, n);
     Lay<T> lx{}, ly{}, lz{};
     QP<T> px{}, py{}, pz{};
     QV<T> vx{}, vy{}, vz{};
@@ -123,9 +129,9 @@ __device__ __forceinline__ void rk_row_point(const RkRowArgs<T> &A, const RowGeo
         else return q + d;
     };
     if constexpr (X) {
-        const RowX q = row_x<T>(G, l.ip, j, k);
+        const RowX q = row_x<T>(G, l.ip, ps.j, k);
         const RowQ<T> &Q = A.q[0];
-        lx = {ldr<T>(A.xs, 0, op), ldr<T>(A.xc, 0, op), (Y || Z) ? ldr<T>(A.xd, 0, op) : T(0), q.act};
+        lx = {ldr<T>(A.xs, 0, ox), ldr<T>(A.xc, 0, ox), (Y || Z) ? ldr<T>(A.xd, 0, ox) : T(0), q.act};
         px.v0 = s(ldr<T>(Q.o[1], 0, q.o), e.v0); px.vj = s(ldr<T>(Q.o[1], 0, q.o + q.dj), e.vj);
         px.w0 = s(ldr<T>(Q.o[2], 0, q.o), e.w0); px.wk = s(ldr<T>(Q.o[2], 0, q.o + q.dk), e.wk);
         if constexpr (TERRAIN) px.vk = s(ldr<T>(Q.o[1], 0, q.o + q.dk), e.vk);
@@ -184,17 +190,18 @@ __device__ __forceinline__ void rk_row_point(const RkRowArgs<T> &A, const RowGeo
 template <typename T> struct RkAux {
     RowX x;
     RowSlab<T> y, z;
+    unsigned o;
     T q[3][4];
 };
 template <typename T>
 __device__ __forceinline__ void rk_aux_read(const RkRowArgs<T> &A, const RowGeo &G, const RowLine<T> &yl, const RowLine<T> &zl, int i,
-                                            int j, int k, RkAux<T> &r)
+                                            const RowPos &ps, int k, RkAux<T> &r)
 {
-    const unsigned o = (unsigned)i * (unsigned)sizeof(T);
-    const size_t row = (size_t)G.nx * ((size_t)j + (size_t)G.ny * k) * sizeof(T);
-    r.x = row_x<T>(G, i, j, k);
+    const unsigned o = r.o = ps.on;
+    const size_t row = (size_t)G.nx * ((size_t)ps.jb + (size_t)G.ny * k) * sizeof(T);
+    r.x = row_x<T>(G, i, ps.j, k);
     r.y = row_slab_y(yl, G.nx, k);
-    r.z = row_slab_z(zl, G.nx, G.ny, j);
+    r.z = row_slab_z(zl, G.nx, G.ny, ps.jb);
     if (!r.x.own && !r.y.in && !r.z.in) return;
     const T dt = A.a.g.dt;
     gptr<const T> c[4] = {A.a.g.un, A.a.g.vn, A.a.g.wn, A.a.g.pn};
@@ -211,9 +218,9 @@ __device__ __forceinline__ void rk_aux_read(const RkRowArgs<T> &A, const RowGeo 
         r.q[2][f] = (((qz + b0) + b1) + b2) + b3;
     }
 }
-template <typename T> __device__ __forceinline__ void rk_aux_write(const RkRowArgs<T> &A, int i, const RkAux<T> &r)
+template <typename T> __device__ __forceinline__ void rk_aux_write(const RkRowArgs<T> &A, const RkAux<T> &r)
 {
-    const unsigned o = (unsigned)i * (unsigned)sizeof(T);
+    const unsigned o = r.o;
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
         if (r.x.own) str<T>(A.q[0].n[f], 0, r.x.o, r.q[0][f]);
@@ -235,9 +242,9 @@ __device__ __forceinline__ void rk_node(const RkRowArgs<T> &A, const RowGeo &G, 
     const unsigned o = (unsigned)i * (unsigned)sizeof(T);
     if constexpr (ST == 3) {
         RkAux<T> r;
-        rk_aux_read(A, G, row_line(A.yl, j), row_line(A.zl, k), i, j, k, r);
+        rk_aux_read(A, G, row_line(A.yl, j), row_line(A.zl, k), i, RowPos{j, j, o, o}, k, r);
         rk_store4(A.dst, row, o, v);
-        rk_aux_write(A, i, r);
+        rk_aux_write(A, r);
     } else {
         rk_store4(A.dst, row, o, v);
     }
@@ -298,12 +305,60 @@ __device__ __forceinline__ void rk_row_pore(const RkRowArgs<T> &A, const RowGeo 
     }
 }
 
-// MODE 0: the whole domain, 1: around the interior box, 2: an ensemble.
+// The air point of a lane: registers, stencil, stores of its node (d: the destination state).
+// YS: the row may lie in a y layer.
+template <typename T, int WM, bool TERRAIN, int ST, bool YS>
+__device__ __forceinline__ void rk_row_air(const RkRowArgs<T> &A, const RowGeo &G, const RowLane &l, const RowPos &ps, int k,
+                                           const RowLine<T> &yl, const RowLine<T> &zl, bool mx, T (&d)[4])
+{
+    constexpr bool COMP = std::is_same<T, float>::value;
+    const int nx = G.nx, ny = G.ny;
+    const RowSlab<T> sy = row_slab_y(yl, nx, k), sz = row_slab_z(zl, nx, ny, ps.jb);
+    const size_t row = (size_t)nx * ((size_t)ps.jb + (size_t)ny * k) * sizeof(T);
+    const unsigned op = ps.op;
+    const size_t e = (size_t)l.ip + (size_t)nx * ((size_t)ps.j + (size_t)ny * k);
+    // the point's registers, the auxiliaries of the last stage, then the stencil
+    T xn[4], ac[4] = {T(0), T(0), T(0), T(0)}, er[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        xn[f] = ST == 0 || (ST == 3 && !COMP) ? T(0) : ldr<T>(A.xn[f], row, op);
+        er[f] = ST == 3 && COMP ? ldr<T>(A.err[f], row, op) : T(0);
+    }
+    if constexpr (ST != 0) acc4_load(A.acc, e, ac);
+    T xc[4], kf[4];
+#define LEE_BODY(X, Y, Z) rk_row_point<T, WM, TERRAIN, ST, X, Y, Z>(A, G, l, ps, k, yl, zl, sy, sz, xc, kf)
+    if (!sz.in) {
+        if (!YS || !sy.in) { if (mx) LEE_BODY(true, false, false); else LEE_BODY(false, false, false); }
+        else { if (mx) LEE_BODY(true, YS, false); else LEE_BODY(false, YS, false); }
+    } else {
+        if (!YS || !sy.in) { if (mx) LEE_BODY(true, false, true); else LEE_BODY(false, false, true); }
+        else { if (mx) LEE_BODY(true, YS, true); else LEE_BODY(false, YS, true); }
+    }
+#undef LEE_BODY
+    T ao[4], eo[4];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) d[f] = rk_point<T, ST>(ST == 0 ? xc[f] : xn[f], kf[f], ac[f], er[f], A.ca, ao[f], eo[f]);
+    if (l.face) d[0] = T(0);
+    if (l.live) {
+        RkAux<T> r;
+        if constexpr (ST == 3) rk_aux_read(A, G, yl, zl, l.in, ps, k, r);
+        rk_store4(A.dst, row, ps.on, d);
+        if (!l.face) {
+            if constexpr (ST != 3) acc4_store(A.acc, e, ao);
+            if constexpr (ST == 3 && COMP) {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) str<T>(A.err[f], row, op, eo[f]);
+            }
+        }
+        if constexpr (ST == 3) rk_aux_write(A, r);
+    }
+}
+
+// MODE 1: a domain (box: the interior its ring's tiles leave out, or empty), 2: an ensemble's.
 template <typename T, int WM, bool TERRAIN, int ST, int MODE>
 __device__ __forceinline__ void rk_row_block(const RkRowArgs<T> &A, int st, int kind, int k, int tx, int ty, long long rec,
                                              double *__restrict__ rec_out, T (&rows)[RY][RX], const int (&box)[4])
 {
-    constexpr bool COMP = std::is_same<T, float>::value;
     const RowGeo G = A.geo;
     const int nx = G.nx, ny = G.ny, nz = G.nz;
     const int lane = threadIdx.x, tj = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
@@ -333,47 +388,8 @@ __device__ __forceinline__ void rk_row_block(const RkRowArgs<T> &A, int st, int 
     }
     T d[4];
     if (kind == RK_AIR) {
-        const RowLine<T> yl = row_line(A.yl, j), zl = row_line(A.zl, k);
-        const RowSlab<T> sy = row_slab_y(yl, nx, k), sz = row_slab_z(zl, nx, ny, j);
-        const bool mx = row_meets_x(G, i0);
-        const size_t row = (size_t)nx * ((size_t)j + (size_t)ny * k) * sizeof(T);
-        const unsigned op = (unsigned)l.ip * (unsigned)sizeof(T);
-        const size_t e = (size_t)l.ip + (size_t)nx * ((size_t)j + (size_t)ny * k);
-        // the point's registers, the auxiliaries of the last stage, then the stencil
-        T xn[4], ac[4] = {T(0), T(0), T(0), T(0)}, er[4];
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-            xn[f] = ST == 0 || (ST == 3 && !COMP) ? T(0) : ldr<T>(A.xn[f], row, op);
-            er[f] = ST == 3 && COMP ? ldr<T>(A.err[f], row, op) : T(0);
-        }
-        if constexpr (ST != 0) acc4_load(A.acc, e, ac);
-        T xc[4], kf[4];
-#define LEE_BODY(X, Y, Z) rk_row_point<T, WM, TERRAIN, ST, X, Y, Z>(A, G, l, j, k, yl, zl, sy, sz, xc, kf)
-        if (!sz.in) {
-            if (!sy.in) { if (mx) LEE_BODY(true, false, false); else LEE_BODY(false, false, false); }
-            else { if (mx) LEE_BODY(true, true, false); else LEE_BODY(false, true, false); }
-        } else {
-            if (!sy.in) { if (mx) LEE_BODY(true, false, true); else LEE_BODY(false, false, true); }
-            else { if (mx) LEE_BODY(true, true, true); else LEE_BODY(false, true, true); }
-        }
-#undef LEE_BODY
-        T ao[4], eo[4];
-#pragma unroll
-        for (int f = 0; f < 4; ++f) d[f] = rk_point<T, ST>(ST == 0 ? xc[f] : xn[f], kf[f], ac[f], er[f], A.ca, ao[f], eo[f]);
-        if (l.face) d[0] = T(0);
-        if (l.live) {
-            RkAux<T> r;
-            if constexpr (ST == 3) rk_aux_read(A, G, yl, zl, l.in, j, k, r);
-            rk_store4(A.dst, row, (unsigned)l.in * (unsigned)sizeof(T), d);
-            if (!l.face) {
-                if constexpr (ST != 3) acc4_store(A.acc, e, ao);
-                if constexpr (ST == 3 && COMP) {
-#pragma unroll
-                    for (int f = 0; f < 4; ++f) str<T>(A.err[f], row, op, eo[f]);
-                }
-            }
-            if constexpr (ST == 3) rk_aux_write(A, l.in, r);
-        }
+        const RowPos ps{j, j, (unsigned)l.ip * (unsigned)sizeof(T), (unsigned)l.in * (unsigned)sizeof(T)};
+        rk_row_air<T, WM, TERRAIN, ST, true>(A, G, l, ps, k, row_line(A.yl, j), row_line(A.zl, k), row_meets_x(G, i0), d);
     } else {
         rk_row_pore<T, TERRAIN, ST>(A, G, st, l, j, k, d);
         if (l.face) d[0] = T(0);
@@ -411,57 +427,92 @@ __device__ __forceinline__ void rk_row_block(const RkRowArgs<T> &A, int st, int 
     }
 }
 
-template <typename T, int WM, bool TERRAIN, int ST, bool RING>
-__global__ __launch_bounds__(RX * RY) void k_rk_row(const RkRowArgs<T> *__restrict__ ap, RowLaunch L, int st, double *__restrict__ rec_out)
+// A strip's block: 4 x S.rows rows from block row `br`, S.rows of them per wavefront, without a face
+// in y or z (row_plan).  Waves of mostly idle lanes cost as much as full ones: the time of these
+// kernels goes by waves (loads, waits and scalar work each) before it goes by bytes.  us per step
+// before -> after: 137 x 91 x 53 FP64 (rows of 64 + 64 + 9) 196 -> 176, 512 x 256 x 128 (an interior
+// leaves 21 columns of the outer tiles) FP32 1570 -> 1532, FP64 3046 -> 2838, 768 x 384 x 192 FP32
+// (25 columns, two rows a wave) 4217 -> 4140.  Strips wider than a third of a wave at a row's end
+// did not pay (160 = 64 + 64 + 32 columns: 3 % slower).  Also tried: a plane's blocks padded to
+// eights (fewer bytes on small grids, 1-5 % slower on the others) and an eighth of the rows to each
+// XCD (4 % slower in FP32), and half the waves for the pressure, half for the velocities (less than
+// half the registers, 3 instead of 2 waves a SIMD in FP64, and 1.15-1.3 times the time).
+template <typename T, int WM, bool TERRAIN, int ST>
+__device__ __forceinline__ void rk_row_strip(const RkRowArgs<T> &A, const RowStrip &S, int ja, int je, int k, int br)
+{
+    const RowGeo G = A.geo;
+    const int lane = threadIdx.x, tj = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int jb = ja + (RY * br + tj) * S.rows;
+    if (jb >= je) return;
+    int r = (lane * S.inv) >> 16;
+    const int c = lane - r * S.n;
+    const bool live = r < S.rows && jb + r < je;
+    if (!live) r = 0;
+    const RowLane l = row_lane(S.x0 + c, G.nx, live);
+    const RowPos ps{jb, jb + r, (unsigned)(l.ip + G.nx * r) * (unsigned)sizeof(T), (unsigned)(l.in + G.nx * r) * (unsigned)sizeof(T)};
+    RowLine<T> yl{};
+    yl.m = ldr<T>(A.a.g.my, 0, (unsigned)ps.j * (unsigned)sizeof(T));
+    T d[4];
+    rk_row_air<T, WM, TERRAIN, ST, false>(A, G, l, ps, k, yl, row_line(A.zl, k), S.x0 < G.xa || S.x0 + S.n > G.xb, d);
+}
+
+// q / d and the remainder from m = 2^32 / d (rounded up; one too large at most).
+__device__ __forceinline__ int row_div(int q, int d, unsigned m, int &rem)
+{
+    int n = (int)__umulhi((unsigned)q, m);
+    rem = q - n * d;
+    if (rem < 0) { --n; rem += d; }
+    if (rem >= d) { ++n; rem -= d; }
+    return n;
+}
+// Block b of a launch: its section (planes below ka, above kb, the listed blocks of those between,
+// porous layer, receivers), plane and tile.  Without strips or an interior the launch is a grid of
+// tiles and planes instead, which spares the divisions (3 % on 160 x 96 x 64).
+template <typename T, int WM, bool TERRAIN, int ST, int MODE>
+__device__ __forceinline__ void rk_row_any(const RkRowArgs<T> &A, const RowLaunch &L, int b, int st, double *__restrict__ rec_out)
 {
     __shared__ T rows[RY][RX];
-    int kind, k, tx, ty;
-    int box[4] = {0, 0, 0, 0};
-    long long rec = 0;
-    if constexpr (!RING) {
+    int box[4] = {0, 0, 0, 0}, idx, k, tx, ty, kind = RK_AIR, f = 0;
+    if (MODE == 1 && L.grid) {
         const int z = blockIdx.z;
         tx = blockIdx.x; ty = blockIdx.y;
         kind = z < L.zair ? RK_AIR : z < L.zair + L.zpore ? RK_PORE : RK_REC;
         k = kind == RK_AIR ? z + 1 : z - L.zair + 1;
-        rec = ((long long)(z - L.zair - L.zpore) * L.nty + ty) * L.ntx + tx;
-    } else {
-        const int b = blockIdx.x, full = L.ntx * L.nty;
-        int s = 0, f = 0, per = full, k0 = 1;
-        if (b >= L.first[1]) { s = 1; f = L.first[1]; k0 = L.kb; }
-        if (b >= L.first[2]) { s = 2; f = L.first[2]; k0 = L.ka; per = L.nring; }
-        if (b >= L.first[3]) { s = 3; f = L.first[3]; k0 = 1; per = full; }
-        if (b >= L.first[5]) { s = 5; f = L.first[5]; }
-        const int q = b - f, kk = q / per, idx = q - kk * per;
-        kind = s <= 2 ? RK_AIR : s == 3 ? RK_PORE : RK_REC;
-        k = k0 + kk;
-        rec = q;
-        if (s == 2) {
-            const int e = ((const __attribute__((address_space(4))) int *)L.ring)[idx];
-            tx = e & 0xffff; ty = e >> 16;
-            box[0] = L.xa; box[1] = L.xb; box[2] = L.ya; box[3] = L.yb;
-        } else {
-            ty = idx / L.ntx;
-            tx = idx - ty * L.ntx;
+        b = ((z - L.zair - L.zpore) * L.nty + ty) * L.ntx + tx;
+    } else if (b >= L.first[2] && b < L.first[3]) {
+        k = L.ka + row_div(b - L.first[2], L.nring, L.by_ring, idx);
+        const int e = ((const __attribute__((address_space(4))) int *)L.ring)[idx];
+        if (e & kStripBlock) {
+            const bool hi = e & (1 << 20);
+            const RowStrip S{hi ? L.strip[1].x0 : L.strip[0].x0, hi ? L.strip[1].n : L.strip[0].n,
+                             hi ? L.strip[1].rows : L.strip[0].rows, hi ? L.strip[1].inv : L.strip[0].inv};
+            rk_row_strip<T, WM, TERRAIN, ST>(A, S, L.ja, L.jb, k, e & 0xfffff);
+            return;
         }
+        tx = e & 0xffff; ty = e >> 16;
+        box[0] = L.xa; box[1] = L.xb; box[2] = L.ya; box[3] = L.yb;
+    } else {
+        int k0 = 1;
+        if (b >= L.first[1]) { f = L.first[1]; k0 = L.kb; }
+        if (b >= L.first[3]) { f = L.first[3]; k0 = 1; kind = RK_PORE; }
+        if (b >= L.first[5]) { f = L.first[5]; kind = RK_REC; }
+        k = k0 + row_div(b - f, L.ntx * L.nty, L.by_full, idx);
+        ty = row_div(idx, L.ntx, L.by_ntx, tx);
     }
-    rk_row_block<T, WM, TERRAIN, ST, RING ? 1 : 0>(*ap, st, kind, k, tx, ty, rec, rec_out, rows, box);
+    rk_row_block<T, WM, TERRAIN, ST, MODE>(A, st, kind, k, tx, ty, b - f, rec_out, rows, box);
 }
-
-// Ensemble: the block's member by binary search over the block prefix, then its plane and tile.
 template <typename T, int WM, bool TERRAIN, int ST>
-__global__ __launch_bounds__(RX * RY) void k_rk_row_batch(const RkRowArgs<T> *__restrict__ ap, const int *__restrict__ first, int n, int st)
+__global__ __launch_bounds__(RX * RY) void k_rk_row(const RkRowArgs<T> *__restrict__ ap, RowLaunch L, int st, double *__restrict__ rec_out)
 {
-    __shared__ T rows[RY][RX];
-    const int b = blockIdx.x;
-    int lo = 0, hi = n - 1;  // largest member with first[member] <= b
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (first[mid] <= b) lo = mid; else hi = mid - 1;
-    }
-    const RkRowArgs<T> &A = ap[lo];
-    const int t = b - A.first, z = t / A.ntile, idx = t - z * A.ntile, ntx = A.ntile / A.geo.nty, ty = idx / ntx;
-    const int kind = z < A.zair ? RK_AIR : RK_PORE, box[4] = {0, 0, 0, 0};
-    rk_row_block<T, WM, TERRAIN, ST, 2>(A, st, kind, kind == RK_AIR ? z + 1 : z - A.zair + 1, idx - ty * ntx, ty, 0, nullptr, rows, box);
+    rk_row_any<T, WM, TERRAIN, ST, 1>(*ap, L, (int)blockIdx.x, st, rec_out);
+}
+// Ensemble: the members' arguments one after the other, the member of each block from a table (a
+// search over the members' first blocks cost five dependent loads per wavefront).
+template <typename T, int WM, bool TERRAIN, int ST>
+__global__ __launch_bounds__(RX * RY) void k_rk_row_batch(const RkRowArgs<T> *__restrict__ ap, const int *__restrict__ member, int st)
+{
+    const RkRowArgs<T> &A = ap[((const __attribute__((address_space(4))) int *)member)[blockIdx.x]];
+    rk_row_any<T, WM, TERRAIN, ST, 2>(A, A.whole, (int)blockIdx.x - A.first, st, nullptr);
 }
 
 // ---- the interior outside every layer and away from every face: two stages per launch ------
@@ -547,7 +598,7 @@ __global__ __launch_bounds__(RX * kPR<T>) void k_rk_pair(const RkRowArgs<T> *__r
     // error of plane k - 1
     T r[3][4], v[4] = {}, xn[4] = {}, ac[4] = {}, er[4] = {};
     T r2[4], v2 = T(0), xn2[4] = {}, ac2[4] = {}, er2[4] = {};  // the next plane's
-    const RowColumn<T> col = row_column<T, TERRAIN>(g, g.nx, i, j);
+    const RowColumn<T> col = row_column<T, TERRAIN>(g, g.nx, i, j, o);
     const T my = lds_<T>(g.my, j);
     auto column = [&](int k, T(&q)[4]) {
         const RowAt<T> at = at_plane(k);
@@ -671,21 +722,15 @@ __global__ __launch_bounds__(RX * kPR<T>) void k_rk_pair(const RkRowArgs<T> *__r
 template <typename T>
 void launch_rk_row(const RkRowArgs<T> *ad, const RowPlan &pl, int st, int wind, bool terrain, bool split, double *rec, hipStream_t s)
 {
-    const dim3 blk(RX, RY);
     const RowPair &bx = pl.pair;
-    RowLaunch L = pl.v;
-    if (st == 0) L = pl.p;  // with the receivers
+    const RowLaunch &L = split ? st ? pl.v : pl.p : st ? pl.w[1] : pl.w[0];  // stage 0 with the receivers
+    const dim3 blocks = L.grid ? dim3((unsigned)L.ntx, (unsigned)L.nty, (unsigned)L.z) : dim3((unsigned)L.first[6]);
 #define LEE_RS(WM, TER, ST)                                                                                            \
     do {                                                                                                               \
-        if (split) {                                                                                                   \
-            hipLaunchKernelGGL((k_rk_row<T, WM, TER, ST, true>), dim3((unsigned)L.first[6]), blk, 0, s, ad, L, st, rec); \
-            if (st == 0 || st == 2)                                                                                    \
-                hipLaunchKernelGGL((k_rk_pair<T, WM, TER, ST != 0>), dim3((unsigned)(bx.nbx * bx.nby * bx.nbz)),        \
-                                   dim3(RX, kPR<T>), 0, s, ad, bx);                                                        \
-        } else {                                                                                                       \
-            hipLaunchKernelGGL((k_rk_row<T, WM, TER, ST, false>), dim3((unsigned)L.ntx, (unsigned)L.nty, (unsigned)L.z), blk, 0, s, \
-                               ad, L, st, rec);                                                                        \
-        }                                                                                                              \
+        hipLaunchKernelGGL((k_rk_row<T, WM, TER, ST>), blocks, dim3(RX, RY), 0, s, ad, L, st, rec);                     \
+        if (split && (st == 0 || st == 2))                                                                             \
+            hipLaunchKernelGGL((k_rk_pair<T, WM, TER, ST != 0>), dim3((unsigned)(bx.nbx * bx.nby * bx.nbz)),            \
+                               dim3(RX, kPR<T>), 0, s, ad, bx);                                                        \
     } while (0)
 #define LEE_RT(WM, TER)                                                                            \
     do {                                                                                           \
@@ -697,11 +742,11 @@ void launch_rk_row(const RkRowArgs<T> *ad, const RowPlan &pl, int st, int wind, 
 #undef LEE_RS
 }
 template <typename T>
-void launch_rk_row_batch(const RkRowArgs<T> *ad, const int *first, int n, int nblocks, int st, int wind, bool terrain, hipStream_t s)
+void launch_rk_row_batch(const RkRowArgs<T> *ad, const int *member, int nblocks, int st, int wind, bool terrain, hipStream_t s)
 {
     if (nblocks <= 0) return;
     const dim3 blk(RX, RY);
-#define LEE_RS(WM, TER, ST) hipLaunchKernelGGL((k_rk_row_batch<T, WM, TER, ST>), dim3((unsigned)nblocks), blk, 0, s, ad, first, n, st)
+#define LEE_RS(WM, TER, ST) hipLaunchKernelGGL((k_rk_row_batch<T, WM, TER, ST>), dim3((unsigned)nblocks), blk, 0, s, ad, member, st)
 #define LEE_RT(WM, TER)                                                                            \
     do {                                                                                           \
         if (st == 0) LEE_RS(WM, TER, 0); else if (st == 3) LEE_RS(WM, TER, 3); else LEE_RS(WM, TER, 1); \
@@ -712,6 +757,6 @@ void launch_rk_row_batch(const RkRowArgs<T> *ad, const int *first, int n, int nb
 #undef LEE_RS
 }
 template void launch_rk_row<LEE_RK_T>(const RkRowArgs<LEE_RK_T> *, const RowPlan &, int, int, bool, bool, double *, hipStream_t);
-template void launch_rk_row_batch<LEE_RK_T>(const RkRowArgs<LEE_RK_T> *, const int *, int, int, int, int, bool, hipStream_t);
+template void launch_rk_row_batch<LEE_RK_T>(const RkRowArgs<LEE_RK_T> *, const int *, int, int, int, bool, hipStream_t);
 
 }  // namespace lee

@@ -250,10 +250,12 @@ __device__ __forceinline__ void row_duvw_layers(const AirArgs<T> &a, const Nb<T>
 
 // The column's part of the metric at point i of row j: x, and over terrain sh, hx, hy.
 template <typename T> struct RowColumn { T x, sh, hx, hy; };
-template <typename T, bool TERRAIN> __device__ __forceinline__ RowColumn<T> row_column(const Grid<T> &g, int nx, int i, int j)
+// op: the column's byte offset from row j's first point (of the lane's row, where that differs).
+template <typename T, bool TERRAIN>
+__device__ __forceinline__ RowColumn<T> row_column(const Grid<T> &g, int nx, int i, int j, unsigned op)
 {
-    const unsigned o = (unsigned)i * (unsigned)sizeof(T);
-    RowColumn<T> c{ldr<T>(g.mx, 0, o), T(0), T(0), T(0)};
+    const unsigned o = op;
+    RowColumn<T> c{ldr<T>(g.mx, 0, (unsigned)i * (unsigned)sizeof(T)), T(0), T(0), T(0)};
     if constexpr (TERRAIN) {
         const size_t r = (size_t)nx * j * sizeof(T);
         c.sh = ldr<T>(g.tsh, r, o);
@@ -288,7 +290,7 @@ template <typename T, bool TERRAIN> __device__ __forceinline__ void row_metric(c
 template <typename T, bool TERRAIN>
 __device__ __forceinline__ void row_metric(const Grid<T> &g, int nx, int i, int j, T yy, T zk, T tk, Nb<T> &n)
 {
-    row_metric<T, TERRAIN>(row_column<T, TERRAIN>(g, nx, i, j), yy, zk, tk, n);
+    row_metric<T, TERRAIN>(row_column<T, TERRAIN>(g, nx, i, j, (unsigned)i * (unsigned)sizeof(T)), yy, zk, tk, n);
 }
 
 // Reader of a field at offsets (di, dj, dk) from the lane's point.
