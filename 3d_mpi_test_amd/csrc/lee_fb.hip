@@ -9,7 +9,9 @@
 // the face, or the three-row extrapolation of the East pressure, for which the last tile row
 // exchanges its rows through LDS; air and porous layer copy each other's planes
 // (calculation_2D.cpp:865-985) the same way.  The node order of the reference's face chain is
-// that of the walks in lee_bc.hip: x faces over y faces over the top, the ground last.
+// that of the walks in lee_bc.hip: x faces over y faces over the top, the ground last.  A row's
+// last tile of at most 21 columns runs as a strip, several rows a wavefront (141 x 201 x 441 FP64
+// with the East TDBC, rows of 64 + 64 + 13: 604 -> 566 us a step).
 #include "lee_faces.h"
 #include "lee_row.h"
 
@@ -25,11 +27,13 @@ enum { RK_AIR = 0, RK_PORE = 1, RK_GROUND = 2, RK_REC = 3 };
 struct RowTile {
     int kind, k, tx, ty;
     long long rec;  // first receiver of the block
+    int strip;      // a strip's block (RowLaunch), or -1
 };
 template <bool RING> __device__ __forceinline__ RowTile row_tile(const RowLaunch &l)
 {
     RowTile t;
     t.rec = 0;
+    t.strip = -1;
     if constexpr (!RING) {
         const int z = blockIdx.z;
         t.tx = blockIdx.x; t.ty = blockIdx.y;
@@ -53,6 +57,7 @@ template <bool RING> __device__ __forceinline__ RowTile row_tile(const RowLaunch
         if (s == 2) {
             const int e = ((const __attribute__((address_space(4))) int *)l.ring)[idx];
             t.tx = e & 0xffff; t.ty = e >> 16;
+            if (e & kStripBlock) t.strip = e & (kStripBlock - 1);
         } else {
             t.ty = idx / l.ntx;
             t.tx = idx - t.ty * l.ntx;
@@ -86,22 +91,22 @@ template <typename T> __device__ __forceinline__ void store_node(const Grid<T> &
 
 // p^{n+1} of the lane's point, and the old Q_p of the lane's node in its x, y and z slabs.
 template <typename T, int WM, bool TERRAIN, bool X, bool Y, bool Z>
-__device__ __forceinline__ T fb_p_point(const RowArgs<T> &A, const RowGeo &G, const RowLane &l, int j, int k, const RowLine<T> &yl,
+__device__ __forceinline__ T fb_p_point(const RowArgs<T> &A, const RowGeo &G, const RowLane &l, const RowPos &ps, int k, const RowLine<T> &yl,
                                         const RowLine<T> &zl, const RowSlab<T> &sy, const RowSlab<T> &sz, const RowX &xn, T &qx,
                                         T &qy, T &qz)
 {
     const AirArgs<T> &a = A.a;
     const Grid<T> &g = a.g;
     const size_t snx = (size_t)G.nx * sizeof(T), sxy = snx * G.ny;
-    const unsigned op = (unsigned)l.ip * (unsigned)sizeof(T), on = l.live ? (unsigned)l.in * (unsigned)sizeof(T) : op;
-    const RowAt<T> at{snx * j + sxy * k, snx, sxy, op};
+    const unsigned op = ps.op, on = l.live ? ps.on : op, ox = (unsigned)l.ip * (unsigned)sizeof(T);
+    const RowAt<T> at{snx * ps.jb + sxy * k, snx, sxy, op};
     Nb<T> n;
-    row_metric<T, TERRAIN>(g, G.nx, l.ip, j, yl.m, zl.m, zl.t, n);
+    row_metric<T, TERRAIN>(row_column<T, TERRAIN>(g, G.nx, l.ip, ps.jb, op), yl.m, zl.m, zl.t, n);
     Lay<T> lx{}, ly{}, lz{};
     QP<T> x{}, y{}, z{};
     if constexpr (X) {
-        const RowX q = row_x<T>(G, l.ip, j, k);
-        lx = {ldr<T>(A.xs, 0, op), ldr<T>(A.xc, 0, op), (Y || Z) ? ldr<T>(A.xd, 0, op) : T(0), q.act};
+        const RowX q = row_x<T>(G, l.ip, ps.j, k);
+        lx = {ldr<T>(A.xs, 0, ox), ldr<T>(A.xc, 0, ox), (Y || Z) ? ldr<T>(A.xd, 0, ox) : T(0), q.act};
         const RowQ<T> &Q = A.q[0];
         x.v0 = ldr<T>(Q.o[1], 0, q.o); x.vj = ldr<T>(Q.o[1], 0, q.o + q.dj);
         x.w0 = ldr<T>(Q.o[2], 0, q.o); x.wk = ldr<T>(Q.o[2], 0, q.o + q.dk);
@@ -141,6 +146,45 @@ __device__ __forceinline__ T fb_p_point(const RowArgs<T> &A, const RowGeo &G, co
     T r = row_dp<T, WM, TERRAIN, false>(a, at, RowState<T>{g, at}, n, ddx, ddy, dwz);
     r = row_dp_layers<T, TERRAIN, X, Y, Z>(a, n, lx, ly, lz, x, y, z, n.pc, ddx, ddy, dwz, r);
     return n.pc + r;
+}
+
+// The air point of a lane: stencil, stores of its node.  YS: the row may lie in a y layer.
+template <typename T, int WM, bool TERRAIN, bool YS>
+__device__ __forceinline__ T fb_p_air(const RowArgs<T> &A, const RowGeo &G, const RowLane &l, const RowPos &ps, int k, const RowLine<T> &yl,
+                                      const RowLine<T> &zl, bool mx)
+{
+    const Grid<T> &g = A.a.g;
+    const RowSlab<T> sy = row_slab_y(yl, G.nx, k), sz = row_slab_z(zl, G.nx, G.ny, ps.jb);
+    const RowX xn = row_x<T>(G, l.in, ps.j, k);
+    T qx = T(0), qy = T(0), qz = T(0), p;
+#define LEE_BODY(X, Y, Z) p = fb_p_point<T, WM, TERRAIN, X, Y, Z>(A, G, l, ps, k, yl, zl, sy, sz, xn, qx, qy, qz)
+    if (!sz.in) {
+        if (!YS || !sy.in) { if (mx) LEE_BODY(true, false, false); else LEE_BODY(false, false, false); }
+        else { if (mx) LEE_BODY(true, YS, false); else LEE_BODY(false, YS, false); }
+    } else {
+        if (!YS || !sy.in) { if (mx) LEE_BODY(true, false, true); else LEE_BODY(false, false, true); }
+        else { if (mx) LEE_BODY(true, YS, true); else LEE_BODY(false, YS, true); }
+    }
+#undef LEE_BODY
+    if (l.live) {
+        str<T>(g.pnn, (size_t)G.nx * ((size_t)ps.jb + (size_t)G.ny * k) * sizeof(T), ps.on, p);
+        const T dq = g.dt * p;
+        if (xn.own) str<T>(A.q[0].n[3], 0, xn.o, qx + dq);
+        if (YS && sy.in) str<T>(A.q[1].n[3], sy.row, ps.on, qy + dq);
+        if (sz.in) str<T>(A.q[2].n[3], sz.row, ps.on, qz + dq);
+    }
+    return p;
+}
+// A strip's block in either phase.
+template <typename T> __device__ __forceinline__ bool fb_strip(const RowArgs<T> &A, const RowGeo &G, const RowLaunch &L, int strip, RowLane &l,
+                                                               RowPos &ps, RowLine<T> &yl, bool &mx)
+{
+    const RowStrip &S = L.strip[0];  // (a row's narrow last tile: the only one)
+    if (!row_strip<T>(S, L.ja, L.jb, strip, G.nx, l, ps)) return false;
+    yl = RowLine<T>{};
+    yl.m = ldr<T>(A.a.g.my, 0, (unsigned)ps.j * (unsigned)sizeof(T));
+    mx = S.x0 < G.xa || S.x0 + S.n > G.xb;
+    return true;
 }
 
 // p^{n+1} of a porous point (porous.cpp:77-95).
@@ -184,6 +228,14 @@ __global__ __launch_bounds__(RX * RY) void k_row_p(const RowArgs<T> *__restrict_
         }
         return;
     }
+    if (RING && t.strip >= 0) {
+        RowLane l;
+        RowPos ps;
+        RowLine<T> yl;
+        bool mx;
+        if (fb_strip(A, G, L, t.strip, l, ps, yl, mx)) fb_p_air<T, WM, TERRAIN, false>(A, G, l, ps, t.k, yl, row_line(A.zl, t.k), mx);
+        return;
+    }
     const int jr = G.j0 + RY * t.ty + tj, k = t.k;
     const bool row_live = jr >= 1;
     const int j = row_live ? jr : 1;
@@ -192,28 +244,7 @@ __global__ __launch_bounds__(RX * RY) void k_row_p(const RowArgs<T> *__restrict_
     const bool last = t.ty == L.nty - 1;  // holds rows ny-4 .. ny-2 (uniform over the block)
     T p;
     if (t.kind == RK_AIR) {
-        const RowLine<T> yl = row_line(A.yl, j), zl = row_line(A.zl, k);
-        const RowSlab<T> sy = row_slab_y(yl, nx, k), sz = row_slab_z(zl, nx, ny, j);
-        const bool mx = row_meets_x(G, G.i0 + t.tx * RX);
-        const RowX xn = row_x<T>(G, l.in, j, k);
-        T qx = T(0), qy = T(0), qz = T(0);
-#define LEE_BODY(X, Y, Z) p = fb_p_point<T, WM, TERRAIN, X, Y, Z>(A, G, l, j, k, yl, zl, sy, sz, xn, qx, qy, qz)
-        if (!sz.in) {
-            if (!sy.in) { if (mx) LEE_BODY(true, false, false); else LEE_BODY(false, false, false); }
-            else { if (mx) LEE_BODY(true, true, false); else LEE_BODY(false, true, false); }
-        } else {
-            if (!sy.in) { if (mx) LEE_BODY(true, false, true); else LEE_BODY(false, false, true); }
-            else { if (mx) LEE_BODY(true, true, true); else LEE_BODY(false, true, true); }
-        }
-#undef LEE_BODY
-        if (l.live) {
-            const unsigned o = (unsigned)l.in * (unsigned)sizeof(T);
-            str<T>(g.pnn, (size_t)nx * ((size_t)j + (size_t)ny * k) * sizeof(T), o, p);
-            const T dq = g.dt * p;
-            if (xn.own) str<T>(A.q[0].n[3], 0, xn.o, qx + dq);
-            if (sy.in) str<T>(A.q[1].n[3], sy.row, o, qy + dq);
-            if (sz.in) str<T>(A.q[2].n[3], sz.row, o, qz + dq);
-        }
+        p = fb_p_air<T, WM, TERRAIN, true>(A, G, l, row_pos<T>(l, j), k, row_line(A.yl, j), row_line(A.zl, k), row_meets_x(G, G.i0 + t.tx * RX));
     } else if (t.kind == RK_PORE) {
         const Grid<T> &h = A.b.pore;
         // (the top plane of an uncoupled layer keeps what it holds)
@@ -289,22 +320,22 @@ template <typename T> __device__ __forceinline__ void pore_node_v(const Grid<T> 
 }
 
 template <typename T, int WM, bool TERRAIN, bool X, bool Y, bool Z>
-__device__ __forceinline__ void fb_v_point(const RowArgs<T> &A, const RowGeo &G, const RowLane &l, int j, int k,
+__device__ __forceinline__ void fb_v_point(const RowArgs<T> &A, const RowGeo &G, const RowLane &l, const RowPos &ps, int k,
                                            const RowLine<T> &yl, const RowLine<T> &zl, const RowSlab<T> &sy, const RowSlab<T> &sz,
                                            const RowX &xn, T (&out)[3], T (&qx)[3], T (&qy)[3], T (&qz)[3])
 {
     const AirArgs<T> &a = A.a;
     const Grid<T> &g = a.g;
     const size_t snx = (size_t)G.nx * sizeof(T), sxy = snx * G.ny;
-    const unsigned op = (unsigned)l.ip * (unsigned)sizeof(T), on = l.live ? (unsigned)l.in * (unsigned)sizeof(T) : op;
-    const RowAt<T> at{snx * j + sxy * k, snx, sxy, op};
+    const unsigned op = ps.op, on = l.live ? ps.on : op, ox = (unsigned)l.ip * (unsigned)sizeof(T);
+    const RowAt<T> at{snx * ps.jb + sxy * k, snx, sxy, op};
     Nb<T> n;
-    row_metric<T, TERRAIN>(g, G.nx, l.ip, j, yl.m, zl.m, zl.t, n);
+    row_metric<T, TERRAIN>(row_column<T, TERRAIN>(g, G.nx, l.ip, ps.jb, op), yl.m, zl.m, zl.t, n);
     Lay<T> lx{}, ly{}, lz{};
     QV<T> x{}, y{}, z{};
     if constexpr (X) {
-        const RowX q = row_x<T>(G, l.ip, j, k);
-        lx = {ldr<T>(A.xs, 0, op), ldr<T>(A.xc, 0, op), (Y || Z) ? ldr<T>(A.xd, 0, op) : T(0), q.act};
+        const RowX q = row_x<T>(G, l.ip, ps.j, k);
+        lx = {ldr<T>(A.xs, 0, ox), ldr<T>(A.xc, 0, ox), (Y || Z) ? ldr<T>(A.xd, 0, ox) : T(0), q.act};
         const RowQ<T> &Q = A.q[0];
         x.p0 = ldr<T>(Q.n[3], 0, q.o); x.pj = ldr<T>(Q.n[3], 0, q.o - q.dj); x.pk = ldr<T>(Q.n[3], 0, q.o - q.dk);
         if constexpr (Y || Z) {
@@ -341,6 +372,37 @@ __device__ __forceinline__ void fb_v_point(const RowArgs<T> &A, const RowGeo &G,
     out[0] = n.uc + du; out[1] = n.vc + dv; out[2] = n.wc + dw;
 }
 
+// The air point of a lane: stencil, stores of its node.
+template <typename T, int WM, bool TERRAIN, bool YS>
+__device__ __forceinline__ void fb_v_air(const RowArgs<T> &A, const RowGeo &G, const RowLane &l, const RowPos &ps, int k,
+                                         const RowLine<T> &yl, const RowLine<T> &zl, bool mx, T (&f)[3])
+{
+    const Grid<T> &g = A.a.g;
+    const RowSlab<T> sy = row_slab_y(yl, G.nx, k), sz = row_slab_z(zl, G.nx, G.ny, ps.jb);
+    const RowX xn = row_x<T>(G, l.in, ps.j, k);
+    T qx[3], qy[3], qz[3];
+#define LEE_BODY(X, Y, Z) fb_v_point<T, WM, TERRAIN, X, Y, Z>(A, G, l, ps, k, yl, zl, sy, sz, xn, f, qx, qy, qz)
+    if (!sz.in) {
+        if (!YS || !sy.in) { if (mx) LEE_BODY(true, false, false); else LEE_BODY(false, false, false); }
+        else { if (mx) LEE_BODY(true, YS, false); else LEE_BODY(false, YS, false); }
+    } else {
+        if (!YS || !sy.in) { if (mx) LEE_BODY(true, false, true); else LEE_BODY(false, false, true); }
+        else { if (mx) LEE_BODY(true, YS, true); else LEE_BODY(false, YS, true); }
+    }
+#undef LEE_BODY
+    if (!l.live) return;
+    if (l.face) f[0] = T(0);
+    const unsigned o = ps.on;
+    const size_t row = (size_t)G.nx * ((size_t)ps.jb + (size_t)G.ny * k) * sizeof(T);
+    str<T>(g.unn, row, o, f[0]); str<T>(g.vnn, row, o, f[1]); str<T>(g.wnn, row, o, f[2]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        if (xn.own) str<T>(A.q[0].n[c], 0, xn.o, qx[c] + g.dt * f[c]);
+        if (YS && sy.in) str<T>(A.q[1].n[c], sy.row, o, qy[c] + g.dt * f[c]);
+        if (sz.in) str<T>(A.q[2].n[c], sz.row, o, qz[c] + g.dt * f[c]);
+    }
+}
+
 // Velocities of a porous point (porous.cpp:112-135).
 template <typename T, bool TERRAIN>
 __device__ __forceinline__ void pore_v_point(const RowArgs<T> &A, const RowLane &l, int j, int k, T (&out)[3])
@@ -368,37 +430,23 @@ __global__ __launch_bounds__(RX * RY) void k_row_v(const RowArgs<T> *__restrict_
     const int nx = G.nx, ny = G.ny, nz = G.nz;
     const int lane = threadIdx.x, tj = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
     const RowTile t = row_tile<RING>(L);
+    if (RING && t.strip >= 0) {
+        RowLane l;
+        RowPos ps;
+        RowLine<T> yl;
+        bool mx;
+        T f[3];
+        if (fb_strip(A, G, L, t.strip, l, ps, yl, mx)) fb_v_air<T, WM, TERRAIN, false>(A, G, l, ps, t.k, yl, row_line(A.zl, t.k), mx, f);
+        return;
+    }
     const int jr = G.j0 + RY * t.ty + tj, k = t.k;
     if (jr < 1) return;
     const int j = jr;
     const RowLane l = row_lane(G.i0 + t.tx * RX + lane, nx, true);
     T f[3];
     if (t.kind == RK_AIR) {
-        const RowLine<T> yl = row_line(A.yl, j), zl = row_line(A.zl, k);
-        const RowSlab<T> sy = row_slab_y(yl, nx, k), sz = row_slab_z(zl, nx, ny, j);
-        const bool mx = row_meets_x(G, G.i0 + t.tx * RX);
-        const RowX xn = row_x<T>(G, l.in, j, k);
-        T qx[3], qy[3], qz[3];
-#define LEE_BODY(X, Y, Z) fb_v_point<T, WM, TERRAIN, X, Y, Z>(A, G, l, j, k, yl, zl, sy, sz, xn, f, qx, qy, qz)
-        if (!sz.in) {
-            if (!sy.in) { if (mx) LEE_BODY(true, false, false); else LEE_BODY(false, false, false); }
-            else { if (mx) LEE_BODY(true, true, false); else LEE_BODY(false, true, false); }
-        } else {
-            if (!sy.in) { if (mx) LEE_BODY(true, false, true); else LEE_BODY(false, false, true); }
-            else { if (mx) LEE_BODY(true, true, true); else LEE_BODY(false, true, true); }
-        }
-#undef LEE_BODY
+        fb_v_air<T, WM, TERRAIN, true>(A, G, l, row_pos<T>(l, j), k, row_line(A.yl, j), row_line(A.zl, k), row_meets_x(G, G.i0 + t.tx * RX), f);
         if (!l.live) return;
-        if (l.face) f[0] = T(0);
-        const unsigned o = (unsigned)l.in * (unsigned)sizeof(T);
-        const size_t row = (size_t)nx * ((size_t)j + (size_t)ny * k) * sizeof(T);
-        str<T>(g.unn, row, o, f[0]); str<T>(g.vnn, row, o, f[1]); str<T>(g.wnn, row, o, f[2]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            if (xn.own) str<T>(A.q[0].n[c], 0, xn.o, qx[c] + g.dt * f[c]);
-            if (sy.in) str<T>(A.q[1].n[c], sy.row, o, qy[c] + g.dt * f[c]);
-            if (sz.in) str<T>(A.q[2].n[c], sz.row, o, qz[c] + g.dt * f[c]);
-        }
     } else if (t.kind == RK_PORE) {
         const Grid<T> &h = A.b.pore;
         if (k == G.pnz - 1) {
@@ -602,6 +650,8 @@ template <typename T> void launch_row_p(const RowArgs<T> *ad, const RowPlan &pl,
             if (sizeof(T) == 4 && vec && !TER && !W) launch_in_vec<T, false, true>(ad, pl.in, s);                                     \
             else hipLaunchKernelGGL((k_row_in<T, W, TER, true>), box, blk, 0, s, ad, pl.in);                        \
             hipLaunchKernelGGL((k_row_p<T, W, TER, true>), dim3((unsigned)pl.p.first[6]), blk, 0, s, ad, pl.p, rec); \
+        } else if (!pl.w[0].grid) {                                                                                 \
+            hipLaunchKernelGGL((k_row_p<T, W, TER, true>), dim3((unsigned)pl.w[0].first[6]), blk, 0, s, ad, pl.w[0], rec); \
         } else {                                                                                                    \
             hipLaunchKernelGGL((k_row_p<T, W, TER, false>), dim3((unsigned)pl.p.ntx, (unsigned)pl.p.nty, (unsigned)pl.p.z), blk, \
                                0, s, ad, pl.p, rec);                                                                \
@@ -621,6 +671,8 @@ template <typename T> void launch_row_v(const RowArgs<T> *ad, const RowPlan &pl,
             if (sizeof(T) == 4 && vec && !W) launch_in_vec<T, TER, false>(ad, pl.in, s);                                              \
             else hipLaunchKernelGGL((k_row_in<T, W, TER, false>), box, blk, 0, s, ad, pl.in);                       \
             hipLaunchKernelGGL((k_row_v<T, W, TER, true>), dim3((unsigned)pl.v.first[6]), blk, 0, s, ad, pl.v);     \
+        } else if (!pl.w[1].grid) {                                                                                 \
+            hipLaunchKernelGGL((k_row_v<T, W, TER, true>), dim3((unsigned)pl.w[1].first[6]), blk, 0, s, ad, pl.w[1]); \
         } else {                                                                                                    \
             hipLaunchKernelGGL((k_row_v<T, W, TER, false>), dim3((unsigned)pl.v.ntx, (unsigned)pl.v.nty, (unsigned)pl.v.z), blk, \
                                0, s, ad, pl.v);                                                                     \
@@ -712,7 +764,7 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
         l.ka = za; l.kb = zb;
         l.xa = pl.pair.xa; l.xb = pl.pair.xb; l.ya = pl.pair.ya; l.yb = pl.pair.yb;
         RowLaunch &w = pl.w[ph];
-        if (m.rk4) {
+        {
             w = l;
             w.xa = w.xb = w.ya = w.yb = 0;
             w.ka = 2; w.kb = std::max(2, m.nz - 2);
@@ -720,7 +772,7 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
             packs(w, RX / 3, 0, ntx > 1 ? tail : m.nx, 0, m.ny);
             w.grid = !w.nstrip;
             if (w.grid) w.ka = w.kb = 1;  // (an ensemble's blocks: whole planes)
-            if (pl.has_in) packs(l, RX / 2, l.xa, l.xb, l.ya, l.yb);
+            if (m.rk4 && pl.has_in) packs(l, RX / 2, l.xa, l.xb, l.ya, l.yb);
         }
         auto sections = [&](RowLaunch &r, int tiles) {
             r.nring = tiles ? tiles : 1;
@@ -746,17 +798,15 @@ void row_plan(RowPlan &pl, std::vector<int> &ring, const RowGeom &m)
                                                 j0 + RY * ty >= pl.pair.ya && j0 + RY * (ty + 1) <= pl.pair.yb
                                           : tx >= tx0 && tx < tx1 && ty >= ty0 && ty < ty1;
                     if (pl.has_in && !in && !packed(l, tx, ty)) ring.push_back(e);
-                    if (m.rk4 && !packed(w, tx, ty)) pl.list.push_back(e);
+                    if (!packed(w, tx, ty)) pl.list.push_back(e);
                 }
-                if (m.rk4) {
-                    if (pl.has_in) strips(ring, l, ty);
-                    strips(pl.list, w, ty);
-                }
+                if (pl.has_in) strips(ring, l, ty);
+                strips(pl.list, w, ty);
             }
         }
         if (pl.has_in) sections(l, (int)ring.size());
         else l.nring = 1;
-        if (m.rk4) sections(w, (int)pl.list.size());
+        sections(w, (int)pl.list.size());
     }
 }
 

@@ -164,7 +164,7 @@ struct RowBox { int tx, nbx, ty, nby, k, nk, i0, j0; };
 // porous planes, the ground plane and the receivers.  Around an interior box: blocks first[q] ..
 // first[q+1]-1 of section q (planes 1 .. ka-1, planes kb .., the ring of planes ka .. kb-1 listed
 // in `ring` as tx | ty << 16, porous, ground, receivers).
-// RK4: strips of n <= 32 columns from x0, which whole tiles would leave mostly empty (what an
+// Strips of n <= 32 columns from x0, which whole tiles would leave mostly empty (what an
 // interior leaves of the outer tiles, or a row's narrow last tile): `rows` rows per wavefront, on
 // the rows [ja, jb) outside the y layers, in the planes ka .. kb - 1.  Their blocks stand in the
 // list of those planes' tiles as kStripBlock | strip << 20 | block; the list is in the order of the
@@ -176,7 +176,7 @@ struct RowLaunch {
     int ka, kb, nring;
     int xa, xb, ya, yb;  // RK4: the interior's points, which the ring's tiles leave out
     int ja, jb, nstrip;
-    int grid;  // RK4: a grid of tiles and planes after all
+    int grid;  // a grid of tiles and planes after all
     RowStrip strip[2];
     unsigned by_full, by_ntx, by_ring;  // 2^32 / divisor, rounded up
     int first[7];
@@ -194,7 +194,7 @@ struct RowPlan {
     RowBox in;     // FB
     RowPair pair;  // RK4
     RowLaunch p, v;
-    RowLaunch w[2];        // RK4, the whole domain: stage 0 (with the receivers), the others
+    RowLaunch w[2];        // the whole domain: pressure phase or stage 0 (with the receivers), the others
     std::vector<int> list; // and the tiles of its planes ka .. kb - 1, as the ring's
 };
 struct RowGeom {

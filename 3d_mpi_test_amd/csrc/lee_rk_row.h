@@ -90,12 +90,6 @@ __device__ __forceinline__ T rk_point_if(int st, T xn, T k, T acc, T lo, T err, 
 // layer terms read.
 template <typename T> struct RkE { T u0, ui, uk, v0, vj, vk, w0, wk, p0, pi, pj, pk; };
 
-// Where a wavefront's lanes stand: a row jb (uniform) that addresses start from, the lane's row j
-// (jb, or one of the next ones) and the byte offsets of its point and node from row jb's first.
-struct RowPos {
-    int jb, j;
-    unsigned op, on;
-};
 // dt R of the four fields at the lane's point; xc: the stage state there.
 template <typename T, int WM, bool TERRAIN, int ST, bool X, bool Y, bool Z>
 __device__ __forceinline__ void rk_row_point(const RkRowArgs<T> &A, const RowGeo &G, const RowLane &l, const RowPos &ps, int k,
@@ -388,8 +382,7 @@ __device__ __forceinline__ void rk_row_block(const RkRowArgs<T> &A, int st, int 
     }
     T d[4];
     if (kind == RK_AIR) {
-        const RowPos ps{j, j, (unsigned)l.ip * (unsigned)sizeof(T), (unsigned)l.in * (unsigned)sizeof(T)};
-        rk_row_air<T, WM, TERRAIN, ST, true>(A, G, l, ps, k, row_line(A.yl, j), row_line(A.zl, k), row_meets_x(G, i0), d);
+        rk_row_air<T, WM, TERRAIN, ST, true>(A, G, l, row_pos<T>(l, j), k, row_line(A.yl, j), row_line(A.zl, k), row_meets_x(G, i0), d);
     } else {
         rk_row_pore<T, TERRAIN, ST>(A, G, st, l, j, k, d);
         if (l.face) d[0] = T(0);
@@ -441,15 +434,9 @@ template <typename T, int WM, bool TERRAIN, int ST>
 __device__ __forceinline__ void rk_row_strip(const RkRowArgs<T> &A, const RowStrip &S, int ja, int je, int k, int br)
 {
     const RowGeo G = A.geo;
-    const int lane = threadIdx.x, tj = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-    const int jb = ja + (RY * br + tj) * S.rows;
-    if (jb >= je) return;
-    int r = (lane * S.inv) >> 16;
-    const int c = lane - r * S.n;
-    const bool live = r < S.rows && jb + r < je;
-    if (!live) r = 0;
-    const RowLane l = row_lane(S.x0 + c, G.nx, live);
-    const RowPos ps{jb, jb + r, (unsigned)(l.ip + G.nx * r) * (unsigned)sizeof(T), (unsigned)(l.in + G.nx * r) * (unsigned)sizeof(T)};
+    RowLane l;
+    RowPos ps;
+    if (!row_strip<T>(S, ja, je, br, G.nx, l, ps)) return;
     RowLine<T> yl{};
     yl.m = ldr<T>(A.a.g.my, 0, (unsigned)ps.j * (unsigned)sizeof(T));
     T d[4];

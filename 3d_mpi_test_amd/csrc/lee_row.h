@@ -65,6 +65,31 @@ __device__ __forceinline__ RowLane row_lane(int i, int nx, bool row_live)
     return l;
 }
 
+// Where a wavefront's lanes stand: a row jb (uniform) that addresses start from, the lane's row j
+// (jb, or one of the next ones) and the byte offsets of its point and node from row jb's first.
+struct RowPos {
+    int jb, j;
+    unsigned op, on;
+};
+template <typename T> __device__ __forceinline__ RowPos row_pos(const RowLane &l, int j)
+{
+    return {j, j, (unsigned)l.ip * (unsigned)sizeof(T), (unsigned)l.in * (unsigned)sizeof(T)};
+}
+// Lanes of block row `br` of a strip (four wavefronts, S.rows rows each); false: no row left.
+template <typename T> __device__ __forceinline__ bool row_strip(const RowStrip &S, int ja, int je, int br, int nx, RowLane &l, RowPos &ps)
+{
+    const int lane = threadIdx.x, tj = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
+    const int jb = ja + (RY * br + tj) * S.rows;
+    if (jb >= je) return false;
+    int r = (lane * S.inv) >> 16;
+    const int c = lane - r * S.n;
+    const bool live = r < S.rows && jb + r < je;
+    if (!live) r = 0;
+    l = row_lane(S.x0 + c, nx, live);
+    ps = {jb, jb + r, (unsigned)(l.ip + nx * r) * (unsigned)sizeof(T), (unsigned)(l.in + nx * r) * (unsigned)sizeof(T)};
+    return true;
+}
+
 // The y or z layer of a row (wave-uniform): whether it lies in a slab, whether the layer terms
 // apply, the byte offset of the row in the axis's block and the byte steps along y and z (0
 // where the neighbour is not read), and the profile.
