@@ -113,6 +113,7 @@ struct lee_ctx {
     long long *rec_idx = nullptr;
     double *rec_buf = nullptr;
     int *flag = nullptr;
+    std::vector<std::vector<unsigned char>> *held = nullptr;  // host buffers of pending uploads (Uploads)
     void *shift_tmp = nullptr;  // frame shift: one field or slab copied out of place
     size_t shift_tmp_bytes = 0;
     int device = 0;
@@ -207,30 +208,48 @@ int dalloc(lee_ctx *c, void **out, size_t bytes)
     return LEE_OK;
 }
 
-// Upload FP64 host values as the device type.
-int upload(lee_ctx *c, void *dst, const double *src, size_t n)
+// Upload FP64 host values as the device type (as FP64 whatever the state precision: upload_f64).  On
+// return the host buffer may be released: the call waits for the copy or, while an Uploads
+// stands, copies from a buffer that it keeps (a frame of a terrain run makes 36 uploads).
+template <typename T> int upload_as(lee_ctx *c, void *dst, const double *src, size_t n)
 {
     if (!n) return LEE_OK;
-    // set-up path only: wait for the copy so the host buffer may be released on return
-    if (c->prec == 64) {
-        HIPCHK(c, hipMemcpyAsync(dst, src, n * 8, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-    } else {
-        std::vector<float> tmp(src, src + n);
-        HIPCHK(c, hipMemcpyAsync(dst, tmp.data(), n * 4, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (c->held && n <= ((size_t)1 << 20)) {  // (a mean-flow field is not copied twice)
+        std::vector<unsigned char> h(n * sizeof(T));
+        T *t = (T *)h.data();
+        for (size_t i = 0; i < n; ++i) t[i] = (T)src[i];
+        c->held->push_back(std::move(h));
+        HIPCHK(c, hipMemcpyAsync(dst, c->held->back().data(), n * sizeof(T), hipMemcpyHostToDevice, c->stream));
+        return LEE_OK;
     }
-    return LEE_OK;
-}
-
-// Upload FP64 host values as FP64 whatever the state precision (coordinates).
-int upload_f64(lee_ctx *c, double *dst, const double *src, size_t n)
-{
-    if (!n) return LEE_OK;
-    HIPCHK(c, hipMemcpyAsync(dst, src, n * 8, hipMemcpyHostToDevice, c->stream));
+    std::vector<T> tmp;
+    if (sizeof(T) != sizeof(double)) tmp.assign(src, src + n);
+    HIPCHK(c, hipMemcpyAsync(dst, tmp.empty() ? (const void *)src : tmp.data(), n * sizeof(T), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return LEE_OK;
 }
+int upload(lee_ctx *c, void *dst, const double *src, size_t n)
+{
+    return c->prec == 64 ? upload_as<double>(c, dst, src, n) : upload_as<float>(c, dst, src, n);
+}
+int upload_f64(lee_ctx *c, double *dst, const double *src, size_t n) { return upload_as<double>(c, dst, src, n); }
+// Uploads of its lifetime wait once, at its end.
+struct Uploads {
+    lee_ctx *c;
+    std::vector<std::vector<unsigned char>> held;
+    explicit Uploads(lee_ctx *ctx) : c(ctx) { c->held = &held; }
+    int finish()
+    {
+        c->held = nullptr;
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        return LEE_OK;
+    }
+    ~Uploads()
+    {
+        if (c->held) (void)hipStreamSynchronize(c->stream);  // an error on the way: the copies end before their buffers
+        c->held = nullptr;
+    }
+};
 
 int download(lee_ctx *c, double *dst, const void *src, size_t n)
 {
@@ -379,6 +398,7 @@ int upload_frame(lee_ctx *c, int N)
 {
     const Model &m = c->m;
     FrameTables t;
+    Uploads pending(c);
     m.frame_tables(N, t, false);
     auto metric = [&](void *dst, const std::vector<double> &v) {
         // FP32 on the separable grid stores the reciprocals (the metric itself); the terrain
@@ -398,9 +418,7 @@ int upload_frame(lee_ctx *c, int N)
         for (int j = 1; j + 1 < m.ny; ++j) gy[j] = 1.0 / t.Yy[j];
         c->gmz = 1.0 / t.Zz[1];
         // FP64 in both precisions (the plane's coefficients are cast per use)
-        HIPCHK(c, hipMemcpyAsync(c->gmx, gx.data(), gx.size() * 8, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipMemcpyAsync(c->gmy, gy.data(), gy.size() * 8, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        if ((rc = upload_f64(c, c->gmx, gx.data(), gx.size())) || (rc = upload_f64(c, c->gmy, gy.data(), gy.size()))) return rc;
         if (m.terrain) {
             // the plane's metric on the terrain-following grid: that of a porous top plane
             // shifted rigidly with the ground (Z_over_z = Zz, Z_over_x = hx, Z_over_y = hy)
@@ -475,8 +493,7 @@ int upload_frame(lee_ctx *c, int N)
     std::vector<long long> idx(nr);
     for (int r = 0; r < nr; ++r) idx[r] = m.receiver_index(r, N);
     if (nr) HIPCHK(c, hipMemcpyAsync(c->rec_idx, idx.data(), nr * sizeof(long long), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return LEE_OK;
+    return pending.finish();
 }
 
 // Row form RK4: while its time gate is closed the y1 layer's auxiliaries are left alone, whichever
