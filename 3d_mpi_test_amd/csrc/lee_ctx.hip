@@ -2120,6 +2120,11 @@ int lee_kernel_stats(const lee_ctx *c, lee_kstat *out, int cap)
         qrk += cnt * (rk_rows(c) ? 5.0 : 16.0);
     }
     const double wrk = m.has_wind ? (m.wind_v_only ? 1.0 : 3.0) * m.nx * m.ny * m.nz : 0.0;
+    // an interior by pairs of stages: 12 + 24 words a step in FP32, 12 + 16 in FP64, V twice
+    const RowPair &in = c->plan.pair;
+    const double n_in = rk_rows(c) && c->plan.has_in && c->rk_variant >= kRkSplit
+                            ? (double)(in.xb - in.xa) * (in.yb - in.ya) * (in.zb - in.za) : 0.0;
+    const double saved = n_in * (rkw - (c->prec == 32 ? 36.0 : 28.0) / 4.0 + (m.has_wind ? (m.wind_v_only ? 0.5 : 1.5) : 0.0));
     const double rr = rk_rows(c) ? 1.0 : 0.0;  // the row form's stage holds the porous layer and the faces as well
     // the row form's FB phases hold the porous layer and the faces as well
     const double fr = !m.rk4 && fb_rows(c) ? 1.0 : 0.0;
@@ -2127,7 +2132,7 @@ int lee_kernel_stats(const lee_ctx *c, lee_kstat *out, int cap)
     double bytes[KS_N] = {(5 * (inner + fr * pinner) + qp + wind + 2 * fr * nb) * es,
                           (7 * (inner + fr * pinner) + qv + wind + 6 * fr * nb) * es + fr * psi, 5 * pinner * es,
                           7 * pinner * es, (8 * inner + qf + wind) * es, 2 * nb * es, 6 * nb * es + psi,
-                          (rkw * inner + qrk + wrk + rr * (prkw * pinner + 8 * nb)) * es, prkw * pinner * es, 8 * nb * es};
+                          (rkw * inner - saved + qrk + wrk + rr * (prkw * pinner + 8 * nb)) * es, prkw * pinner * es, 8 * nb * es};
     double pts[KS_N] = {inner + fr * pinner, inner + fr * pinner, pinner, pinner, inner, nb, nb, inner + rr * pinner, pinner, nb};
     int n = 0;
     for (int k = 0; k < KS_N && n < cap; ++k) {

@@ -52,10 +52,7 @@ if ROOT not in sys.path:
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 # launch shapes of the RK4 air stage (lee_options.rk_tile 1..11), as the autotuner reports them
-RK_TILES = ["64x4 planes", "64x4 xcd-columns", "64x8 xcd-columns", "64x8 planes", "64x16 xcd-columns",
-            "64x4 interior + layer shell", "64x4 interior + layers by axis", "64x4 LDS-staged interior + layer shell",
-            "64x4 LDS-staged interior + layers by axis", "64x4 LDS-staged interior + LDS-staged layer shell",
-            "64x4 LDS-staged interior + LDS-staged layers by axis"]
+RK_TILES = ["whole domain in one launch a stage"] * 5 + ["interior two stages a launch, the rest one"] * 6
 # launch forms of the FB_p_v air passes (lee_options.fb_form 1..7), as the autotuner reports them
 FB_FORMS = ["split", "split, padded tile lists", "fused, 2 blocks/CU", "fused, 4 blocks/CU", "fused, 8 blocks/CU",
             "fused, 16 blocks/CU", "split, one point per lane"]

@@ -116,18 +116,16 @@ typedef struct lee_options {
     int ground_poles;       /* 0: off, else 1..LEE_MAX_POLES pole/residue pairs */
     double ground_a[8], ground_r[8];
     double ground_zinf, ground_tau;
-    /* RK4 air-stage launch shape: 0 = autotune on the first steps (times the candidates on the
-     * context's own buffers), 1..11 = candidate 0..10 (64x4 plane order, 64x4 / 64x8 XCD
-     * columns, 64x8 plane order, 64x16 XCD columns, 64x4 tiles split into the interior outside
-     * every layer and the layer shell, the same with the shell split by slab axes, those two
-     * with the interior's stage state staged through LDS, and with the shell's staged as
-     * well).  All give the same bits. */
+    /* RK4 stage launch shape: 0 = autotune on the first step (times the candidates on the
+     * context's own buffers), 1..5 = the whole domain in one launch a stage, 6..11 = the interior
+     * outside every layer two stages a launch and the rest of the domain in another, where the grid
+     * has such an interior.  All give the same bits. */
     int rk_tile;
     /* FB_p_v air-pass launch form: 0 = autotune on the first step among the forms `path`
      * allows (times each form's air and face passes on the coming step), 1 = the split
      * passes (in FP32 the interior box four points per lane, 16-byte accesses, when there is
      * no mean flow and nx is a multiple of 4; over terrain in the velocity pass only), 2 = the
-     * same with each plane's tiles padded to a multiple of 8 (a tile column on one XCD),
+     * whole domain in one launch a phase (narrow columns: 0 takes several steps a launch),
      * 3..6 = the fused pass with pencils deep enough for about 2, 4, 8, 16 blocks per CU,
      * 7 = the split passes with one point per lane throughout.  1, 2 and 7 need path AUTO or SPLIT, 3..6 AUTO or FUSED.  All give
      * the same bits. */
